@@ -329,12 +329,14 @@ static hipError_t size_dist_enqueue(pmc_gpu *h, int box, int quantity, int n_bin
   for (int lo = 0; lo < n_bin; lo += DIST_WIN) {
     const int win = std::min(DIST_WIN, n_bin - lo);
     int key_bits = 1;
-    while ((1 << key_bits) <= win) key_bits++;  // keys 0..win, win for "not in this window"
-    hipLaunchKernelGGL(k_dist_partial, dim3(DIST_BLOCKS), dim3(DIST_THREADS), 0, h->stream,
+    while ((1 << key_bits) < win) key_bits++;  // keys 0..win - 1
+    const int waves = dist_waves(win);
+    hipLaunchKernelGGL(k_dist_partial, dim3(DIST_BLOCKS), dim3(waves * 64),
+                       waves * win * sizeof(double), h->stream,
                        h->d_box, h->A, box, quantity, n_bin, log_lo, log_hi, lo, win, key_bits,
                        partials);
-    hipLaunchKernelGGL(k_dist_reduce, dim3((win + 255) / 256), dim3(256), 0, h->stream, partials,
-                       DIST_BLOCKS, lo, win, n_bin, d_hist);
+    hipLaunchKernelGGL(k_dist_reduce, dim3((win + RED_BINS - 1) / RED_BINS), dim3(RED_THREADS), 0,
+                       h->stream, partials, lo, win, n_bin, d_hist);
   }
   return hipGetLastError();
 }

@@ -8,58 +8,54 @@
 // 1243-1261), times its mass or volume for the mass and volume
 // distributions.
 //
-// Two passes, with no device-wide sort and no atomics, so a histogram does
-// not depend on the order in which work lands:
+// Two passes, with no sort and no atomics, so a histogram does not depend on
+// the order in which work lands:
 //   k_dist_partial: DIST_BLOCKS workgroups each take a fixed slice of the
-//     box's particles (slice b is [b n / NB, (b+1) n / NB)), in tiles of
-//     DIST_TILE.  A tile is sorted by bin in LDS (block radix sort) and
-//     summed per bin by a segmented scan; the last element of each run adds
-//     the run's sum to the workgroup's LDS histogram, one writer per bin per
-//     tile.  The workgroup writes its whole histogram window (zeros
-//     included) to partials[b][.].
-//   k_dist_reduce: one thread per bin adds partials[0..NB)[bin] in order.
+//     box's particles (slice b is [b n / NB, (b+1) n / NB)).  Each wavefront
+//     keeps its own LDS histogram.  Lanes that hold the same bin find each
+//     other with one ballot per bit of the bin; the first of them adds the
+//     others' values in lane order and updates the bin, one writer per bin.  The workgroup adds its wavefronts'
+//     histograms in order and writes the whole window (zeros included) to
+//     partials[b][.].
+//   k_dist_reduce: adds partials[0..NB)[bin], RED_ROWS rows a thread and
+//     the rows' sums in order.
 // Bins are handled in windows of at most DIST_WIN, one pair of passes per
 // window.  Both passes read the particle count from the box descriptor on
 // the device, so the host never waits on the device to enqueue them.
 #pragma once
-
-#include <rocprim/block/block_radix_sort.hpp>
-#include <rocprim/block/block_scan.hpp>
 
 #include "pmc_exact.h"
 
 namespace pmc {
 
 constexpr int DIST_NUM = 0, DIST_MASS = 1, DIST_VOL = 2;
-constexpr int DIST_THREADS = 256;
-constexpr int DIST_ITEMS = 4;
-constexpr int DIST_TILE = DIST_THREADS * DIST_ITEMS;
+constexpr int DIST_ITEMS = 3;     // particles a lane in flight together
 constexpr int DIST_BLOCKS = 512;  // workgroups of the partial pass: fixed, so sums do not depend on the device
 constexpr int DIST_WIN = 2048;    // bins per window: the LDS histogram and a row of partials
 
-struct DistSeg {  // segmented-sum element: starts a run, running sum
-  int head;
-  double v;
-};
-struct DistSegOp {
-  __device__ DistSeg operator()(const DistSeg &a, const DistSeg &b) const {
-    return b.head ? b : DistSeg{a.head, a.v + b.v};
-  }
-};
-
 // bin (1-based, 0 / n_bin + 1 outside the grid) and weight / width of
-// particle slot p of box B
-__device__ inline int dist_item(const BoxDesc *B, const Arrays &A, int64_t p, int quantity,
-                                int n_bin, double log_lo, double log_hi, double *val) {
+// particle slot p, w_box the box's weights
+__device__ inline int dist_item(const Weights &w_box, const Arrays &A, int64_t p,
+                                int quantity, int n_bin, double log_lo, double log_hi,
+                                double *val) {
+  const int ns = A.n_spec;
+  const int klass = A.klass[p];
   double v = 0.0, m = 0.0;
-  for (int s = 0; s < A.n_spec; ++s) {
-    const double x = A.vol[(int64_t)s * A.total_cap + p];
-    v += x;
-    m += x * A.density[s];
+  for (int s0 = 0; s0 < ns; s0 += SPEC_CHUNK) {
+    double x[SPEC_CHUNK];
+#pragma unroll
+    for (int u = 0; u < SPEC_CHUNK; ++u)
+      x[u] = A.vol[(int64_t)(s0 + u < ns ? s0 + u : ns - 1) * A.total_cap + p];
+#pragma unroll
+    for (int u = 0; u < SPEC_CHUNK; ++u)
+      if (s0 + u < ns) {
+        v += x[u];
+        m += x[u] * A.density[s0 + u];
+      }
   }
   const double r = vol2rad(v);
   const int b = linspace_find(log_lo, log_hi, n_bin + 1, log(2.0 * r));
-  double w = nc_at_radius(B->w, A.klass[p], r);
+  double w = nc_at_radius(w_box, klass, r);
   if (quantity == DIST_MASS) w *= m;
   else if (quantity == DIST_VOL) w *= v;
   const double width = (log_hi - log_lo) / (double)n_bin;
@@ -67,70 +63,121 @@ __device__ inline int dist_item(const BoxDesc *B, const Arrays &A, int64_t p, in
   return b;
 }
 
+// Wavefronts of a partial-pass workgroup: as many as fit their histograms of
+// `win` bins in 64 KB of LDS, up to eight.  Two workgroups a compute unit
+// then leave 16 wavefronts to hide the arithmetic's latency.
+constexpr int DIST_WAVES = 8;
+inline int dist_waves(int win) { return std::min(DIST_WAVES, 65536 / (win * 8)); }
+static_assert(65536 / (DIST_WIN * 8) >= 1, "a window's histogram fits the LDS");
+
+// The sum of `v` over the lanes of the wavefront that hold the same key, in
+// lane order, on the first of them (which this returns true for); key < 0:
+// this lane holds nothing.  Every lane takes part.
+__device__ inline bool wave_key_sum(int key, int key_bits, double v, double *sum) {
+  const int lane = threadIdx.x & 63;
+  uint64_t peers = __ballot(key >= 0);
+  if (!peers) return false;
+  for (int b = 0; b < key_bits; ++b) {
+    const uint64_t m = __ballot((key >> b) & 1);
+    peers &= ((key >> b) & 1) ? m : ~m;
+  }
+  const bool first = key >= 0 && __ffsll((long long)peers) - 1 == lane;
+  // the leaders walk their peers together, one peer each a pass
+  uint64_t rest = first ? peers : 0ull;
+  double s = 0.0;
+  while (__ballot(rest != 0)) {
+    const double x = __shfl(v, rest ? __ffsll((long long)rest) - 1 : lane);
+    if (rest) {
+      s += x;
+      rest &= rest - 1;
+    }
+  }
+  *sum = s;
+  return first;
+}
+
 // partials[blockIdx.x][0 .. win): this workgroup's sums over bins
-// [win_lo, win_lo + win) (0-based) of its slice of the box's particles
-__global__ void __launch_bounds__(DIST_THREADS)
+// [win_lo, win_lo + win) (0-based) of its slice of the box's particles.
+// Bound by FP64 arithmetic (a pow, a log and the weight per particle): a
+// lane takes DIST_ITEMS particles at a time, whose chains are independent.
+// 1.5e6 particles of 4 species in 160 bins take 50 us, 20000 in 60 bins
+// 7.7 us (68 and 21 us with a block sort and a segmented scan per tile of
+// 1024; 63 us with 4 wavefronts a workgroup in place of 8).
+__global__ void __launch_bounds__(DIST_WAVES * 64)
 k_dist_partial(const BoxDesc *boxes, Arrays A, int box, int quantity, int n_bin, double log_lo,
                double log_hi, int win_lo, int win, int key_bits, double *partials) {
-  using Sort = rocprim::block_radix_sort<int, DIST_THREADS, DIST_ITEMS, double>;
-  using Scan = rocprim::block_scan<DistSeg, DIST_THREADS>;
-  __shared__ union {
-    typename Sort::storage_type sort;
-    typename Scan::storage_type scan;
-  } st;
-  __shared__ int s_key[DIST_TILE];
-  __shared__ double s_hist[DIST_WIN];
+  extern __shared__ double s_hist[];  // [wavefronts][win]
+  __shared__ Weights s_w;
   const BoxDesc *B = &boxes[box];
-  const int64_t n = B->n_part;
+  const int64_t n = B->n_part, off = B->off;
   const int64_t lo = (int64_t)blockIdx.x * n / gridDim.x;
   const int64_t hi = (int64_t)(blockIdx.x + 1) * n / gridDim.x;
-  const int t = threadIdx.x;
-  for (int j = t; j < win; j += DIST_THREADS) s_hist[j] = 0.0;
+  const int t = threadIdx.x, threads = blockDim.x, waves = threads >> 6;
+  for (int j = t; j < waves * win; j += threads) s_hist[j] = 0.0;
+  for (int j = t; j < (int)(sizeof(Weights) / sizeof(int)); j += threads)
+    ((int *)&s_w)[j] = ((const int *)&B->w)[j];
   __syncthreads();
-  for (int64_t base = lo; base < hi; base += DIST_TILE) {
+  double *hist = s_hist + (t >> 6) * win;
+  for (int64_t base = lo; base < hi; base += threads * DIST_ITEMS) {
     int key[DIST_ITEMS];
     double val[DIST_ITEMS];
+#pragma unroll
     for (int k = 0; k < DIST_ITEMS; ++k) {
-      const int64_t i = base + (int64_t)t * DIST_ITEMS + k;
-      key[k] = win;  // padding and particles outside the window sort last
+      const int64_t i = base + (int64_t)k * threads + t;
+      key[k] = -1;  // past the slice or outside the window
       val[k] = 0.0;
       if (i < hi) {
         double x;
-        const int b = dist_item(B, A, B->off + i, quantity, n_bin, log_lo, log_hi, &x) - 1 - win_lo;
+        const int b = dist_item(s_w, A, off + i, quantity, n_bin, log_lo, log_hi, &x) - 1 - win_lo;
         if (b >= 0 && b < win && b + win_lo < n_bin) {
           key[k] = b;
           val[k] = x;
         }
       }
     }
-    Sort().sort(key, val, st.sort, 0, key_bits);
-    for (int k = 0; k < DIST_ITEMS; ++k) s_key[t * DIST_ITEMS + k] = key[k];
-    __syncthreads();  // s_key complete; the sort's storage is free for the scan
-    DistSeg seg[DIST_ITEMS];
+#pragma unroll
     for (int k = 0; k < DIST_ITEMS; ++k) {
-      const int i = t * DIST_ITEMS + k;
-      seg[k] = DistSeg{i == 0 || s_key[i - 1] != key[k], val[k]};
+      double sum;
+      if (wave_key_sum(key[k], key_bits, val[k], &sum)) hist[key[k]] += sum;
     }
-    Scan().inclusive_scan(seg, seg, st.scan, DistSegOp());
-    for (int k = 0; k < DIST_ITEMS; ++k) {
-      const int i = t * DIST_ITEMS + k;
-      const bool tail = (i == DIST_TILE - 1) || s_key[i + 1] != key[k];
-      if (tail && key[k] < win) s_hist[key[k]] += seg[k].v;
-    }
-    __syncthreads();  // before the next tile reuses s_key and the storage
   }
+  __syncthreads();
   double *out = partials + (int64_t)blockIdx.x * win;
-  for (int j = t; j < win; j += DIST_THREADS) out[j] = s_hist[j];
+  for (int j = t; j < win; j += threads) {
+    double s = s_hist[j];
+    for (int w = 1; w < waves; ++w) s += s_hist[w * win + j];
+    out[j] = s;
+  }
 }
 
-// hist[win_lo + j] = sum over workgroups, in workgroup order, of partials[.][j]
-__global__ void k_dist_reduce(const double *partials, int n_part_blocks, int win_lo, int win,
-                              int n_bin, double *hist) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= win || win_lo + j >= n_bin) return;
+// hist[win_lo + j] = sum over workgroups of partials[.][j]: RED_BINS bins
+// (a 128-byte line of a row) a workgroup, each thread RED_ROWS consecutive
+// rows with its loads in flight together, then the threads' sums in row
+// order: 3.6 us for 60 bins and 5.9 for 160.  (One thread a bin waits for
+// its 512 loads in turn, 124 us for any bin count.)
+constexpr int RED_BINS = 16, RED_ROWS = 8;
+constexpr int RED_THREADS = RED_BINS * (DIST_BLOCKS / RED_ROWS);
+static_assert(RED_THREADS <= 1024 && DIST_BLOCKS % RED_ROWS == 0, "one workgroup covers the rows");
+
+__global__ void __launch_bounds__(RED_THREADS)
+k_dist_reduce(const double *partials, int win_lo, int win, int n_bin, double *hist) {
+  __shared__ double s_sum[RED_THREADS];
+  const int t = threadIdx.x, row0 = (t / RED_BINS) * RED_ROWS;
+  const int j = blockIdx.x * RED_BINS + t % RED_BINS;
   double s = 0.0;
-  for (int b = 0; b < n_part_blocks; ++b) s += partials[(int64_t)b * win + j];
-  hist[win_lo + j] = s;
+  if (j < win) {
+    double x[RED_ROWS];
+#pragma unroll
+    for (int r = 0; r < RED_ROWS; ++r) x[r] = partials[(int64_t)(row0 + r) * win + j];
+#pragma unroll
+    for (int r = 0; r < RED_ROWS; ++r) s += x[r];
+  }
+  s_sum[t] = s;
+  __syncthreads();
+  if (t < RED_BINS && j < win && win_lo + j < n_bin) {
+    for (int r = 1; r < RED_THREADS / RED_BINS; ++r) s += s_sum[r * RED_BINS + t];
+    hist[win_lo + j] = s;
+  }
 }
 
 }  // namespace pmc
