@@ -659,6 +659,37 @@ static int check_box_errors(pmc_gpu *h, std::vector<BoxDesc> &hb) {
   return 0;
 }
 
+static int rebal_ensure(pmc_gpu *h, bool slots);
+static int run_removal_tiles(pmc_gpu *h, const Removal &X, int64_t n_max, int action);
+
+// The segment passes of a preparation (pmc_prepare.h): the list counters of
+// a wavefront sit in LDS while all of a workgroup's fit.
+static int enqueue_prep_keys(pmc_gpu *h, int only_box) {
+  const int keys = h->max_bin * h->tab_classes;
+  const dim3 g(SORT_THREADS / PREP_WAVES, only_box >= 0 ? 1 : h->n_box), b(64 * PREP_WAVES);
+  if (keys <= PREP_LDS_KEYS)
+    hipLaunchKernelGGL(k_prep_keys<true>, g, b, PREP_WAVES * keys * sizeof(int), h->stream,
+                       h->d_box, h->A, only_box, keys);
+  else
+    hipLaunchKernelGGL(k_prep_keys<false>, g, b, 0, h->stream, h->d_box, h->A, only_box, keys);
+  HIPCHECK(hipGetLastError());
+  return 0;
+}
+
+static int enqueue_prep_lists(pmc_gpu *h, int only_box) {
+  const int keys = h->max_bin * h->tab_classes, nb = only_box >= 0 ? 1 : h->n_box;
+  const dim3 g(SORT_THREADS / PREP_WAVES, nb), b(64 * PREP_WAVES);
+  hipLaunchKernelGGL(k_prep_lists, dim3(nb), dim3(SORT_THREADS), 0, h->stream, h->d_box, h->A,
+                     only_box);
+  if (keys <= PREP_LDS_KEYS)
+    hipLaunchKernelGGL(k_prep_scatter<true>, g, b, PREP_WAVES * keys * sizeof(int), h->stream,
+                       h->d_box, h->A, only_box, keys);
+  else
+    hipLaunchKernelGGL(k_prep_scatter<false>, g, b, 0, h->stream, h->d_box, h->A, only_box, keys);
+  HIPCHECK(hipGetLastError());
+  return 0;
+}
+
 int pmc_gpu_set_bin_grid(pmc_gpu *h, int box, int n_bin, double r_min, double r_max) {
   int e = check_box(h, box);
   if (e) return e;
@@ -671,9 +702,26 @@ int pmc_gpu_set_bin_grid(pmc_gpu *h, int box, int n_bin, double r_min, double r_
   if ((e = SET_FIELD(h, box, grid_req_n_bin, n_bin))) return e;
   if ((e = SET_FIELD(h, box, grid_req_min, r_min))) return e;
   if ((e = SET_FIELD(h, box, grid_req_max, r_max))) return e;
-  hipLaunchKernelGGL(k_prepare, dim3(1), dim3(SORT_THREADS), 0, h->stream, h->d_box, h->A,
-                     box);
+  hipLaunchKernelGGL(k_prep_plan, dim3(1), dim3(64), 0, h->stream, h->d_box, h->A, box);
   HIPCHECK(hipGetLastError());
+  if ((e = enqueue_prep_keys(h, box))) return e;
+  BoxDesc B;
+  HIPCHECK(hipMemcpyAsync(&B, h->d_box + box, sizeof(B), hipMemcpyDeviceToHost, h->stream));
+  HIPCHECK(hipStreamSynchronize(h->stream));
+  std::vector<int> plan(h->n_box, 0);
+  if (!B.error && B.prep_outside > 0) {
+    // particles outside the grid leave in the reference's swap-last order,
+    // and the bins are counted again over the rest
+    if ((e = rebal_ensure(h, true))) return e;
+    plan[box] = 1;
+    HIPCHECK(hipMemcpyAsync(h->rw.plan, plan.data(), sizeof(int) * h->n_box,
+                            hipMemcpyHostToDevice, h->stream));
+    Removal X{};
+    X.kind = RM_OUTSIDE;
+    if ((e = run_removal_tiles(h, X, B.n_part, 0))) return e;
+    if ((e = enqueue_prep_keys(h, box))) return e;
+  }
+  if ((e = enqueue_prep_lists(h, box))) return e;
   HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
   HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
@@ -795,8 +843,15 @@ int pmc_gpu_mc_coag_async(pmc_gpu *h, int kernel_type, double del_t) {
       if (h->tape_buf[b])
         return fail(ERR_STATE, "box %d records or replays a tape: that is the exact mode's", b);
   if (h->mode == PMC_MODE_EXACT) {
-    LAUNCH_TIMED(h, "k_prepare", k_prepare, dim3(h->n_box), dim3(SORT_THREADS), 0, h->stream,
-                 h->d_box, h->A, -1);
+    hipEvent_t ev;
+    timing_begin(h, "k_prepare", &ev);
+    hipLaunchKernelGGL(k_prep_radii, dim3(PREP_RADII_WG, h->n_box), dim3(256), 0, h->stream,
+                       h->d_box, h->A, -1);
+    hipLaunchKernelGGL(k_prep_plan, dim3(h->n_box), dim3(64), 0, h->stream, h->d_box, h->A, -1);
+    HIPCHECK(hipGetLastError());
+    if ((e = enqueue_prep_keys(h, -1))) return e;
+    if ((e = enqueue_prep_lists(h, -1))) return e;
+    timing_end(h, "k_prepare", ev);
     if ((e = enqueue_tables(h, kernel_type))) return e;
     LAUNCH_TIMED(h, "k_exact_sweep", k_exact_sweep, dim3(h->n_box), dim3(64), 0, h->stream,
                  h->d_box, h->A, kernel_type, del_t, h->seed, h->step);
@@ -1120,6 +1175,24 @@ static int rebal_ensure(pmc_gpu *h, bool slots) {
   return 0;
 }
 
+// The passes of a removal over the boxes of rw.plan (as many slots as n_max
+// each): mark, prefix, move.
+static int run_removal_tiles(pmc_gpu *h, const Removal &X, int64_t n_max, int action) {
+  RebalWork &R = h->rw;
+  const int nb = h->n_box;
+  const dim3 bb(64), gb((nb + 63) / 64);
+  const dim3 gt((unsigned)std::max<int64_t>(1, (n_max + REBAL_TILE - 1) / REBAL_TILE), nb);
+  hipLaunchKernelGGL(k_remove_mark, gt, dim3(REBAL_THREADS), 0, h->stream, h->d_box, h->A, R, X,
+                     h->seed, h->step);
+  hipLaunchKernelGGL(k_tile_scan, dim3(nb), dim3(REBAL_THREADS), 0, h->stream, h->d_box, R, 1);
+  hipLaunchKernelGGL(k_remove_prefix, gt, dim3(REBAL_THREADS), 0, h->stream, h->d_box, h->A, R,
+                     action);
+  hipLaunchKernelGGL(k_remove_move, gt, dim3(REBAL_THREADS), 0, h->stream, h->d_box, h->A, R);
+  hipLaunchKernelGGL(k_remove_finish, gb, bb, 0, h->stream, h->d_box, R, nb, X);
+  HIPCHECK(hipGetLastError());
+  return 0;
+}
+
 // One removal pass over the boxes with want[b] != 0.  Boxes with current
 // bin lists (exact mode) remove one at a time through the lists, in the
 // reference's order; the others settle every slot at once.  hb must hold
@@ -1145,16 +1218,8 @@ static int run_removal(pmc_gpu *h, const std::vector<BoxDesc> &hb, const std::ve
   if (any_lists)
     hipLaunchKernelGGL(k_remove_lists, gb, bb, 0, h->stream, h->d_box, h->A, nb, R.plan + nb, X,
                        h->seed, h->step);
-  if (any_tiles) {
-    const dim3 gt((unsigned)std::max<int64_t>(1, (n_max + REBAL_TILE - 1) / REBAL_TILE), nb);
-    hipLaunchKernelGGL(k_remove_mark, gt, dim3(REBAL_THREADS), 0, h->stream, h->d_box, h->A, R, X,
-                       h->seed, h->step);
-    hipLaunchKernelGGL(k_tile_scan, dim3(nb), dim3(REBAL_THREADS), 0, h->stream, h->d_box, R, 1);
-    hipLaunchKernelGGL(k_remove_prefix, gt, dim3(REBAL_THREADS), 0, h->stream, h->d_box, h->A, R,
-                       X.kind == RM_HALVE ? INFO_HALVED : INFO_DILUTION);
-    hipLaunchKernelGGL(k_remove_move, gt, dim3(REBAL_THREADS), 0, h->stream, h->d_box, h->A, R);
-    hipLaunchKernelGGL(k_remove_finish, gb, bb, 0, h->stream, h->d_box, R, nb, X);
-  }
+  if (any_tiles)
+    return run_removal_tiles(h, X, n_max, X.kind == RM_HALVE ? INFO_HALVED : INFO_DILUTION);
   HIPCHECK(hipGetLastError());
   return 0;
 }

@@ -1,5 +1,5 @@
-// pmc_exact.h -- per-box preparation (sort / regrid), majorant and
-// pair tables, and the exact sequential-order sweep.
+// pmc_exact.h -- majorant and pair tables, and the exact sequential-order
+// sweep (the lists it walks are made in pmc_prepare.h).
 //
 // The exact sweep replays mc_coag's loop order (src/coagulation.F90:74-94)
 // inside one wavefront per box.  Tests of a bin pair are evaluated 64 at a
@@ -11,6 +11,7 @@
 #pragma once
 
 #include "pmc_state.h"
+#include "pmc_prepare.h"
 
 namespace pmc {
 
@@ -160,271 +161,6 @@ __device__ inline void copy_particle(const Arrays &A, int64_t from, int64_t to) 
         A.ctime[comp_at(to, c0 + j)] = ct[j];
       }
     }
-  }
-}
-
-// -------------------------------------------------------------- prepare
-// One block of SORT_THREADS per box: aero_sorted_remake_if_needed
-// (src/aero_sorted.F90:214-373), explicit-grid sorts (:254-262 with
-// aero_sorted_discard_outside_grid :153-180) and aero_sorted_sort_particles
-// (:185-209).  Lists are rebuilt into the other pool half every call so
-// every list starts the sweep with slack.
-__global__ void __launch_bounds__(SORT_THREADS)
-k_prepare(BoxDesc *boxes, Arrays A, int only_box) {
-  const int box = only_box >= 0 ? only_box : (int)blockIdx.x;
-  const int t = threadIdx.x;
-  BoxDesc *B = &boxes[box];
-  __shared__ int s_need_sort, s_err, s_n;
-  __shared__ double s_min[SORT_THREADS], s_max[SORT_THREADS];
-  if (B->error) return;
-  const int64_t base = B->off;
-  double *edges = A.edges + (int64_t)box * (A.max_bin + 1);
-  double *centers = A.centers + (int64_t)box * A.max_bin;
-  double *widths = A.widths + (int64_t)box * A.max_bin;
-  int *lstart = A.lstart + (int64_t)box * A.max_keys;
-  int *llen = A.llen + (int64_t)box * A.max_keys;
-  int *lcap = A.lcap + (int64_t)box * A.max_keys;
-  const int n_class = B->w.n_class;
-  if (t == 0) {
-    s_need_sort = 0;
-    s_err = 0;
-    s_n = B->n_part;
-  }
-  __syncthreads();
-
-  // refresh the cached total volumes (uploads and merges keep them too)
-  for (int i = t; i < s_n; i += SORT_THREADS) A.vtot[base + i] = particle_volume(A, base + i);
-  __syncthreads();
-
-  if (B->grid_req_n_bin >= 0) {
-    if (t == 0) {
-      int nb = B->grid_req_n_bin;
-      if (nb > A.max_bin) {
-        s_err = ERR_CAPACITY;
-      } else {
-        make_log_grid(nb, B->grid_req_min, B->grid_req_max, edges, centers, widths);
-        B->n_bin = nb;
-        B->log_lo = log(edges[0]);
-        B->log_hi = log(edges[nb]);
-        B->bounds_valid = 0;
-        B->tables_valid = 0;
-        B->regridded = 1;
-      }
-    }
-    __syncthreads();
-    if (s_err) {
-      if (t == 0) B->error = s_err;
-      return;
-    }
-    const int nb = B->n_bin;
-    int outside = 0;
-    for (int i = t; i < s_n; i += SORT_THREADS) {
-      const int b = bin_find_log(nb, B->log_lo, B->log_hi, vol2rad(A.vtot[base + i]));
-      A.fwd_bin[base + i] = b;
-      outside += (b < 1 || b > nb) ? 1 : 0;
-    }
-    __shared__ int s_outside;
-    if (t == 0) s_outside = 0;
-    __syncthreads();
-    if (outside) atomicAdd(&s_outside, outside);
-    __syncthreads();
-    if (t == 0) {
-      int n = s_n;
-      // aero_sorted_discard_outside_grid's swap-last pass, needed only when
-      // some particle lies outside the grid
-      for (int i = s_outside ? n - 1 : -1; i >= 0; --i) {
-        int b = A.fwd_bin[base + i];
-        if (b < 1 || b > nb) {
-          if (i < n - 1) copy_particle(A, base + n - 1, base + i);
-          n--;
-        }
-      }
-      s_n = n;
-      B->n_part = n;
-      B->grid_req_n_bin = -1;
-      s_need_sort = 1;
-    }
-    __syncthreads();
-  } else {
-    // r_min / r_max; lists left stale by the parallel mode count as unsorted
-    const bool use_lists = B->valid_sort && B->xlists_valid;
-    double rmin = 0.0, rmax = 0.0;
-    if (!use_lists) {
-      double lo = 1e300, hi = -1e300;
-      for (int i = t; i < s_n; i += SORT_THREADS) {
-        double r = vol2rad(A.vtot[base + i]);
-        lo = fmin(lo, r);
-        hi = fmax(hi, r);
-      }
-      s_min[t] = lo;
-      s_max[t] = hi;
-      __syncthreads();
-      for (int w = SORT_THREADS / 2; w > 0; w >>= 1) {
-        if (t < w) {
-          s_min[t] = fmin(s_min[t], s_min[t + w]);
-          s_max[t] = fmax(s_max[t], s_max[t + w]);
-        }
-        __syncthreads();
-      }
-      if (s_n > 0) {
-        rmin = s_min[0];
-        rmax = s_max[0];
-      }
-    }
-    if (t == 0) {
-      B->regridded = 0;
-      const int nb = B->n_bin;
-      if (!use_lists && B->valid_sort && nb > 0) {
-        // a valid sort without current lists: the occupied bins are those
-        // of the radius extremes
-        if (s_n == 0) {
-          rmin = edges[nb];
-          rmax = edges[0];
-        } else {
-          const int b_lo = bin_find_log(nb, B->log_lo, B->log_hi, rmin);
-          const int b_hi = bin_find_log(nb, B->log_lo, B->log_hi, rmax);
-          rmin = edges[max(b_lo, 1) - 1];
-          rmax = edges[min(b_hi, nb)];
-        }
-      }
-      if (use_lists) {
-        int i_min = 0, i_max = 0;
-        for (int b = 1; b <= nb; ++b) {
-          int tot = 0;
-          for (int c = 1; c <= n_class; ++c) tot += llen[(b - 1) + nb * (c - 1)];
-          if (tot > 0) {
-            if (i_min == 0) i_min = b;
-            i_max = b;
-          }
-        }
-        if (i_min == 0) {
-          if (nb > 0) {
-            rmin = edges[nb];
-            rmax = edges[0];
-          }
-        } else {
-          rmin = edges[i_min - 1];
-          rmax = edges[i_max];
-        }
-      }
-      bool done = false;
-      if (rmax == 0.0) {
-        if (!use_lists) {
-          B->n_bin = 0;
-          B->bounds_valid = 0;
-          B->tables_valid = 0;
-        }
-        done = true;
-      }
-      if (!done) {
-        bool need = false;
-        if (nb < 1) {
-          need = true;
-        } else if ((rmin / edges[0] < 3.0) || (edges[nb] / rmax < 3.0)) {
-          need = true;
-        }
-        if (need) {
-          double gmin = rmin / 10.0, gmax = rmax * 10.0;
-          double nbf = ceil((log10(gmax) - log10(gmin)) * 10.0);
-          if (nbf < 0.0) {
-            s_err = 538534122;
-          } else if (nbf > (double)A.max_bin) {
-            s_err = ERR_CAPACITY;
-          } else {
-            int nn = (int)nbf;
-            make_log_grid(nn, gmin, gmax, edges, centers, widths);
-            B->n_bin = nn;
-            B->log_lo = log(edges[0]);
-            B->log_hi = log(edges[nn]);
-            B->bounds_valid = 0;
-            B->tables_valid = 0;
-            B->regridded = 1;
-            s_need_sort = 1;
-          }
-        } else if (!use_lists) {
-          s_need_sort = 1;
-        }
-      }
-    }
-    __syncthreads();
-    if (s_err) {
-      if (t == 0) B->error = s_err;
-      return;
-    }
-  }
-
-  const int nb = B->n_bin;
-  const int K = nb * n_class;
-  const int n = s_n;
-  int *scr = A.sort_scratch + (int64_t)box * SORT_THREADS * A.max_keys + (int64_t)t * A.max_keys;
-  if (s_need_sort) {
-    // stable counting sort: thread t owns the contiguous segment
-    // [t*S, (t+1)*S), so list order = particle order as appends produce.
-    const int S = (n + SORT_THREADS - 1) / SORT_THREADS;
-    const int i0 = t * S, i1 = min(n, i0 + S);
-    for (int k = 0; k < K; ++k) scr[k] = 0;
-    for (int i = i0; i < i1; ++i) {
-      int b = bin_find_log(nb, B->log_lo, B->log_hi, vol2rad(A.vtot[base + i]));
-      if (b < 1 || b > nb) {
-        atomicExch(&s_err, 708651144);
-        b = 1;
-      }
-      int c = A.klass[base + i];
-      A.fwd_bin[base + i] = b;
-      A.fwd_class[base + i] = c;
-      scr[(b - 1) + nb * (c - 1)]++;
-    }
-    __syncthreads();
-    int *scr0 = A.sort_scratch + (int64_t)box * SORT_THREADS * A.max_keys;
-    for (int k = t; k < K; k += SORT_THREADS) {
-      int run = 0;
-      for (int tt = 0; tt < SORT_THREADS; ++tt) {
-        int c = scr0[(int64_t)tt * A.max_keys + k];
-        scr0[(int64_t)tt * A.max_keys + k] = run;
-        run += c;
-      }
-      llen[k] = run;
-    }
-    __syncthreads();
-  }
-  if (t == 0) {
-    int h = 1 - B->pool_cur;
-    int64_t pbase = B->pool_off + (int64_t)h * B->pool_half;
-    int64_t pos = 0;
-    for (int k = 0; k < K; ++k) {
-      lstart[k] = (int)(pbase + pos);
-      lcap[k] = llen[k] + llen[k] / 4 + 8;
-      pos += lcap[k];
-    }
-    if (pos > B->pool_half) s_err = ERR_CAPACITY;
-    B->pool_top = (int)pos;
-    B->pool_cur = h;
-  }
-  __syncthreads();
-  if (s_err) {
-    if (t == 0) B->error = s_err;
-    return;
-  }
-  if (s_need_sort) {
-    const int S = (n + SORT_THREADS - 1) / SORT_THREADS;
-    const int i0 = t * S, i1 = min(n, i0 + S);
-    for (int i = i0; i < i1; ++i) {
-      int key = (A.fwd_bin[base + i] - 1) + nb * (A.fwd_class[base + i] - 1);
-      int p = scr[key]++;
-      A.pool[lstart[key] + p] = i + 1;
-      A.fwd_idx[base + i] = p + 1;
-    }
-  } else {
-    for (int i = t; i < n; i += SORT_THREADS) {
-      int key = (A.fwd_bin[base + i] - 1) + nb * (A.fwd_class[base + i] - 1);
-      A.pool[lstart[key] + A.fwd_idx[base + i] - 1] = i + 1;
-    }
-  }
-  __syncthreads();
-  if (t == 0) {
-    B->valid_sort = 1;
-    B->xlists_valid = 1;
-    B->pkeys_valid = 0;
   }
 }
 

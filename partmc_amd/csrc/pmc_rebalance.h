@@ -27,7 +27,7 @@ constexpr int LOSS_INVALID = 0, LOSS_NONE = 1, LOSS_CONSTANT = 2, LOSS_VOLUME = 
               LOSS_DRYDEP = 4, LOSS_CHAMBER = 5;
 
 // what a removal pass removes
-constexpr int RM_HALVE = 0, RM_DILUTE = 1, RM_LOSS = 2;
+constexpr int RM_HALVE = 0, RM_DILUTE = 1, RM_LOSS = 2, RM_OUTSIDE = 3;
 struct Removal {
   int kind;               // RM_*
   int g, c, k;            // halving: the (group, class) and its pass
@@ -237,7 +237,9 @@ __device__ inline double loss_rate(int type, double vol, double density, const E
   }
 }
 
-// Whether slot i of the box goes in this pass.  The particle at 1-based
+// Whether slot i of the box goes in this pass.  A discard of particles
+// outside the box's grid (aero_sorted_discard_outside_grid,
+// src/aero_sorted.F90:153-180) reads their bins; otherwise the particle at 1-based
 // index i draws the first uniform of stream (step, site, i, kind) and goes
 // when it is below its probability: 1/2 for a halving pass of its class,
 // the box's probability for dilution, 1 - exp(-del_t rate) for particle
@@ -249,6 +251,7 @@ __device__ inline bool removal_draw(const Arrays &A, const BoxDesc *B, int box, 
   const int64_t p = B->off + i;
   double prob;
   uint32_t site = 0, kind;
+  if (R.kind == RM_OUTSIDE) return A.fwd_bin[p] < 1 || A.fwd_bin[p] > B->n_bin;
   if (R.kind == RM_HALVE) {
     if (!in_gc(A, p, R.g, R.c)) return false;
     prob = 0.5;
@@ -350,7 +353,7 @@ k_remove_mark(const BoxDesc *boxes, Arrays A, RebalWork R, Removal X, uint64_t s
 }
 
 // Inclusive removal counts per slot, and the removal log in the reference's
-// order (from the last index down).
+// order (from the last index down; discards are not logged, action 0).
 __global__ void __launch_bounds__(REBAL_THREADS)
 k_remove_prefix(BoxDesc *boxes, Arrays A, RebalWork R, int action) {
   const int box = blockIdx.y, t = threadIdx.x;
@@ -369,7 +372,7 @@ k_remove_prefix(BoxDesc *boxes, Arrays A, RebalWork R, int action) {
     const int incl = block_scan_incl<REBAL_THREADS>(flag, OpSum(), ts, &total);
     if (i < n) {
       R.rp[base + i] = done + incl;
-      if (flag) {
+      if (flag && action) {
         const int64_t slot = B->n_info + (n_rm - (done + incl));
         if (slot < B->info_cap) {
           A.info_id[B->info_off + slot] = A.id[base + i];
@@ -409,7 +412,7 @@ __global__ void k_remove_finish(BoxDesc *boxes, RebalWork R, int n_box, Removal 
   if (!R.plan[box] || B->error) return;
   const int n_rm = R.box_tot[box];
   B->n_part -= n_rm;
-  B->n_info += n_rm;
+  if (X.kind != RM_OUTSIDE) B->n_info += n_rm;
   B->xlists_valid = 0;
   B->pkeys_valid = 0;
   B->terms_kernel = 0;

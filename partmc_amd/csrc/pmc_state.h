@@ -40,6 +40,8 @@ struct BoxDesc {
   int bounds_kernel;         // kernel type the cached bounds were made for
   int grid_req_n_bin;        // explicit grid request (-1 = none)
   double grid_req_min, grid_req_max;
+  int prep_sort;             // exact-mode preparation: the box sorts its particles
+  int prep_outside;          // ... and its particles outside an explicit grid
   int error;
   int n_rounds, n_dropped;   // parallel mode: tail claim rounds, dropped samples
   int64_t n_tail_tests;      // parallel mode: tests finished in the tail
