@@ -853,8 +853,13 @@ int pmc_gpu_mc_coag_async(pmc_gpu *h, int kernel_type, double del_t) {
     if ((e = enqueue_prep_lists(h, -1))) return e;
     timing_end(h, "k_prepare", ev);
     if ((e = enqueue_tables(h, kernel_type))) return e;
-    LAUNCH_TIMED(h, "k_exact_sweep", k_exact_sweep, dim3(h->n_box), dim3(64), 0, h->stream,
-                 h->d_box, h->A, kernel_type, del_t, h->seed, h->step);
+    const size_t ws = sweep_bytes(h->max_bin, h->tab_classes);
+    if (ws <= (size_t)SWEEP_LDS)
+      LAUNCH_TIMED(h, "k_exact_sweep", k_exact_sweep<true>, dim3(h->n_box), dim3(64), ws,
+                   h->stream, h->d_box, h->A, kernel_type, del_t, h->seed, h->step);
+    else
+      LAUNCH_TIMED(h, "k_exact_sweep", k_exact_sweep<false>, dim3(h->n_box), dim3(64), 0,
+                   h->stream, h->d_box, h->A, kernel_type, del_t, h->seed, h->step);
     HIPCHECK(hipGetLastError());
   } else {
     e = parallel_step(h->work, h->A, h->d_box, h->n_box, h->cap, h->max_bin, h->stream,

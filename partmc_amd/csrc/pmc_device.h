@@ -146,8 +146,10 @@ struct Stream {
   }
 };
 
-// pmc_rand_int (non-GSL), src/rand.F90:202
-__device__ inline int rand_int(Stream &s, int n) {
+// pmc_rand_int (non-GSL), src/rand.F90:202.  The samplers that a wavefront
+// also draws together take either kind of stream.
+template <class S>
+__device__ inline int rand_int(S &s, int n) {
   double u = s.uniform();
   int k = (int)(u * (double)n);
   return (k % n) + 1;
@@ -164,7 +166,8 @@ __device__ inline double rand_normal_ref(Stream &s, double mean, double stddev) 
 }
 
 // prob_round, src/rand.F90:214-227
-__device__ inline int prob_round(Stream &s, double val) {
+template <class S>
+__device__ inline int prob_round(S &s, double val) {
   if (s.uniform() < ceil(val) - val) return (int)floor(val);
   return (int)ceil(val);
 }
@@ -283,8 +286,26 @@ __device__ inline void sample_without_replacement(Stream &s, int sample_size,
   }
 }
 
+// the same as a mask of the entries taken (bit t - 1 for entry t), in the
+// order of the draws
+template <class S>
+__device__ inline uint64_t sample_mask(S &s, int sample_size, int population_size) {
+  uint64_t mask = 0;
+  int t = 0, m = 0;
+  while (m < sample_size) {
+    const double r = s.uniform();
+    if (!((double)(population_size - t) * r >= (double)(sample_size - m))) {
+      mask |= 1ull << t;
+      m = m + 1;
+    }
+    t = t + 1;
+  }
+  return mask;
+}
+
 // sample_cts_pdf, src/rand.F90:550-576 (1-based)
-__device__ inline int sample_cts_pdf(Stream &s, int n, const double *pdf) {
+template <class S>
+__device__ inline int sample_cts_pdf(S &s, int n, const double *pdf) {
   double pdf_max = pdf[0];
   for (int i = 1; i < n; ++i)
     if (pdf[i] > pdf_max) pdf_max = pdf[i];

@@ -19,7 +19,7 @@ WEIGHTS = ([[1, 1]], [[2.0, 3.0]], [[0.0, 0.0]])
     (1, (10, 1e-9, 1e-5), 256), (63, (40, 1e-9, 1e-5), 256), (65, (1, 1e-9, 1e-5), 256),
     (16384, (150, 1e-9, 1e-5), 256), (16385, (150, 2e-8, 4e-7), 256),
     (40001, (100, 3e-8, 1e-7), 256), (3000, (60, 1e-4, 1e-3), 256),
-    (5000, (900, 1e-9, 1e-5), 900)])
+    (5000, (900, 1e-9, 1e-5), 900), (5000, (900, 1e-9, 1e-5), 1600)])
 def test_set_bin_grid_matches_oracle_sort(n, grid, max_bin):
     rng = np.random.default_rng(n)
     vol = 10 ** rng.uniform(-24, -19.5, size=(n, 1)) * rng.dirichlet([1, 1], size=n)
