@@ -116,6 +116,18 @@ struct Stream {
     have = 0;
     tape = nullptr;
   }
+  // a block by number; the stream's own position stays
+  __host__ __device__ inline void philox_block(uint32_t b, uint32_t o[4]) const {
+    philox4x32_10(c0, c1, c2, c3 | (b & 0xFFFFFFu), k0, k1, o);
+  }
+  // the position after n uniforms of a stream without a tape, with the block
+  // the last one came from when it has another left
+  __host__ __device__ inline void seek(int n, const uint32_t last[4]) {
+    block = (uint32_t)(n + 1) / 2;
+    have = n & 1;
+    buf2 = last[2];
+    buf3 = last[3];
+  }
   __host__ __device__ inline double uniform() {
     if (tape) {
       if (tape->mode == TAPE_REPLAY) {
@@ -613,23 +625,35 @@ __device__ inline double fall_g(double r) {
   double stb = 32.0 * rhoa * (rhow - rhoa) * grav / (3.0 * eta * eta);
   double phy = sigma * sigma * sigma * rhoa * rhoa /
                (powi(eta, 4) * grav * (rhow - rhoa));
-  double py = pow(phy, 1.0 / 6.0);
   double rr = r * 1e2;
   double w = 0.0;
   if (rr <= 1e-3) {
     w = stok * (rr * rr + cunh * rr);
   } else if (rr > 1e-3 && rr <= 5.35e-2) {
     double x = log(stb * rr * rr * rr);
-    double y = 0.0;
-    for (int i = 1; i <= 7; ++i) y = y + b[i - 1] * powi(x, i - 1);
+    // the terms of powi(x, 0..6), with the squares they share formed once
+    const double x2 = x * x, x4 = x2 * x2;
+    double y = 0.0 + b[0];
+    y = y + b[1] * x;
+    y = y + b[2] * x2;
+    y = y + b[3] * (x * x2);
+    y = y + b[4] * x4;
+    y = y + b[5] * (x * x4);
+    y = y + b[6] * (x2 * x4);
     double xrey = (1.0 + cunh / rr) * exp(y);
     w = xrey * eta / (2.0 * rhoa * rr);
   } else if (rr > 5.35e-2) {
     double bond = grav * (rhow - rhoa) * (rr * rr) / sigma;
     if (rr > 0.35) bond = grav * (rhow - rhoa) * (0.35 * 0.35) / sigma;
+    const double py = pow(phy, 1.0 / 6.0);  // only this branch pays for it
     double x = log(16.0 * bond * py / 3.0);
-    double y = 0.0;
-    for (int i = 1; i <= 6; ++i) y = y + c[i - 1] * powi(x, i - 1);
+    const double x2 = x * x, x4 = x2 * x2;
+    double y = 0.0 + c[0];
+    y = y + c[1] * x;
+    y = y + c[2] * x2;
+    y = y + c[3] * (x * x2);
+    y = y + c[4] * x4;
+    y = y + c[5] * (x * x4);
     double xrey = py * exp(y);
     w = xrey * eta / (2.0 * rhoa * rr);
     if (rr > 0.35) w = xrey * eta / (2.0 * rhoa * 0.35);

@@ -49,18 +49,29 @@ constexpr int PAR_ROUNDS = 2;  // device-wide claim rounds before the per-box ta
 static_assert(PAR_ROUNDS >= 1, "the tail runs on the pending list of a round");
 constexpr int MAX_REDRAW = 64;
 
+// What the claims and the list bookkeeping of a step keep per particle slot,
+// in one 32-byte record: an event that touches a particle at random then
+// touches one line (and one page) for all of it, not one per field.  The
+// second half is read as one 16-byte word.
+struct alignas(32) SlotRec {
+  uint32_t claim;     // earliest event that accesses the particle this round
+  uint32_t claim_wr;  // ... and earliest that changes it
+  uint32_t dead_t;    // test index of the winner that consumed it
+  int dead_r;         // claim round (step-wide count) of that winner
+  int key0;           // a touched slot's list key at step start
+  uint32_t depart_t;  // when a touched slot's step-start particle left that list
+  int arr_of;         // pool entry of the arrival a slot holds
+  uint32_t st;        // (epoch << 2) | state; another step's epoch reads as live
+};
+
 struct PW {  // device view of the parallel work arrays
   int K_stride;     // keys per box of the list tables (the allocation's grid)
   int K_hist;       // keys per box of this step's histogram (the step's grid)
   int64_t P_stride; // pair slots per box
   int tab_classes, max_bin;
   int *key;         // [total_cap] list key, -1 for no key
-  uint8_t *status;  // [total_cap] (epoch << 2) | state; another step's epoch reads as live
+  SlotRec *slot;    // [total_cap]
   int epoch;        // this step's status epoch, 1..63
-  uint32_t *claim;  // [total_cap]
-  uint32_t *claim_wr;  // [total_cap] tail: earliest claim of a test that changes the particle
-  uint32_t *dead_t; // [total_cap] test index of the winner that consumed it
-  int *dead_r;      // [total_cap] claim round (step-wide count) of that winner
   float4 *terms;    // [total_cap]
   int *perm;        // [total_cap] global slots sorted by (box, key)
   int *tile_box, *tile_start, *tiles_in_box;
@@ -125,9 +136,6 @@ struct PW {  // device view of the parallel work arrays
   uint32_t *ap_top;   // [1] overflow entries used this step
   int64_t ap_ovf;     // n_box * K_stride * A_MAX
   uint32_t ap_cap;    // overflow entries
-  int *arr_of;        // [total_cap] pool entry of the arrival a slot holds
-  int *key0;          // [total_cap] a touched slot's list key at step start
-  uint32_t *depart_t; // [total_cap] when a touched slot's step-start particle left that list
   uint8_t *thin;      // [T_cap] the test's last draw was thinned (per batch)
   // Per (box, bin): the lowest index of an event pending at the start of
   // this round whose results land in that bin or a lower one (tests on an
@@ -512,14 +520,33 @@ k_par_scatter(BoxDesc *boxes, PW W, int key_bits) {
   }
 }
 
+// 64-bit divisions take about five times a 32-bit one: used only where an
+// operand needs them.
 __device__ inline void decode_pair(int64_t q, int tc, int mb, int *c1, int *c2, int *b1, int *b2) {
-  int64_t mb2 = (int64_t)mb * mb;
-  int cls = (int)(q / mb2);
-  int rem = (int)(q % mb2);
-  *c1 = cls / tc + 1;
-  *c2 = cls % tc + 1;
-  *b1 = rem / mb + 1;
-  *b2 = rem % mb + 1;
+  uint32_t cls, rem;
+  if (((uint64_t)q >> 32) == 0) {
+    const uint32_t mb2 = (uint32_t)mb * (uint32_t)mb;
+    cls = (uint32_t)q / mb2;
+    rem = (uint32_t)q - cls * mb2;
+  } else {
+    const int64_t mb2 = (int64_t)mb * mb;
+    cls = (uint32_t)(q / mb2);
+    rem = (uint32_t)(q % mb2);
+  }
+  const uint32_t k1 = cls / (uint32_t)tc, r1 = rem / (uint32_t)mb;
+  *c1 = (int)k1 + 1;
+  *c2 = (int)(cls - k1 * (uint32_t)tc) + 1;
+  *b1 = (int)r1 + 1;
+  *b2 = (int)(rem - r1 * (uint32_t)mb) + 1;
+}
+
+// the box of global pair k, and the pair's index in it
+__device__ inline int pair_box(const PW &W, int64_t k, int64_t *q) {
+  int box;
+  if (((uint64_t)(k | W.P_stride) >> 32) == 0) box = (int)((uint32_t)k / (uint32_t)W.P_stride);
+  else box = (int)(k / W.P_stride);
+  *q = k - (int64_t)box * W.P_stride;
+  return box;
 }
 
 // the record without its components (they are read in a second pass
@@ -716,18 +743,23 @@ __device__ inline void atomic_max_double(double *addr, double v) {
 // set them, so a new step starts with every particle live without clearing
 // the array (it is cleared when the epoch wraps).
 __device__ inline uint8_t st_get(const PW &W, int64_t p) {
-  const uint8_t v = W.status[p];
+  const uint32_t v = W.slot[p].st;
   return (int)(v >> 2) == W.epoch ? (uint8_t)(v & 3) : ST_LIVE;
 }
 __device__ inline void st_set(const PW &W, int64_t p, uint8_t s) {
-  W.status[p] = (uint8_t)((W.epoch << 2) | s);
+  W.slot[p].st = (uint32_t)((W.epoch << 2) | s);
 }
 
 // a slot of a step-start list can be drawn while it holds a particle of
 // that list's (bin, class): untouched, or changed in place by an earlier
 // merge without leaving the list
+__device__ inline bool drawable_as(const PW &W, uint32_t st, int key_p, int key) {
+  return !((int)(st >> 2) == W.epoch && (st & 3) == ST_HOLE) && key_p == key;
+}
 __device__ inline bool drawable(const PW &W, int p, int key) {
-  return st_get(W, p) != ST_HOLE && W.key[p] == key;
+  const uint32_t st = W.slot[p].st;
+  const int key_p = W.key[p];
+  return drawable_as(W, st, key_p, key);
 }
 
 // ---- list membership within a step
@@ -741,28 +773,25 @@ __device__ inline bool drawable(const PW &W, int p, int key) {
 // of the members present when the pair begins.  Within the pair, a member
 // that left after the pair began is drawn again among the present ones.
 
-// the first change of slot p in this step: remember its step-start key
 // The fields of slot p that the list bookkeeping reads, loaded together
-// (one memory round trip instead of a chain of them); a slot first touched
-// this step records its step-start list and no departure yet.
+// (one memory round trip instead of a chain of them).
 struct SlotView {
   int key, key0, e;
-  uint32_t dep;
+  uint32_t dep, st;
 };
-__device__ inline SlotView slot_touch(const PW &W, int64_t p) {
-  SlotView v;
-  const uint8_t stv = W.status[p];
-  v.key = W.key[p];
-  v.key0 = W.key0[p];
-  v.dep = W.depart_t[p];
-  v.e = W.arr_of[p];
-  if ((int)(stv >> 2) != W.epoch || (stv & 3) == ST_LIVE) {
+__device__ inline SlotView slot_load(const PW &W, int64_t p) {
+  const uint4 h = *(const uint4 *)&W.slot[p].key0;
+  return SlotView{W.key[p], (int)h.x, (int)h.z, h.y, h.w};
+}
+// a slot first changed this step records its step-start list and no
+// departure yet
+__device__ inline void slot_touch(const PW &W, int64_t p, SlotView &v) {
+  if ((int)(v.st >> 2) != W.epoch || (v.st & 3) == ST_LIVE) {
     v.key0 = v.key;
     v.dep = UNCLAIMED;
-    W.key0[p] = v.key;
-    W.depart_t[p] = UNCLAIMED;
+    W.slot[p].key0 = v.key;
+    W.slot[p].depart_t = UNCLAIMED;
   }
-  return v;
 }
 
 // An arrival takes the next entry of its list's array, or past A_MAX of
@@ -789,7 +818,7 @@ __device__ inline void record_arrival(const PW &W, BoxDesc *B, int box, int key,
   W.ap_p[e] = (int)p;
   W.ap_t[e] = t;
   W.ap_dep[e] = UNCLAIMED;
-  W.arr_of[p] = (int)e;
+  W.slot[p].arr_of = (int)e;
   atomicAdd((unsigned long long *)&B->n_arrivals, 1ull);
   if (i < A_MAX) return;
   int old = __hip_atomic_load(&W.arr_head[L], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -817,7 +846,7 @@ __device__ inline void arrivals_each(const PW &W, int64_t L, F f) {
 __device__ inline void slot_leave_view(const PW &W, int64_t p, uint32_t t, const SlotView &v) {
   if (v.key < 0) return;
   if (v.key == v.key0 && v.dep == UNCLAIMED) {
-    W.depart_t[p] = t;  // the slot's step-start member
+    W.slot[p].depart_t = t;  // the slot's step-start member
     return;
   }
   const int e = v.e;  // an arrival of list v.key
@@ -825,16 +854,20 @@ __device__ inline void slot_leave_view(const PW &W, int64_t p, uint32_t t, const
     W.ap_dep[e] = t;
 }
 
+__device__ inline void slot_leave(const PW &W, int64_t p, uint32_t t, SlotView v) {
+  slot_touch(W, p, v);
+  slot_leave_view(W, p, t, v);
+}
 __device__ inline void slot_leave(const PW &W, int64_t p, uint32_t t) {
-  slot_leave_view(W, p, t, slot_touch(W, p));
+  slot_leave(W, p, t, slot_load(W, p));
 }
 
 // slot p receives a particle of list new_key in place of the one it held
 // (a merge into a parent's slot, a target merged in place): the old one
 // leaves its list at t_leave, the new one joins at t_join
 __device__ inline void slot_write(const PW &W, BoxDesc *B, int box, int64_t p, uint32_t t_leave,
-                                  uint32_t t_join, int new_key) {
-  const SlotView v = slot_touch(W, p);
+                                  uint32_t t_join, int new_key, SlotView v) {
+  slot_touch(W, p, v);
   if (v.key == new_key) return;  // changed in place, still in its list
   slot_leave_view(W, p, t_leave, v);
   if (new_key != v.key0) record_arrival(W, B, box, new_key, p, t_join);
@@ -843,8 +876,8 @@ __device__ inline void slot_write(const PW &W, BoxDesc *B, int box, int64_t p, u
 // an appended slot receives a particle of list new_key at sequence index t
 __device__ inline void slot_append(const PW &W, BoxDesc *B, int box, int64_t p, uint32_t t,
                                    int new_key) {
-  W.key0[p] = -1;
-  W.depart_t[p] = 0;
+  W.slot[p].key0 = -1;
+  W.slot[p].depart_t = 0;
   record_arrival(W, B, box, new_key, p, t);
 }
 
@@ -865,11 +898,11 @@ __device__ inline uint32_t mix32(uint32_t h) {
 // which one is drawn uniformly among them (not `exclude`, the first draw of
 // a test on the same list) as the one whose slot hashes lowest under u.  So
 // each arrival present at tau is drawn at the rate of a member.  Returns
-// the pool entry, or -1.
+// the pool entry and its slot, or -1.
 constexpr int ACHUNK = 8;  // arrival entries loaded together
 
 __device__ inline int64_t arrival_draw(const PW &W, int64_t L, int j, uint32_t tau, uint32_t u,
-                                       int exclude) {
+                                       int exclude, int *p_out) {
   int n_before = 0;
   int64_t best = -1;
   uint32_t best_h = 0;
@@ -905,6 +938,7 @@ __device__ inline int64_t arrival_draw(const PW &W, int64_t L, int j, uint32_t t
   }
   if (n > A_MAX)
     for (int e = W.arr_head[L]; e >= 0; e = W.ap_next[e]) consider((int64_t)e, W.ap_t[e], W.ap_p[e]);
+  *p_out = best_p;
   return j <= n_before ? best : -1;
 }
 
@@ -933,16 +967,24 @@ __device__ inline int64_t arrival_rank(const PW &W, int64_t L, int r, uint32_t t
 // reserved entry takes one more draw from `ts` to pick its arrival.
 __device__ inline int draw_entry(const PW &W, int64_t base, int64_t L, int key, int n, int s,
                                  int c, uint32_t tau, Stream &ts, int exclude) {
+  // (the fields that decide are loaded together, needed or not)
   if (c <= n) {
     const int p = W.perm[base + s + c - 1];
-    if (drawable(W, p, key)) return p;
-    return W.depart_t[p] < tau ? DRAW_THIN : DRAW_AGAIN;
+    const uint32_t stv = W.slot[p].st;
+    const int kp = W.key[p];
+    const uint32_t dep = W.slot[p].depart_t;
+    if (drawable_as(W, stv, kp, key)) return p;
+    return dep < tau ? DRAW_THIN : DRAW_AGAIN;
   }
   const uint32_t u = (uint32_t)(ts.uniform() * 4294967296.0);
-  const int64_t e = arrival_draw(W, L, c - n, tau, u, exclude);
-  if (e < 0 || W.ap_dep[e] < tau) return DRAW_ATHIN;
-  const int p = W.ap_p[e];
-  return drawable(W, p, key) ? p : DRAW_AGAIN;
+  int p;
+  const int64_t e = arrival_draw(W, L, c - n, tau, u, exclude, &p);
+  if (e < 0) return DRAW_ATHIN;
+  const uint32_t dep = W.ap_dep[e];
+  const uint32_t stv = W.slot[p].st;
+  const int kp = W.key[p];
+  if (dep < tau) return DRAW_ATHIN;
+  return drawable_as(W, stv, kp, key) ? p : DRAW_AGAIN;
 }
 
 // reserved arrival entries and a fresh arrival log for every list: lists
@@ -1004,18 +1046,19 @@ struct TestOut {
             // arrival entry of the first (second) list
 };
 
-__device__ __forceinline__ void perset_test(BoxDesc *B, const Arrays &A, const PW &W, int box, int64_t k,
-                                   uint32_t t, int type, uint64_t seed, uint32_t step,
-                                   int precision, double band, int validation, TestOut &o,
-                                        const Weights *wl = nullptr) {
+__device__ __forceinline__ void perset_test(BoxDesc *B, const Arrays &A, const PW &W, int box,
+                                            int64_t k, int64_t q, uint32_t t, int type,
+                                            uint64_t seed, uint32_t step, int precision,
+                                            double band, int validation, TestOut &o,
+                                            const Weights *wl = nullptr) {
   o.p1 = o.p2 = -1;
   o.accept = false;
   o.warn = false;
   o.thin = 0;
   int c1, c2, b1, b2;
-  decode_pair(k % W.P_stride, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
-  const uint32_t j = t - W.pair_exc[k];
+  decode_pair(q, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
   const uint32_t tau = W.pair_exc[k];  // where the pair begins in the sequence
+  const uint32_t j = t - tau;
   const Weights &w = wl ? *wl : B->w;
   const int nb = B->n_bin, nc = w.n_class;
   const int64_t ti = table_index(A, box, nb, nc, b1, b2, c1, c2);
@@ -1123,8 +1166,9 @@ __device__ inline MergeCtx merge_ctx(BoxDesc *boxes, const PW &W, int n_box, uin
   MergeCtx m;
   const int64_t NP = (int64_t)n_box * W.P_stride;
   const int64_t k = test_pair(W, NP, t);
-  m.box = (int)(k / W.P_stride);
-  decode_pair(k % W.P_stride, W.tab_classes, W.max_bin, &m.c1, &m.c2, &m.b1, &m.b2);
+  int64_t q;
+  m.box = pair_box(W, k, &q);
+  decode_pair(q, W.tab_classes, W.max_bin, &m.c1, &m.c2, &m.b1, &m.b2);
   m.j = t - W.pair_exc[k];
   return m;
 }
@@ -1137,24 +1181,45 @@ __device__ inline int merge_decide(const Arrays &A, const PW &W, const BoxDesc *
                                    int *new_group, const Weights *wl = nullptr) {
   const Weights &w = wl ? *wl : B->w;
   // the parents' volumes and lists, read together up front
-  const double v1 = particle_volume(A, p1), v2 = particle_volume(A, p2);
+  const double v1 = A.vtot[p1], v2 = A.vtot[p2];
   const int key_p1 = W.key[p1], key_p2 = W.key[p2];
+  // With one group its draw always stands (its pdf over the largest is 1),
+  // and the three uniforms after it come from blocks 1 and 2, drawn side by
+  // side; s stands after them as it would draw by draw.
+  const bool one = w.n_group == 1;
+  uint32_t o1[4], o2[4];
+  if (one) {
+    s.philox_block(1, o1);
+    s.philox_block(2, o2);
+    s.seek(5, o2);
+  }
   double r1 = vol2rad(v1);
   double r2 = vol2rad(v2);
   double rc = vol2rad(rad2vol(r1) + rad2vol(r2));
   double nc1 = nc_at_radius(w, c1, r1);
   double nc2 = nc_at_radius(w, c2, r2);
   double ncc = nc_at_radius(w, cc, rc);
-  double pdf[MAX_GROUP];
-  for (int g = 0; g < w.n_group; ++g) {
-    int idx = g + w.n_group * (cc - 1);
-    pdf[g] = 1.0 / weight_nc(w.type[idx], w.mag[idx], w.expo[idx], rc);
+  double u1, u2, u3;
+  if (one) {
+    *new_group = 1;
+    u1 = u52(o1[0], o1[1]);
+    u2 = u52(o1[2], o1[3]);
+    u3 = u52(o2[0], o2[1]);
+  } else {
+    double pdf[MAX_GROUP];
+    for (int g = 0; g < w.n_group; ++g) {
+      int idx = g + w.n_group * (cc - 1);
+      pdf[g] = 1.0 / weight_nc(w.type[idx], w.mag[idx], w.expo[idx], rc);
+    }
+    *new_group = sample_cts_pdf(s, w.n_group, pdf);
+    u1 = s.uniform();
+    u2 = s.uniform();
+    u3 = s.uniform();
   }
-  *new_group = sample_cts_pdf(s, w.n_group, pdf);
   double nc_min = fmin(nc1, fmin(nc2, ncc));
-  bool rm1 = s.uniform() < nc_min / nc1;
-  bool rm2 = s.uniform() < nc_min / nc2;
-  bool cr = s.uniform() < nc_min / ncc;
+  bool rm1 = u1 < nc_min / nc1;
+  bool rm2 = u2 < nc_min / nc2;
+  bool cr = u3 < nc_min / ncc;
   int o = 0;
   if (rm1) o |= O_RM1;
   if (rm2) o |= O_RM2;
@@ -1196,17 +1261,17 @@ __device__ inline int merge_decide(const Arrays &A, const PW &W, const BoxDesc *
 // it win together, a test that changes it waits for earlier readers, and a
 // reader waits for earlier writers.
 __device__ inline void claim_write(const PW &W, int p, uint32_t t) {
-  atomicMin(&W.claim[p], t);
-  atomicMin(&W.claim_wr[p], t);
+  atomicMin(&W.slot[p].claim, t);
+  atomicMin(&W.slot[p].claim_wr, t);
 }
 
 // the merge decisions of an accepted per-set test (which parents it
 // removes), on the particles as they are before the round's winners apply
 __device__ inline int perset_decide(BoxDesc *B, const Arrays &A, const PW &W, int box, int64_t k,
-                                    uint32_t t, int p1, int p2, uint64_t seed, uint32_t step,
-                                    Stream &ms) {
+                                    int64_t q, uint32_t t, int p1, int p2, uint64_t seed,
+                                    uint32_t step, Stream &ms) {
   int c1, c2, b1, b2;
-  decode_pair(k % W.P_stride, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
+  decode_pair(q, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
   const int nb = B->n_bin, nc = B->w.n_class;
   const int cc = A.cc[table_index(A, box, nb, nc, b1, b2, c1, c2)];
   ms.open(seed, box, step, pair_site(nb, nc, b1, b2, c1, c2), t - W.pair_exc[k], RNG_MERGE);
@@ -1234,11 +1299,12 @@ __device__ __forceinline__ void par_test(BoxDesc *boxes, const Arrays &A, const 
   W.tp2[i] = -1;
   W.trec[i] = -1;
   W.tns[i] = 0;
-  const int box = (int)(k / W.P_stride);
+  int64_t q;
+  const int box = pair_box(W, k, &q);
   BoxDesc *B = &boxes[box];
   if (B->error) return;
   TestOut o;
-  perset_test(B, A, W, box, k, t, type, seed, step, precision, band, validation, o);
+  perset_test(B, A, W, box, k, q, t, type, seed, step, precision, band, validation, o);
   W.tp1[i] = o.p1;
   W.tp2[i] = o.p2;
   W.thin[t - t0] = o.thin ? 1 : 0;
@@ -1248,11 +1314,11 @@ __device__ __forceinline__ void par_test(BoxDesc *boxes, const Arrays &A, const 
   if (o.accept) {
     W.acc[i] = 1;
     Stream ms;
-    const int d = perset_decide(B, A, W, box, k, t, o.p1, o.p2, seed, step, ms);
+    const int d = perset_decide(B, A, W, box, k, q, t, o.p1, o.p2, seed, step, ms);
     if (d & O_RM1) claim_write(W, o.p1, t);
-    else atomicMin(&W.claim[o.p1], t);
+    else atomicMin(&W.slot[o.p1].claim, t);
     if (d & O_RM2) claim_write(W, o.p2, t);
-    else atomicMin(&W.claim[o.p2], t);
+    else atomicMin(&W.slot[o.p2].claim, t);
   }
 }
 
@@ -1543,7 +1609,7 @@ __device__ inline int acc_sample_source(const Arrays &A, const PW &W, BoxDesc *B
         ps = q;
         break;
       }
-      if (a == 0 && !drawable(W, q, skey) && W.depart_t[q] < tau) {
+      if (a == 0 && !drawable(W, q, skey) && W.slot[q].depart_t < tau) {
         thinned = true;
         break;
       }
@@ -1593,7 +1659,7 @@ __device__ inline int acc_sample_source(const Arrays &A, const PW &W, BoxDesc *B
   // the samples the early exit left undrawn thin as the drawn ones did
   for (int i = i_samp; i <= n_total; ++i) {
     const int q = W.perm[sbase + rand_int(smp, n_s) - 1];
-    if (!drawable(W, q, skey) && W.depart_t[q] < tau) n_thin++;
+    if (!drawable(W, q, skey) && W.slot[q].depart_t < tau) n_thin++;
   }
   double prob_coag_mean = prob_coag_tot / (double)n_samp;
   if (!(prob_coag_mean <= 1.0)) *warn = 1;
@@ -1660,15 +1726,14 @@ __device__ __noinline__ int acc_visit(BoxDesc *boxes, const Arrays &A, const PW 
                                       double del_t, bool claim, int *p_out, int *tns) {
   *p_out = -1;
   *tns = 0;
-  const int box = (int)(k / W.P_stride);
+  int64_t q;
+  const int box = pair_box(W, k, &q);
   BoxDesc *B = &boxes[box];
   if (B->error) return -1;
   const int nb = B->n_bin, nc = B->w.n_class;
   const int64_t lb = (int64_t)box * W.K_stride;
-  const int64_t pb = (int64_t)box * W.P_stride;
   const double *edges = A.edges + (int64_t)box * (A.max_bin + 1);
   int c1, c2, b1, b2;
-  const int64_t q = k - pb;
   decode_pair(q, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
   const int kind = W.pair_acc[k];
   const int bt = kind == 1 ? b1 : b2, ct = kind == 1 ? c1 : c2;
@@ -1888,9 +1953,9 @@ __device__ inline void resolve_event(BoxDesc *boxes, const Arrays &A, const PW &
   if (r >= 0) {
     // a target event wins when it holds the target and every removed source
     // ... and no earlier event claimed a source it read
-    bool win = W.claim[p1] == t;
-    rm_walk(W, r, [&](int q) { win = win && W.claim[q] == t; });
-    rd_walk(W, r, [&](int q) { win = win && W.claim_wr[q] >= t; });
+    bool win = W.slot[p1].claim == t;
+    rm_walk(W, r, [&](int q) { win = win && W.slot[q].claim == t; });
+    rd_walk(W, r, [&](int q) { win = win && W.slot[q].claim_wr >= t; });
     const int died = (W.r_flags[r] & RF_DIED) ? 1 : 0;
     W.ev_out[e] = win ? O_WIN : 0;
     W.f_app[e] = win ? W.r_ndup[r] : 0;
@@ -1909,8 +1974,8 @@ __device__ inline void resolve_event(BoxDesc *boxes, const Arrays &A, const PW &
   s.open(seed, m.box, step, pair_site(nb, nc, m.b1, m.b2, m.c1, m.c2), m.j, RNG_MERGE);
   int g;
   const int d = merge_decide(A, W, B, s, p1, p2, m.c1, m.c2, cc, &g);
-  const bool win = ((d & O_RM1) ? W.claim[p1] == t : W.claim_wr[p1] > t) &&
-                   ((d & O_RM2) ? W.claim[p2] == t : W.claim_wr[p2] > t);
+  const bool win = ((d & O_RM1) ? W.slot[p1].claim == t : W.slot[p1].claim_wr > t) &&
+                   ((d & O_RM2) ? W.slot[p2].claim == t : W.slot[p2].claim_wr > t);
   int o = 0;
   if (win) o = d | O_WIN | (g << 16);
   W.ev_out[e] = o;
@@ -1967,7 +2032,7 @@ __device__ inline void write_new_particle(const Arrays &A, const PW &W, BoxDesc 
   }
   int k = par_key(b, r.klass, nb);
   if (appended) slot_append(W, B, box, slot, t_join, k);
-  else slot_write(W, B, box, slot, t_leave, t_join, k);
+  else slot_write(W, B, box, slot, t_leave, t_join, k, slot_load(W, slot));
   st_set(W, slot, ST_NEW);
   W.key[slot] = k;
   if (want_terms) W.terms[slot] = particle_terms(type, v, m / v, B->env);
@@ -2100,84 +2165,168 @@ __device__ inline void put_info(const Arrays &A, BoxDesc *B, Alloc &al, int64_t 
   }
 }
 
-// Both parents' components, read before any is written (dst may be either
-// parent's slot) and all in flight at once.  The loads are unconditional
-// (every one of a particle's MAX_COMP entries, which sit together): a load
-// under `if (c < n)` becomes a branch, and the compiler waits for every
-// load in flight at each one, one memory round trip per component.
-__device__ inline void load_comps2(const Arrays &A, int64_t p1, int64_t p2, int n1, int n2,
-                                   int *s1, double *t1, int *s2, double *t2) {
-  (void)n1;
-  (void)n2;
+// A particle's components, all MAX_COMP of them in wide loads that go out
+// together (a particle's 80 and 160 bytes are 16-byte aligned).  A load under
+// `if (c < n)` becomes a branch, and the compiler waits for every load in
+// flight at each one, one memory round trip per component.
+__device__ inline void load_comps(const Arrays &A, int64_t p, int *s, double *t) {
+  static_assert(MAX_COMP % 4 == 0, "whole 16-byte words");
+  const int4 *ps = (const int4 *)(A.csrc + comp_at(p, 0));
+  const double2 *pt = (const double2 *)(A.ctime + comp_at(p, 0));
 #pragma unroll
-  for (int c = 0; c < MAX_COMP; ++c) {
-    s1[c] = A.csrc[comp_at(p1, c)];
-    t1[c] = A.ctime[comp_at(p1, c)];
-    s2[c] = A.csrc[comp_at(p2, c)];
-    t2[c] = A.ctime[comp_at(p2, c)];
+  for (int c = 0; c < MAX_COMP / 4; ++c) {
+    const int4 x = ps[c];
+    s[4 * c] = x.x;
+    s[4 * c + 1] = x.y;
+    s[4 * c + 2] = x.z;
+    s[4 * c + 3] = x.w;
+  }
+#pragma unroll
+  for (int c = 0; c < MAX_COMP / 2; ++c) {
+    const double2 x = pt[c];
+    t[2 * c] = x.x;
+    t[2 * c + 1] = x.y;
   }
 }
 
-// the merged particle's components when the parents hold more than
+// Which components the merged particle keeps when the parents hold more than
 // MAX_COMP together (aero_particle_coagulate, src/aero_particle.F90:
 // 917-1033): prob_round of the first parent's share, then two selection
-// samples (sample_without_replacement keeps sorted order) from the parents'
-// components, which are read into registers first; the loops are unrolled
-// so the arrays stay in registers.
+// samples (sample_without_replacement keeps sorted order).  take: a bit per
+// component of each parent; returns the first parent's share.
+template <class S>
+__device__ inline int resample_masks(S &s, int n1, int n2, int np1, int np2, uint32_t *take1,
+                                     uint32_t *take2) {
+  const int n1_new = prob_round(s, (double)np1 / (double)(np1 + np2) * (double)MAX_COMP);
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const int n = side ? n2 : n1, want = side ? MAX_COMP - n1_new : n1_new;
+    uint32_t take = 0;
+    int m = 0;
+    for (int c = 0; c < n && m < want; ++c) {
+      const double r = s.uniform();
+      if (!((double)(n - c) * r >= (double)(want - m))) {
+        take |= 1u << c;
+        m++;
+      }
+    }
+    (side ? *take2 : *take1) = take;
+  }
+  return n1_new;
+}
+
 __device__ inline void resample_components(const Arrays &A, Stream &s, int64_t p1, int64_t p2,
                                            int64_t dst, int n1, int n2, int np1, int np2) {
   int s1[MAX_COMP], s2[MAX_COMP];
   double t1[MAX_COMP], t2[MAX_COMP];
-  load_comps2(A, p1, p2, n1, n2, s1, t1, s2, t2);
-  const int n1_new = prob_round(s, (double)np1 / (double)(np1 + np2) * (double)MAX_COMP);
-  const int n2_new = MAX_COMP - n1_new;
-  // first parent: n1_new of its n1 components into positions 0 ..
-  {
-    int m = 0;
+  load_comps(A, p1, s1, t1);
+  load_comps(A, p2, s2, t2);
+  uint32_t take1, take2;
+  const int n1_new = resample_masks(s, n1, n2, np1, np2, &take1, &take2);
+  int m1 = 0, m2 = n1_new;
 #pragma unroll
-    for (int c = 0; c < MAX_COMP; ++c) {
-      if (c < n1 && m < n1_new) {
-        const double r = s.uniform();
-        if (!((double)(n1 - c) * r >= (double)(n1_new - m))) {
-          A.csrc[comp_at(dst, m)] = s1[c];
-          A.ctime[comp_at(dst, m)] = t1[c];
-          m++;
-        }
-      }
+  for (int c = 0; c < MAX_COMP; ++c) {
+    if ((take1 >> c) & 1u) {
+      A.csrc[comp_at(dst, m1)] = s1[c];
+      A.ctime[comp_at(dst, m1)] = t1[c];
+      ++m1;
     }
   }
-  // second parent: n2_new of its n2 components after them
-  {
-    int m = 0;
 #pragma unroll
-    for (int c = 0; c < MAX_COMP; ++c) {
-      if (c < n2 && m < n2_new) {
-        const double r = s.uniform();
-        if (!((double)(n2 - c) * r >= (double)(n2_new - m))) {
-          A.csrc[comp_at(dst, n1_new + m)] = s2[c];
-          A.ctime[comp_at(dst, n1_new + m)] = t2[c];
-          m++;
-        }
-      }
+  for (int c = 0; c < MAX_COMP; ++c) {
+    if ((take2 >> c) & 1u) {
+      A.csrc[comp_at(dst, m2)] = s2[c];
+      A.ctime[comp_at(dst, m2)] = t2[c];
+      ++m2;
     }
   }
+}
+
+// One lane's resampling by its whole wavefront: about 40 uniforms of one
+// stream are 20 Philox blocks, one a lane, and the components go through the
+// lanes.  Every lane takes part; the arguments are the resampling lane's,
+// broadcast.  i0: the stream's next uniform.  A drizzle drop's merge spends
+// 13 us on this alone on one lane, about 4 here.
+struct LaneUniforms {
+  double a, b;  // this lane's block
+  int at;
+  __device__ inline double uniform() {
+    const double v = __shfl((at & 1) ? b : a, at >> 1);
+    ++at;
+    return v;
+  }
+};
+__device__ inline void wave_resample(const Arrays &A, const Stream &s, int i0, int64_t p1,
+                                     int64_t p2, int64_t dst, int n1, int n2, int np1, int np2) {
+  const int lane = threadIdx.x & 63;
+  int s1 = 0, s2 = 0;
+  double t1 = 0.0, t2 = 0.0;
+  if (lane < MAX_COMP) {
+    s1 = A.csrc[comp_at(p1, lane)];
+    t1 = A.ctime[comp_at(p1, lane)];
+    s2 = A.csrc[comp_at(p2, lane)];
+    t2 = A.ctime[comp_at(p2, lane)];
+  }
+  uint32_t o[4];
+  s.philox_block((uint32_t)(i0 >> 1) + lane, o);
+  LaneUniforms u{u52(o[0], o[1]), u52(o[2], o[3]), i0 & 1};
+  uint32_t take1, take2;
+  const int n1_new = resample_masks(u, n1, n2, np1, np2, &take1, &take2);
+  const uint32_t below = lane < 32 ? (1u << lane) - 1u : 0u;
+  if (lane < MAX_COMP) {
+    if ((take1 >> lane) & 1u) {
+      const int c = __popc(take1 & below);
+      A.csrc[comp_at(dst, c)] = s1;
+      A.ctime[comp_at(dst, c)] = t1;
+    }
+    if ((take2 >> lane) & 1u) {
+      const int c = n1_new + __popc(take2 & below);
+      A.csrc[comp_at(dst, c)] = s2;
+      A.ctime[comp_at(dst, c)] = t2;
+    }
+  }
+}
+
+// What a merge reads of its parents, loaded together before anything is
+// written: one memory round trip where reading each field as it is needed,
+// between the stores, costs one apiece (in the tail of 3e5-drop boxes 1.2 us
+// left of 6.3, the rest behind the claims' barrier).
+struct MergeParents {
+  SlotView v1, v2;
+  int64_t id1, id2;
+  int n1, n2, np1, np2;
+  double least, greatest;
+};
+__device__ inline MergeParents load_parents(const Arrays &A, const PW &W, int64_t p1, int64_t p2) {
+  MergeParents P;
+  P.v1 = slot_load(W, p1);
+  P.v2 = slot_load(W, p2);
+  P.id1 = A.id[p1];
+  P.id2 = A.id[p2];
+  P.n1 = A.ncomp[p1];
+  P.n2 = A.ncomp[p2];
+  P.np1 = A.nprim[p1];
+  P.np2 = A.nprim[p2];
+  const double l1 = A.least[p1], l2 = A.least[p2], g1 = A.greatest[p1], g2 = A.greatest[p2];
+  P.least = fmin(l1, l2);
+  P.greatest = fmax(g1, g2);
+  return P;
 }
 
 // the merged particle of an accepted per-set test written straight from
 // its parents' slots into dst (which may be either parent's slot):
 // aero_particle_coagulate (src/aero_particle.F90:917-1033).  Components
 // are concatenated, or resampled on `rs` (the merge stream after the merge
-// decisions) when the parents hold more than MAX_COMP together.
+// decisions) when the parents hold more than MAX_COMP together, unless the
+// wavefront has done so already.
 __device__ inline int direct_merge(const Arrays &A, const PW &W, BoxDesc *B, int box, uint32_t t,
                                    int64_t p1, int64_t p2, int64_t dst, bool appended, int64_t id,
-                                   int group, int klass, int type, int want_terms, Stream *rs) {
+                                   int group, int klass, int type, int want_terms, Stream *rs,
+                                   const MergeParents &P, bool resampled) {
   const int64_t tc = A.total_cap;
-  const int n1 = A.ncomp[p1], n2 = A.ncomp[p2];
-  const int np1 = A.nprim[p1], np2 = A.nprim[p2];
-  if (np1 < n1) return 465791384;
-  if (np2 < n2) return 465791385;
-  const double least = fmin(A.least[p1], A.least[p2]);
-  const double greatest = fmax(A.greatest[p1], A.greatest[p2]);
+  const int n1 = P.n1, n2 = P.n2;
+  if (P.np1 < n1) return 465791384;
+  if (P.np2 < n2) return 465791385;
   // dst may be a parent's slot: each species' sum depends only on its own
   // row, so it is written once formed; a chunk's loads go out together
   double v = 0.0, m = 0.0;
@@ -2200,36 +2349,41 @@ __device__ inline int direct_merge(const Arrays &A, const PW &W, BoxDesc *B, int
     }
   }
   // components: the first parent's, then the second's, all loaded before
-  // any is written (dst may be a parent's slot), so the loads go out
-  // together
+  // any is written; the first parent's are in place when it is the slot
   int n_out = n1 + n2;
   if (n1 + n2 > MAX_COMP) {
-    resample_components(A, *rs, p1, p2, dst, n1, n2, np1, np2);
+    if (!resampled) resample_components(A, *rs, p1, p2, dst, n1, n2, P.np1, P.np2);
     n_out = MAX_COMP;
   } else {
-    int s1[MAX_COMP], s2[MAX_COMP];
-    double t1[MAX_COMP], t2[MAX_COMP];
-    load_comps2(A, p1, p2, n1, n2, s1, t1, s2, t2);
+    int s2[MAX_COMP];
+    double t2[MAX_COMP];
+    load_comps(A, p2, s2, t2);
+    if (dst != p1) {
+      int s1[MAX_COMP];
+      double t1[MAX_COMP];
+      load_comps(A, p1, s1, t1);
 #pragma unroll
-    for (int c = 0; c < MAX_COMP; ++c) {
-      if (c < n1) {
-        A.csrc[comp_at(dst, c)] = s1[c];
-        A.ctime[comp_at(dst, c)] = t1[c];
-      }
+      for (int c = 0; c < MAX_COMP; ++c)
+        if (c < n1) {
+          A.csrc[comp_at(dst, c)] = s1[c];
+          A.ctime[comp_at(dst, c)] = t1[c];
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < MAX_COMP; ++c)
       if (c < n2) {
         A.csrc[comp_at(dst, n1 + c)] = s2[c];
         A.ctime[comp_at(dst, n1 + c)] = t2[c];
       }
-    }
   }
   A.vtot[dst] = v;
   A.id[dst] = id;
   A.group[dst] = group;
   A.klass[dst] = klass;
-  A.nprim[dst] = np1 + np2;
+  A.nprim[dst] = P.np1 + P.np2;
   A.ncomp[dst] = n_out;
-  A.least[dst] = least;
-  A.greatest[dst] = greatest;
+  A.least[dst] = P.least;
+  A.greatest[dst] = P.greatest;
   const int nb = B->n_bin;
   const int b = bin_find_log(nb, B->log_lo, B->log_hi, vol2rad(v));
   if (b < 1 || b > nb) {
@@ -2239,7 +2393,7 @@ __device__ inline int direct_merge(const Arrays &A, const PW &W, BoxDesc *B, int
   }
   const int k_new = par_key(b, klass, nb);
   if (appended) slot_append(W, B, box, dst, t, k_new);
-  else slot_write(W, B, box, dst, t, t, k_new);
+  else slot_write(W, B, box, dst, t, t, k_new, dst == p1 ? P.v1 : P.v2);
   st_set(W, dst, ST_NEW);
   W.key[dst] = k_new;
   if (want_terms) W.terms[dst] = particle_terms(type, v, m / v, B->env);
@@ -2247,41 +2401,35 @@ __device__ inline int direct_merge(const Arrays &A, const PW &W, BoxDesc *B, int
 }
 
 // coagulate_weighting + coagulate (src/coagulation.F90:810-985) of an
-// accepted per-set test: removals become holes (or the slot the merged
-// particle takes), the merged particle is written, removal records follow
-// the reference's order.  o_known >= 0 passes the outcome of merge_decide
-// already taken on this test's stream (with the new group in bits 16+),
-// and post, if given, that stream after them.
+// accepted per-set test, o the decisions of merge_decide: removals become
+// holes (or the slot the merged particle takes), the merged particle is
+// written, removal records follow the reference's order.  post: the merge
+// stream after the decisions, or null to find it again.  resampled: the
+// merged particle's components are in its slot already.
 template <class Alloc>
 __device__ inline void perset_merge(BoxDesc *B, const Arrays &A, const PW &W, int box, int64_t k,
-                                    uint32_t t, int64_t p1, int64_t p2, uint64_t seed,
+                                    int64_t q, uint32_t t, int64_t p1, int64_t p2, uint64_t seed,
                                     uint32_t step, int type, int want_terms, int rid, Alloc &al,
-                                    int o_known = -1, const Stream *post = nullptr) {
+                                    int o_group, const Stream *post, bool resampled,
+                                    const MergeParents &P) {
   int c1, c2, b1, b2;
-  decode_pair(k % W.P_stride, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
-  const uint32_t j = t - W.pair_exc[k];
+  decode_pair(q, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
   al.count(0, 1, 0);
   const int nb = B->n_bin, nc = B->w.n_class;
   const int cc = A.cc[table_index(A, box, nb, nc, b1, b2, c1, c2)];
-  const int key1 = W.key[p1], key2 = W.key[p2];
-  const int64_t id1 = A.id[p1], id2 = A.id[p2];
-  int o, new_group;
+  const int o = o_group & 0xFFFF;
+  int new_group = o_group >> 16;
   Stream s;
-  const bool resample = (A.ncomp[p1] + A.ncomp[p2] > MAX_COMP);
-  if (o_known >= 0 && (!resample || post)) {
-    // the merge decisions are known; a resampling continues the stream
-    // where they left it
-    o = o_known & 0xFFFF;
-    new_group = o_known >> 16;
-    if (post) s = *post;
-  } else {
-    s.open(seed, box, step, pair_site(nb, nc, b1, b2, c1, c2), j, RNG_MERGE);
-    o = merge_decide(A, W, B, s, p1, p2, c1, c2, cc, &new_group);
+  if (post) {
+    s = *post;
+  } else if (P.n1 + P.n2 > MAX_COMP && !resampled) {
+    s.open(seed, box, step, pair_site(nb, nc, b1, b2, c1, c2), t - W.pair_exc[k], RNG_MERGE);
+    (void)merge_decide(A, W, B, s, p1, p2, c1, c2, cc, &new_group);
   }
   int64_t info_other = 0;
   int64_t slot = -1;
   if (o & O_NEW) {
-    const int64_t nid = (o & O_ID1) ? id1 : (o & O_ID2) ? id2 : al.new_id();
+    const int64_t nid = (o & O_ID1) ? P.id1 : (o & O_ID2) ? P.id2 : al.new_id();
     info_other = nid;
     if (o & O_SLOT1) slot = p1;
     else if (o & O_SLOT2) slot = p2;
@@ -2294,32 +2442,78 @@ __device__ inline void perset_merge(BoxDesc *B, const Arrays &A, const PW &W, in
     }
     const bool appended = !(o & (O_SLOT1 | O_SLOT2));
     const int err = direct_merge(A, W, B, box, t, p1, p2, slot, appended, nid, new_group, cc, type,
-                                 want_terms, &s);
+                                 want_terms, &s, P, resampled);
     if (err) atomicExch(&B->error, err);
   }
   if (o & O_RM1) {
-    W.dead_t[p1] = t;
-    W.dead_r[p1] = rid;
-    al.live_add(key1, -1);
+    W.slot[p1].dead_t = t;
+    W.slot[p1].dead_r = rid;
+    al.live_add(P.v1.key, -1);
     if (!(o & O_SLOT1)) {
-      slot_leave(W, p1, t);
+      slot_leave(W, p1, t, P.v1);
       st_set(W, p1, ST_HOLE);
       W.holes[al.hole_index()] = ((uint64_t)box << 32) | (uint64_t)(p1 - B->off);
     }
   }
   if (o & O_RM2) {
-    W.dead_t[p2] = t;
-    W.dead_r[p2] = rid;
-    al.live_add(key2, -1);
+    W.slot[p2].dead_t = t;
+    W.slot[p2].dead_r = rid;
+    al.live_add(P.v2.key, -1);
     if (!(o & O_SLOT2)) {
-      slot_leave(W, p2, t);
+      slot_leave(W, p2, t, P.v2);
       st_set(W, p2, ST_HOLE);
       W.holes[al.hole_index()] = ((uint64_t)box << 32) | (uint64_t)(p2 - B->off);
     }
   }
   if (slot >= 0) al.live_add(W.key[slot], 1);
-  if (o & O_INFO1) put_info(A, B, al, id1, 2, info_other);
-  if (o & O_INFO2) put_info(A, B, al, id2, 2, info_other);
+  if (o & O_INFO1) put_info(A, B, al, P.id1, 2, info_other);
+  if (o & O_INFO2) put_info(A, B, al, P.id2, 2, info_other);
+}
+
+// The resamplings among a wavefront's winning per-set merges, done together
+// while they are few: each takes the wavefront about 2 us, where all of them
+// side by side, a lane each, take 13.  win: this lane merges p1 and p2 with
+// decisions o into an existing slot or the append_rank-th new one; ms: its
+// merge stream after the decisions.  Returns whether this lane's components
+// are done.  Every lane of the wavefront takes part.
+constexpr int RESAMPLE_MOST = 6;
+__device__ inline bool wave_resamplings(const Arrays &A, const BoxDesc *B, bool win, int o,
+                                        int64_t p1, int64_t p2, int64_t append_rank,
+                                        const Stream &ms) {
+  bool mine = false;
+  int64_t dst = 0;
+  int n1 = 0, n2 = 0, np1 = 0, np2 = 0;
+  if (win && (o & O_NEW)) {
+    n1 = A.ncomp[p1];
+    n2 = A.ncomp[p2];
+    np1 = A.nprim[p1];
+    np2 = A.nprim[p2];
+    mine = n1 + n2 > MAX_COMP && np1 >= n1 && np2 >= n2;
+    if (mine) {
+      if (o & O_SLOT1) dst = p1;
+      else if (o & O_SLOT2) dst = p2;
+      else if (B->n_part + append_rank < B->cap) dst = B->off + B->n_part + append_rank;
+      else mine = false;  // the merge fails
+    }
+  }
+  uint64_t todo = __ballot(mine);
+  if (__popcll(todo) > RESAMPLE_MOST) return false;
+  while (todo) {
+    const int src = __ffsll((long long)todo) - 1;
+    todo &= todo - 1;
+    Stream s;
+    s.k0 = __shfl(ms.k0, src);
+    s.k1 = __shfl(ms.k1, src);
+    s.c0 = __shfl(ms.c0, src);
+    s.c1 = __shfl(ms.c1, src);
+    s.c2 = __shfl(ms.c2, src);
+    s.c3 = __shfl(ms.c3, src);
+    const int i0 = 2 * (int)__shfl(ms.block, src) - __shfl(ms.have, src);
+    wave_resample(A, s, i0, __shfl((long long)p1, src), __shfl((long long)p2, src),
+                  __shfl((long long)dst, src), __shfl(n1, src), __shfl(n2, src),
+                  __shfl(np1, src), __shfl(np2, src));
+  }
+  return mine;
 }
 
 // a winning target event (coag_target_with_source and
@@ -2357,8 +2551,8 @@ __device__ __noinline__ void acc_apply(BoxDesc *B, const Arrays &A, const PW &W,
         owner = copy_id(-1 - q);
         return;
       }
-      W.dead_t[q] = t;
-      W.dead_r[q] = rid;
+      W.slot[q].dead_t = t;
+      W.slot[q].dead_r = rid;
       al.live_add(W.key[q], -1);
       slot_leave(W, q, t);
       st_set(W, q, ST_HOLE);
@@ -2375,8 +2569,8 @@ __device__ __noinline__ void acc_apply(BoxDesc *B, const Arrays &A, const PW &W,
   if (!(flags & RF_MERGED)) return;
   Rec np;
   pool_load(W, ns, r, klass, target_id, np);
-  W.dead_t[p] = t;
-  W.dead_r[p] = rid;
+  W.slot[p].dead_t = t;
+  W.slot[p].dead_r = rid;
   al.live_add(W.key[p], -1);
   write_new_particle(A, W, B, box, t, t, p, false, np, nb, type, want_terms);
   if (flags & RF_DIED) {
@@ -2427,8 +2621,9 @@ __device__ inline void apply_event(BoxDesc *boxes, const Arrays &A, const PW &W,
                 W.r_nchain[W.ev_rec[e]] > CHAIN_WAVE_MIN);
     } else {
       const int64_t k = test_pair(W, (int64_t)n_box * W.P_stride, t);
-      perset_merge(B, A, W, box, k, t, W.ev_p1[e], W.ev_p2[e], seed, step, type, want_terms, rid,
-                   al, W.ev_out[e] & ~O_WIN);
+      perset_merge(B, A, W, box, k, k - (int64_t)box * W.P_stride, t, W.ev_p1[e], W.ev_p2[e], seed,
+                   step, type, want_terms, rid, al, W.ev_out[e] & ~O_WIN, nullptr, false,
+                   load_parents(A, W, W.ev_p1[e], W.ev_p2[e]));
     }
     cs = al.n_samp;
     cc = al.n_coag;
@@ -2495,8 +2690,8 @@ __device__ inline void apply_chain(BoxDesc *boxes, const Arrays &A, const PW &W,
     const int64_t own = mk ? id_first + (int64_t)(-1 - qm - 1) * B->id_stride : owner;
     if (here && q >= 0) {
       const int ord = done + __popcll(rems & below);
-      W.dead_t[q] = t;
-      W.dead_r[q] = rid;
+      W.slot[q].dead_t = t;
+      W.slot[q].dead_r = rid;
       atomicAdd(&live[W.key[q]], -1);
       slot_leave(W, q, t);
       st_set(W, q, ST_HOLE);
@@ -2552,17 +2747,17 @@ __global__ void k_par_box_totals(BoxDesc *boxes, PW W, int n_box) {
 }
 
 __device__ inline void release_event(const PW &W, int e) {
-  W.claim[W.ev_p1[e]] = UNCLAIMED;
-  W.claim_wr[W.ev_p1[e]] = UNCLAIMED;
+  W.slot[W.ev_p1[e]].claim = UNCLAIMED;
+  W.slot[W.ev_p1[e]].claim_wr = UNCLAIMED;
   const int r = W.ev_rec[e];
   if (r >= 0) {
     rm_walk(W, r, [&](int q) {
-      W.claim[q] = UNCLAIMED;
-      W.claim_wr[q] = UNCLAIMED;
+      W.slot[q].claim = UNCLAIMED;
+      W.slot[q].claim_wr = UNCLAIMED;
     });
   } else {
-    W.claim[W.ev_p2[e]] = UNCLAIMED;
-    W.claim_wr[W.ev_p2[e]] = UNCLAIMED;
+    W.slot[W.ev_p2[e]].claim = UNCLAIMED;
+    W.slot[W.ev_p2[e]].claim_wr = UNCLAIMED;
   }
 }
 
@@ -2578,7 +2773,10 @@ __global__ void k_par_release(PW W) {
 // seen the particles as that winner left them.  A particle changed in an
 // earlier round was drawn in its changed state.
 __device__ inline bool consumed_before(const PW &W, int p, uint32_t t, int rid) {
-  return p >= 0 && st_get(W, p) != ST_LIVE && W.dead_t[p] < t && W.dead_r[p] == rid;
+  if (p < 0) return false;
+  const uint32_t st = W.slot[p].st, dead_t = W.slot[p].dead_t;
+  const int dead_r = W.slot[p].dead_r;
+  return (int)(st >> 2) == W.epoch && (st & 3) != ST_LIVE && dead_t < t && dead_r == rid;
 }
 
 // A test on an empty arrival entry of list L (bin bL) of a pair that
@@ -2593,9 +2791,10 @@ __device__ inline void pending_test(BoxDesc *boxes, const PW &W, int n_box, int 
   uint32_t t = W.tid[i];
   const int64_t NP = (int64_t)n_box * W.P_stride;
   const int64_t k = test_pair(W, NP, t);
-  const int box = (int)(k / W.P_stride);
+  int64_t q;
+  const int box = pair_box(W, k, &q);
   int c1, c2, b1, b2;
-  decode_pair(k % W.P_stride, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
+  decode_pair(q, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
   const int kind = W.pair_acc[k];
   // the lowest bin this event's results can land in
   const int b_lo = kind ? (kind == 1 ? b1 : b2) : max(b1, b2);
@@ -2727,14 +2926,14 @@ constexpr int TF_EFFECT = 1, TF_ACC = 2, TF_RUN = 4, TF_WARN = 8, TF_ATHIN = 16,
 // claims inside one kernel are read and released with device-scope atomics,
 // so they need no cache maintenance between the phases of a round
 __device__ inline uint32_t claim_load(const PW &W, int p) {
-  return __hip_atomic_load(&W.claim[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __hip_atomic_load(&W.slot[p].claim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ inline uint32_t claim_wr_load(const PW &W, int p) {
-  return __hip_atomic_load(&W.claim_wr[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __hip_atomic_load(&W.slot[p].claim_wr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ inline void claim_release(const PW &W, int p) {
-  __hip_atomic_store(&W.claim[p], UNCLAIMED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(&W.claim_wr[p], UNCLAIMED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(&W.slot[p].claim, UNCLAIMED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(&W.slot[p].claim_wr, UNCLAIMED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 
@@ -2846,7 +3045,7 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
         p2 = -1;
       } else {
         TestOut o;
-        perset_test(B, A, W, box, k, t, type, seed, step, precision, band, 0, o, &s_w);
+        perset_test(B, A, W, box, k, k - pb, t, type, seed, step, precision, band, 0, o, &s_w);
         p1 = o.p1;
         p2 = o.p2;
         W.thin[t - batch_t0] = o.thin ? 1 : 0;
@@ -2860,10 +3059,10 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
     // the merge decisions of an accepted per-set test, from the particles as
     // they are now: they say which parents it changes
     int o_win = -1;
-    Stream ms;  // a per-set test's merge stream, after its decisions
+    Stream ms{};  // a per-set test's merge stream, after its decisions
     if (effect && !is_acc) {
       int c1, c2, b1, b2;
-      decode_pair(k % W.P_stride, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
+      decode_pair(k - pb, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
       const int nb = B->n_bin, nc = B->w.n_class;
       const int cc = A.cc[table_index(A, box, nb, nc, b1, b2, c1, c2)];
       ms.open(seed, box, step, pair_site(nb, nc, b1, b2, c1, c2), t - W.pair_exc[k], RNG_MERGE);
@@ -2877,11 +3076,15 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
         rm_walk(W, rec, [&](int q) { claim_write(W, q, t); });
       } else {
         if (o_win & O_RM1) claim_write(W, p1, t);
-        else atomicMin(&W.claim[p1], t);
+        else atomicMin(&W.slot[p1].claim, t);
         if (o_win & O_RM2) claim_write(W, p2, t);
-        else atomicMin(&W.claim[p2], t);
+        else atomicMin(&W.slot[p2].claim, t);
       }
     }
+    // what a merge reads of its parents travels while the claims settle: no
+    // winner of the round changes a particle that another one reads
+    MergeParents par{};
+    if (effect && !is_acc) par = load_parents(A, W, p1, p2);
     __syncthreads();
     // 3. resolve, and what each winner creates
     bool win = false;
@@ -2929,6 +3132,8 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
     }
     __syncthreads();
     // 4. apply the winners at their ranks
+    const bool resampled =
+        wave_resamplings(A, B, win && !is_acc, o_win, p1, p2, r_app, ms);
     if (win) {
       TailAlloc al;
       al.B = B;
@@ -2940,8 +3145,8 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
       al.s_live = s_live;
       al.n_samp = al.n_coag = al.n_warn = 0;
       if (is_acc) acc_apply(B, A, W, box, t, rec, p1, type, want_terms, rid, al);
-      else perset_merge(B, A, W, box, k, t, p1, p2, seed, step, type, want_terms, rid, al, o_win,
-                        &ms);
+      else perset_merge(B, A, W, box, k, k - pb, t, p1, p2, seed, step, type, want_terms, rid, al,
+                        o_win, &ms, resampled, par);
       c_samp += al.n_samp;
       c_coag += al.n_coag;
       c_warn += al.n_warn;
@@ -3103,6 +3308,14 @@ __global__ void k_fill_u32(uint32_t *p, int64_t n, uint32_t v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
+__global__ void k_init_slots(SlotRec *p, int64_t n) {
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = SlotRec{UNCLAIMED, UNCLAIMED, 0u, 0, 0, 0u, 0, ST_LIVE};
+}
+__global__ void k_clear_status(SlotRec *p, int64_t n) {
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i].st = ST_LIVE;
+}
 __global__ void k_fill_u8(uint8_t *p, int64_t n, uint8_t v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -3166,7 +3379,7 @@ __global__ void k_compact_move(BoxDesc *boxes, Arrays A, PW W, int n_holes) {
   copy_particle(A, pf, pt);
   W.key[pt] = W.key[pf];
   W.terms[pt] = W.terms[pf];
-  W.status[pt] = W.status[pf];
+  W.slot[pt].st = W.slot[pf].st;
 }
 
 __global__ void k_compact_finish(BoxDesc *boxes, PW W, int n_box) {
@@ -3198,7 +3411,8 @@ __global__ void __launch_bounds__(256) k_thin_counts(BoxDesc *boxes, PW W, int64
                                                      int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   int box = -1;
-  if (i < n && W.thin[i]) box = (int)(test_pair(W, NP, t0 + (uint32_t)i) / W.P_stride);
+  int64_t q;
+  if (i < n && W.thin[i]) box = pair_box(W, test_pair(W, NP, t0 + (uint32_t)i), &q);
   wave_flush_counts(boxes, box, -1, 0, 0);
 }
 
@@ -3258,18 +3472,18 @@ inline int parallel_alloc_records(ParallelWork &W, int n_spec) {
 
 inline void parallel_free_arrays(ParallelWork &W) {
   PW &d = W.d;
-  void *ptrs[] = {d.key,  d.status, d.claim, d.claim_wr, d.terms, d.perm, d.tile_box, d.tile_start,
+  void *ptrs[] = {d.key,  d.slot, d.terms, d.perm, d.tile_box, d.tile_start,
                   d.tiles_in_box, d.tile_first, d.hist, d.hist_scan, d.lstart, d.lcnt, d.live,
                   d.pair_n, d.pair_exc, d.acc, d.acc_scan, d.tp1, d.tp2, d.tid, d.pend, d.ev_t,
                   d.ev_p1, d.ev_p2, d.ev_box, d.ev_out, d.f_app, d.f_id, d.f_info, d.f_hole,
-                  d.f_lose, d.f_pend, d.s_pend, d.dead_t, d.dead_r, d.s_app, d.s_id, d.s_info, d.s_hole,
+                  d.f_lose, d.f_pend, d.s_pend, d.s_app, d.s_id, d.s_info, d.s_hole,
                   d.s_lose, d.box_first,
                   d.holes, d.holes_sorted, d.cmp_lo, d.cmp_hi, d.cmp_head, d.acc_samp,
                   d.scan_part, W.sort_tmp, d.rc,
                   d.pair_acc, d.pair_accn, d.acc_exc, d.trec, d.tns, d.ev_rec, d.misc,
                   d.hole_top, d.pend_k, d.tp_in, d.tpair,
                   d.acap, d.arr_n, d.arr_head, d.ap_p, d.ap_t, d.ap_dep, d.ap_next, d.ap_top,
-                  d.arr_of, d.key0, d.depart_t, d.thin, d.minpend, d.minpend_next};
+                  d.thin, d.minpend, d.minpend_next};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   parallel_free_records(W);
@@ -3331,16 +3545,9 @@ inline int parallel_layout(ParallelWork &W, const Arrays &A, int n_box,
   }
   const int64_t tc = A.total_cap;
   PCHECK(pmalloc(&d.key, tc));
-  PCHECK(pmalloc(&d.status, tc));
-  PCHECK(pmalloc(&d.claim, tc));
-  PCHECK(pmalloc(&d.claim_wr, tc));
-  PCHECK(pmalloc(&d.dead_t, tc));
-  PCHECK(pmalloc(&d.dead_r, tc));
+  PCHECK(pmalloc(&d.slot, tc));
   PCHECK(pmalloc(&d.terms, tc));
   PCHECK(pmalloc(&d.perm, tc));
-  PCHECK(pmalloc(&d.key0, tc));
-  PCHECK(pmalloc(&d.depart_t, tc));
-  PCHECK(pmalloc(&d.arr_of, tc));
   // tiles over each box's capacity
   std::vector<int> tb, ts;
   std::vector<int64_t> hoff(n_box);
@@ -3445,9 +3652,7 @@ inline int parallel_layout(ParallelWork &W, const Arrays &A, int n_box,
   PCHECK(rocprim::radix_sort_keys(nullptr, W.sort_tmp_bytes, d.holes, d.holes_sorted,
                                   (unsigned)W.hole_cap, 0u, 64u, (hipStream_t)0));
   PCHECK(hipMalloc(&W.sort_tmp, W.sort_tmp_bytes));
-  hipLaunchKernelGGL(k_fill_u32, dim3((tc + 255) / 256), dim3(256), 0, 0, d.claim, tc, UNCLAIMED);
-  hipLaunchKernelGGL(k_fill_u32, dim3((tc + 255) / 256), dim3(256), 0, 0, d.claim_wr, tc, UNCLAIMED);
-  hipLaunchKernelGGL(k_fill_u8, dim3((tc + 255) / 256), dim3(256), 0, 0, d.status, tc, ST_LIVE);
+  hipLaunchKernelGGL(k_init_slots, dim3((tc + 255) / 256), dim3(256), 0, 0, d.slot, tc);
   W.epoch = 0;
   PCHECK(hipGetLastError());
   PCHECK(hipDeviceSynchronize());
@@ -3564,8 +3769,8 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
   // array when the 6-bit epoch wraps
   if (++W.epoch > 63) {
     W.epoch = 1;
-    hipLaunchKernelGGL(k_fill_u8, dim3((unsigned)((A.total_cap + 255) / 256)), dim3(256), 0, st,
-                       d.status, A.total_cap, ST_LIVE);
+    hipLaunchKernelGGL(k_clear_status, dim3((unsigned)((A.total_cap + 255) / 256)), dim3(256), 0,
+                       st, d.slot, A.total_cap);
   }
   d.epoch = W.epoch;
   // 5. tests, claims and merges, in batches of T_cap tests.  The rounds of
