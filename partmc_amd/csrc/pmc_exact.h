@@ -260,14 +260,19 @@ __device__ inline int64_t table_index(const Arrays &A, int box, int nb, int nc,
 
 // --------------------------------------------------------- exact sweep
 // A detached particle record, as aero_particle_t on the path.
-struct Rec {
-  double vol[MAX_SPEC];
+// NS bounds the species it holds: the records of up to FEW_SPEC species keep
+// their volumes in registers.
+constexpr int FEW_SPEC = 4;
+template <int NS>
+struct RecN {
+  double vol[NS];
   int64_t id;
   int group, klass, nprim, ncomp;
   int csrc[MAX_COMP];
   double ctime[MAX_COMP];
   double least, greatest;
 };
+using Rec = RecN<MAX_SPEC>;
 
 struct ExactBox {
   const Arrays *A;

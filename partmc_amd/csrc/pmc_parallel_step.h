@@ -64,6 +64,22 @@ struct alignas(32) SlotRec {
   uint32_t st;        // (epoch << 2) | state; another step's epoch reads as live
 };
 
+// A target event's outcome, in one line.
+struct alignas(64) EventRec {
+  int nsamp, ncoag;    // samples and coagulations
+  int nrm;             // removed sources
+  int nchain, head;    // their chain: entries (with copy markers), first chunk
+  int ndup, dhead;     // copies of the target, the first one's pool entry
+  int flags, err;
+  int nrd, rdhead;     // distinct sources read from small source lists
+};
+// A pool entry's fields beside its volumes and components.
+struct alignas(32) PoolRec {
+  int group, nprim, ncomp;
+  int next;            // the next copy's entry, -1 after the last
+  double least, greatest;
+};
+
 struct PW {  // device view of the parallel work arrays
   int K_stride;     // keys per box of the list tables (the allocation's grid)
   int K_hist;       // keys per box of this step's histogram (the step's grid)
@@ -98,17 +114,13 @@ struct PW {  // device view of the parallel work arrays
   int *tns;                    // [T_cap] n_samp (+ ACC_WARN) of a target without effect
   int *ev_rec;                 // [T_cap] record of an event, -1 for per-set events
   int acc_cap, pool_cap;
-  // event records [acc_cap]
-  int *r_nsamp, *r_ncoag, *r_nrm, *r_nchain, *r_head, *r_ndup, *r_dhead, *r_flags,
-      *r_err;
-  int *r_rdhead, *r_nrd;       // distinct sources read from small source lists
+  EventRec *ev;                // [acc_cap] event records
   // particle pool [pool_cap]: entry r < acc_cap is the final target of
   // record r; entries from acc_cap on are the copies (aero_state_dup_particle)
-  double *q_vol;               // [n_spec][pool_cap]
-  int *q_group, *q_nprim, *q_ncomp, *q_next;
-  int *q_csrc;                 // [MAX_COMP][pool_cap]
-  double *q_ctime;             // [MAX_COMP][pool_cap]
-  double *q_least, *q_greatest;
+  double *q_vol;               // [pool_cap][n_spec]
+  PoolRec *q;                  // [pool_cap]
+  int *q_csrc;                 // [pool_cap][MAX_COMP]
+  double *q_ctime;             // [pool_cap][MAX_COMP]
   int *dup_top;                // [1] copy allocator of the round
   int *rm_buf;                 // chunks: [0] next chunk or -1, [1..RM_CHUNK) removed slots
   int *rm_top;                 // [1] chunk allocator of the round
@@ -549,10 +561,43 @@ __device__ inline int pair_box(const PW &W, int64_t k, int64_t *q) {
   return box;
 }
 
+// loops over a record's species: unrolled over NS where that is few, so
+// that the record stays in registers
+// The step's arguments for the functions called out of line (target visits
+// and their merges), in LDS: passed by reference they would live in each
+// lane's private memory, and every pointer read from there waits for all
+// loads in flight.  A kernel that calls them fills it first.  With this, the
+// volumes in registers (RecN) and the records in one line each, a tail round
+// of 1e5 Brownian particles spends 23 us on visits and tests (28 before).
+struct StepCtx {
+  Arrays A;
+  PW W;
+};
+static __shared__ StepCtx s_ctx;
+__device__ inline void step_ctx_fill(const Arrays &A, const PW &W) {
+  for (int q = threadIdx.x; q < (int)(sizeof(Arrays) / sizeof(int)); q += blockDim.x)
+    ((int *)&s_ctx.A)[q] = ((const int *)&A)[q];
+  for (int q = threadIdx.x; q < (int)(sizeof(PW) / sizeof(int)); q += blockDim.x)
+    ((int *)&s_ctx.W)[q] = ((const int *)&W)[q];
+  __syncthreads();
+}
+
+#define REC_FOR(s, ns) for (int s = 0; s < (NS <= FEW_SPEC ? NS : (ns)); ++s) if (NS > FEW_SPEC || s < (ns))
+
 // the record without its components (they are read in a second pass
 // that depends on ncomp, so a reader that may not need them defers it)
-__device__ inline void load_rec_head(const Arrays &A, int64_t p, Rec &r) {
-  for (int s = 0; s < A.n_spec; ++s) r.vol[s] = A.vol[(int64_t)s * A.total_cap + p];
+template <int NS>
+__device__ inline void load_rec_head(const Arrays &A, int64_t p, RecN<NS> &r) {
+  const int ns = A.n_spec;
+  if (NS <= FEW_SPEC) {
+    double x[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) x[s] = A.vol[(int64_t)(s < ns ? s : ns - 1) * A.total_cap + p];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) r.vol[s] = x[s];
+  } else {
+    for (int s = 0; s < ns; ++s) r.vol[s] = A.vol[(int64_t)s * A.total_cap + p];
+  }
   r.id = A.id[p];
   r.group = A.group[p];
   r.klass = A.klass[p];
@@ -562,22 +607,25 @@ __device__ inline void load_rec_head(const Arrays &A, int64_t p, Rec &r) {
   r.greatest = A.greatest[p];
 }
 
-__device__ inline void load_rec_comps(const Arrays &A, int64_t p, Rec &r) {
+template <int NS>
+__device__ inline void load_rec_comps(const Arrays &A, int64_t p, RecN<NS> &r) {
   for (int c = 0; c < r.ncomp; ++c) {
     r.csrc[c] = A.csrc[comp_at(p, c)];
     r.ctime[c] = A.ctime[comp_at(p, c)];
   }
 }
 
-__device__ inline void load_rec(const Arrays &A, int64_t p, Rec &r) {
+template <int NS>
+__device__ inline void load_rec(const Arrays &A, int64_t p, RecN<NS> &r) {
   load_rec_head(A, p, r);
   load_rec_comps(A, p, r);
 }
 
 // aero_particle_coagulate for the parallel path (same rules as rec_coagulate)
-__device__ inline int par_rec_coagulate(int n_spec, Stream &s, const Rec &p1, const Rec &p2,
-                                        Rec &o) {
-  for (int k = 0; k < n_spec; ++k) o.vol[k] = p1.vol[k] + p2.vol[k];
+template <int NS>
+__device__ inline int par_rec_coagulate(int n_spec, Stream &s, const RecN<NS> &p1,
+                                        const RecN<NS> &p2, RecN<NS> &o) {
+  REC_FOR(k, n_spec) o.vol[k] = p1.vol[k] + p2.vol[k];
   o.group = 0;
   o.klass = 0;
   o.id = 0;
@@ -1050,7 +1098,7 @@ __device__ __forceinline__ void perset_test(BoxDesc *B, const Arrays &A, const P
                                             int64_t k, int64_t q, uint32_t t, int type,
                                             uint64_t seed, uint32_t step, int precision,
                                             double band, int validation, TestOut &o,
-                                            const Weights *wl = nullptr) {
+                                            const Weights &w) {
   o.p1 = o.p2 = -1;
   o.accept = false;
   o.warn = false;
@@ -1059,7 +1107,6 @@ __device__ __forceinline__ void perset_test(BoxDesc *B, const Arrays &A, const P
   decode_pair(q, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
   const uint32_t tau = W.pair_exc[k];  // where the pair begins in the sequence
   const uint32_t j = t - tau;
-  const Weights &w = wl ? *wl : B->w;
   const int nb = B->n_bin, nc = w.n_class;
   const int64_t ti = table_index(A, box, nb, nc, b1, b2, c1, c2);
   const int cc = A.cc[ti];
@@ -1174,12 +1221,10 @@ __device__ inline MergeCtx merge_ctx(BoxDesc *boxes, const PW &W, int n_box, uin
 }
 
 // coagulate_weighting (src/coagulation.F90:810-922): decisions only
-// wl: the box's weights staged in LDS by the caller, or null to read them
-// from the box
+// w: the box's weights (the tail stages them in LDS)
 __device__ inline int merge_decide(const Arrays &A, const PW &W, const BoxDesc *B, Stream &s,
                                    int64_t p1, int64_t p2, int c1, int c2, int cc,
-                                   int *new_group, const Weights *wl = nullptr) {
-  const Weights &w = wl ? *wl : B->w;
+                                   int *new_group, const Weights &w) {
   // the parents' volumes and lists, read together up front
   const double v1 = A.vtot[p1], v2 = A.vtot[p2];
   const int key_p1 = W.key[p1], key_p2 = W.key[p2];
@@ -1276,7 +1321,7 @@ __device__ inline int perset_decide(BoxDesc *B, const Arrays &A, const PW &W, in
   const int cc = A.cc[table_index(A, box, nb, nc, b1, b2, c1, c2)];
   ms.open(seed, box, step, pair_site(nb, nc, b1, b2, c1, c2), t - W.pair_exc[k], RNG_MERGE);
   int g;
-  return merge_decide(A, W, B, ms, p1, p2, c1, c2, cc, &g) | (g << 16);
+  return merge_decide(A, W, B, ms, p1, p2, c1, c2, cc, &g, B->w) | (g << 16);
 }
 
 // The kernels of a claim round read their item counts from device memory
@@ -1304,7 +1349,8 @@ __device__ __forceinline__ void par_test(BoxDesc *boxes, const Arrays &A, const 
   BoxDesc *B = &boxes[box];
   if (B->error) return;
   TestOut o;
-  perset_test(B, A, W, box, k, q, t, type, seed, step, precision, band, validation, o);
+  perset_test(B, A, W, box, k, q, t, type, seed, step, precision, band, validation, o,
+              B->w);
   W.tp1[i] = o.p1;
   W.tp2[i] = o.p2;
   W.thin[t - t0] = o.thin ? 1 : 0;
@@ -1362,38 +1408,18 @@ __device__ inline int rand_group_w(Stream &s, const Weights &w, int cls, double 
   return sample_cts_pdf(s, w.n_group, pdf);
 }
 
-__device__ inline double rec_vol(int n_spec, const Rec &r) {
+template <int NS>
+__device__ inline double rec_vol(int n_spec, const RecN<NS> &r) {
   double v = 0.0;
-  for (int s = 0; s < n_spec; ++s) v += r.vol[s];
+  REC_FOR(s, n_spec) v += r.vol[s];
   return v;
 }
 
-__device__ inline double rec_density(const Arrays &A, const Rec &r) {
+template <int NS>
+__device__ inline double rec_density(const Arrays &A, const RecN<NS> &r) {
   double m = 0.0;
-  for (int s = 0; s < A.n_spec; ++s) m += r.vol[s] * A.density[s];
+  REC_FOR(s, A.n_spec) m += r.vol[s] * A.density[s];
   return m / rec_vol(A.n_spec, r);
-}
-
-// weighted kernel of two detached records (as weighted_kernel64)
-__device__ inline int weighted_kernel_rec(const Arrays &A, const Weights &w, const Env &env,
-                                          int type, const Rec &a, const Rec &b, int c1, int c2,
-                                          int cc, double *k_out) {
-  double v1 = rec_vol(A.n_spec, a), v2 = rec_vol(A.n_spec, b);
-  double k = 0.0;
-  int err = 0;
-  switch (type) {
-    case KERNEL_ADDITIVE: k = env.beta * (v1 + v2); break;
-    case KERNEL_CONSTANT: k = C_BETA_0; break;
-    case KERNEL_ZERO: k = 0.0; break;
-    case KERNEL_BROWN:
-      k = kernel_brown_helper(v1, rec_density(A, a), v2, rec_density(A, b), env.temp,
-                              env.pressure);
-      break;
-    case KERNEL_SEDI: err = kernel_sedi_helper(v1, v2, &k); break;
-    default: err = 200724934;
-  }
-  *k_out = k * coag_num_conc_factor(w, vol2rad(v1), vol2rad(v2), c1, c2, cc);
-  return err;
 }
 
 // the sources a target removes, in a chain of RM_CHUNK-int chunks
@@ -1439,8 +1465,8 @@ __device__ inline bool rm_has(const PW &W, const RmChain &c, int slot) {
 // owner markers (-1 - k: the removals that follow belong to copy k)
 template <class F>
 __device__ inline void chain_walk(const PW &W, int r, F f) {
-  int left = W.r_nchain[r];
-  for (int ch = W.r_head[r]; ch >= 0 && left > 0; ch = W.rm_buf[ch]) {
+  int left = W.ev[r].nchain;
+  for (int ch = W.ev[r].head; ch >= 0 && left > 0; ch = W.rm_buf[ch]) {
     int m = left < RM_CHUNK - 1 ? left : RM_CHUNK - 1;
     for (int q = 1; q <= m; ++q) f(W.rm_buf[ch + q]);
     left -= m;
@@ -1458,41 +1484,27 @@ __device__ inline void rm_walk(const PW &W, int r, F f) {
 // visit the sources record r read from small lists
 template <class F>
 __device__ inline void rd_walk(const PW &W, int r, F f) {
-  int left = W.r_nrd[r];
-  for (int ch = W.r_rdhead[r]; ch >= 0 && left > 0; ch = W.rm_buf[ch]) {
+  int left = W.ev[r].nrd;
+  for (int ch = W.ev[r].rdhead; ch >= 0 && left > 0; ch = W.rm_buf[ch]) {
     int m = left < RM_CHUNK - 1 ? left : RM_CHUNK - 1;
     for (int q = 1; q <= m; ++q) f(W.rm_buf[ch + q]);
     left -= m;
   }
 }
 
-__device__ inline void pool_store(const PW &W, int n_spec, int i, const Rec &s) {
-  for (int k = 0; k < n_spec; ++k) W.q_vol[(int64_t)k * W.pool_cap + i] = s.vol[k];
-  W.q_group[i] = s.group;
-  W.q_nprim[i] = s.nprim;
-  W.q_ncomp[i] = s.ncomp;
+template <int NS>
+__device__ inline void pool_store(const PW &W, int n_spec, int i, const RecN<NS> &s) {
+  REC_FOR(k, n_spec) W.q_vol[(int64_t)i * n_spec + k] = s.vol[k];
+  PoolRec &q = W.q[i];
+  q.group = s.group;
+  q.nprim = s.nprim;
+  q.ncomp = s.ncomp;
   for (int c = 0; c < s.ncomp; ++c) {
-    W.q_csrc[(int64_t)c * W.pool_cap + i] = s.csrc[c];
-    W.q_ctime[(int64_t)c * W.pool_cap + i] = s.ctime[c];
+    W.q_csrc[comp_at(i, c)] = s.csrc[c];
+    W.q_ctime[comp_at(i, c)] = s.ctime[c];
   }
-  W.q_least[i] = s.least;
-  W.q_greatest[i] = s.greatest;
-}
-
-// a pool entry as a particle of class `klass` with identifier `id`
-__device__ inline void pool_load(const PW &W, int n_spec, int i, int klass, int64_t id, Rec &s) {
-  for (int k = 0; k < n_spec; ++k) s.vol[k] = W.q_vol[(int64_t)k * W.pool_cap + i];
-  s.id = id;
-  s.group = W.q_group[i];
-  s.klass = klass;
-  s.nprim = W.q_nprim[i];
-  s.ncomp = W.q_ncomp[i];
-  for (int c = 0; c < s.ncomp; ++c) {
-    s.csrc[c] = W.q_csrc[(int64_t)c * W.pool_cap + i];
-    s.ctime[c] = W.q_ctime[(int64_t)c * W.pool_cap + i];
-  }
-  s.least = W.q_least[i];
-  s.greatest = W.q_greatest[i];
+  q.least = s.least;
+  q.greatest = s.greatest;
 }
 
 // sample_source_particle (src/coagulation.F90:333-517) against the running
@@ -1500,16 +1512,17 @@ __device__ inline void pool_load(const PW &W, int n_spec, int i, int klass, int6
 // the particles still present that this target has not removed; returns
 // an error code, 0 on success.  Sources it removes are pushed to `chain`
 // and claimed with index t.
-// The target's side of weighted_kernel_rec, the same for every source drawn
-// for one pair: its Brownian terms, volume, radius and weight.
+// The target's side of the weighted kernel (as weighted_kernel64), the same
+// for every source drawn for one pair: its Brownian terms, volume, radius and weight.
 struct TargetSide {
   BrownAir air;
   BrownTerms terms;
   double vol, rad, nc;
 };
 
+template <int NS>
 __device__ inline TargetSide target_side(const Arrays &A, const Weights &w, const Env &env,
-                                         int type, const Rec &b, int c2) {
+                                         int type, const RecN<NS> &b, int c2) {
   TargetSide ts;
   ts.vol = rec_vol(A.n_spec, b);
   if (type == KERNEL_BROWN) {
@@ -1521,9 +1534,10 @@ __device__ inline TargetSide target_side(const Arrays &A, const Weights &w, cons
   return ts;
 }
 
-// weighted_kernel_rec(a, b, c1, c2, cc) with b's side from target_side(b, c2)
+// the weighted kernel of a record a of class c1 and the target
+template <int NS>
 __device__ inline int weighted_kernel_tgt(const Arrays &A, const Weights &w, const Env &env,
-                                          int type, const Rec &a, const TargetSide &ts,
+                                          int type, const RecN<NS> &a, const TargetSide &ts,
                                           int c1, int cc, double *k_out) {
   double v1 = rec_vol(A.n_spec, a), v2 = ts.vol;
   double k = 0.0;
@@ -1542,14 +1556,15 @@ __device__ inline int weighted_kernel_tgt(const Arrays &A, const Weights &w, con
   return err;
 }
 
+template <int NS>
 __device__ inline int acc_sample_source(const Arrays &A, const PW &W, BoxDesc *B, int type,
-                                        const Rec &target, int ct, int cs, double nc_src_min,
+                                        const RecN<NS> &target, int ct, int cs, double nc_src_min,
                                         int64_t sbase, int skey, int n_s, double n_spt,
                                         double accept_factor, Stream &aps, Stream &smp,
                                         Stream &fin, uint32_t tau, uint32_t t, bool claim,
                                         RmChain &chain,
                                         RmChain &reads, int *n_samp_out,
-                                        int *n_coag_out, int *warn, Rec &source) {
+                                        int *n_coag_out, int *warn, RecN<NS> &source) {
   const int ns = A.n_spec;
   const Weights &w = B->w;
   const Env env = B->env;
@@ -1563,8 +1578,8 @@ __device__ inline int acc_sample_source(const Arrays &A, const PW &W, BoxDesc *B
   const int n_total = n_remove + n_extra;
   int n_avg = 0, n_samp = 0, n_rm_here = 0, n_thin = 0, n_samp_rm = 0;
   double prob_coag_tot = 0.0;
-  double vol_sq[MAX_SPEC], vol_cv[MAX_SPEC];
-  for (int q = 0; q < ns; ++q) {
+  double vol_sq[NS], vol_cv[NS];
+  REC_FOR(q, ns) {
     vol_sq[q] = 0.0;
     vol_cv[q] = 0.0;
     source.vol[q] = 0.0;
@@ -1576,7 +1591,7 @@ __device__ inline int acc_sample_source(const Arrays &A, const PW &W, BoxDesc *B
     source.ctime[c] = 0.0;
   }
   source.least = source.greatest = 0.0;
-  Rec pi;
+  RecN<NS> pi;
   TargetSide ts;  // formed at the first sample: many pairs draw none
   bool have_ts = false;
   int i_samp = 1;
@@ -1585,7 +1600,7 @@ __device__ inline int acc_sample_source(const Arrays &A, const PW &W, BoxDesc *B
     // the reference's n_samp > n_samp_remove (:413) over the samples kept
     if (i_samp > n_remove && n_samp > n_samp_rm && n_avg >= 2) {
       double cvmax = 0.0;
-      for (int q = 0; q < ns; ++q) {
+      REC_FOR(q, ns) {
         double vm = source.vol[q] / (double)n_avg;
         if (vm > 0.0) vol_cv[q] = sqrt(vol_sq[q] / (double)n_avg - vm * vm) / vm;
         if (q == 0 || vol_cv[q] > cvmax) cvmax = vol_cv[q];
@@ -1642,7 +1657,7 @@ __device__ inline int acc_sample_source(const Arrays &A, const PW &W, BoxDesc *B
       load_rec_comps(A, ps, pi);
       err = par_rec_coagulate(ns, smp, source, pi, source);
       if (err) return err;
-      for (int q = 0; q < ns; ++q) vol_sq[q] += pi.vol[q] * pi.vol[q];
+      REC_FOR(q, ns) vol_sq[q] += pi.vol[q] * pi.vol[q];
       if (i_samp <= n_remove) {
         double nc_i = nc_at_radius(w, pi.klass, vol2rad(rec_vol(ns, pi)));
         double prob_remove_i = nc_target / nc_i;
@@ -1664,7 +1679,7 @@ __device__ inline int acc_sample_source(const Arrays &A, const PW &W, BoxDesc *B
   double prob_coag_mean = prob_coag_tot / (double)n_samp;
   if (!(prob_coag_mean <= 1.0)) *warn = 1;
   int n_coag = rand_binomial(fin, n_total - n_thin, prob_coag_mean);
-  for (int q = 0; q < ns; ++q) source.vol[q] = source.vol[q] * ((double)n_coag / (double)n_avg);
+  REC_FOR(q, ns) source.vol[q] = source.vol[q] * ((double)n_coag / (double)n_avg);
   source.nprim = prob_round(fin, (double)source.nprim * ((double)n_coag / (double)n_avg));
   const int n_comp = source.ncomp;
   const int n_comp_new = source.nprim < MAX_COMP ? source.nprim : MAX_COMP;
@@ -1721,9 +1736,12 @@ __device__ inline int acc_sample_source(const Arrays &A, const PW &W, BoxDesc *B
 // with index t when `claim`), 0 when it has none (*tns = its samples +
 // ACC_WARN, or TNS_ATHIN for an arrival entry with no arrival yet), -1 on
 // a box error.  *p_out is the target's slot, or -1 when there is none.
-__device__ __noinline__ int acc_visit(BoxDesc *boxes, const Arrays &A, const PW &W, int64_t k,
-                                      uint32_t t, int rec, int type, uint64_t seed, uint32_t step,
-                                      double del_t, bool claim, int *p_out, int *tns) {
+template <int NS>
+__device__ __noinline__ int acc_visit(BoxDesc *boxes, int64_t k, uint32_t t, int rec, int type,
+                                      uint64_t seed, uint32_t step, double del_t, bool claim,
+                                      int *p_out, int *tns) {
+  const Arrays &A = s_ctx.A;
+  const PW &W = s_ctx.W;
   *p_out = -1;
   *tns = 0;
   int64_t q;
@@ -1758,11 +1776,12 @@ __device__ __noinline__ int acc_visit(BoxDesc *boxes, const Arrays &A, const PW 
   *p_out = p;
   // the record's chains start empty, so an attempt cut short by an error
   // leaves nothing to walk
-  W.r_nrd[rec] = 0;
-  W.r_rdhead[rec] = -1;
-  W.r_nchain[rec] = 0;
-  W.r_nrm[rec] = 0;
-  W.r_head[rec] = -1;
+  EventRec &ev = W.ev[rec];
+  ev.nrd = 0;
+  ev.rdhead = -1;
+  ev.nchain = 0;
+  ev.nrm = 0;
+  ev.head = -1;
   const int ns = A.n_spec;
   const Weights &w = B->w;
   const uint32_t ordinal = (uint32_t)j + 1;
@@ -1775,7 +1794,7 @@ __device__ __noinline__ int acc_visit(BoxDesc *boxes, const Arrays &A, const PW 
   aps.open(seed, box, step, site, ordinal, RNG_ACC_POISSON);
   smp.open(seed, box, step, site, ordinal, RNG_ACC_SAMPLE);
   fin.open(seed, box, step, site, ordinal, RNG_ACC_FINISH);
-  Rec target, source;
+  RecN<NS> target, source;
   load_rec(A, p, target);
   RmChain chain{-1, -1, RM_CHUNK, 0, 0ull};
   RmChain reads{-1, -1, RM_CHUNK, 0, 0ull};
@@ -1790,7 +1809,7 @@ __device__ __noinline__ int acc_visit(BoxDesc *boxes, const Arrays &A, const PW 
   }
   const int n_rm = chain.n;
   int n_dup = 0, dup_head = -1, dup_tail = -1;
-  Rec np = target;
+  RecN<NS> np = target;
   if (n_coag > 0) {
     // coag_target_with_source (src/coagulation.F90:522-582)
     Stream ft;
@@ -1820,11 +1839,11 @@ __device__ __noinline__ int acc_visit(BoxDesc *boxes, const Arrays &A, const PW 
           atomicExch(&B->error, ERR_CAPACITY);
           return -1;
         }
-        Rec cp = np;
+        RecN<NS> cp = np;
         cp.group = rand_group_w(ft, w, np.klass, r_new);
         pool_store(W, ns, d, cp);
-        W.q_next[d] = -1;
-        if (dup_tail >= 0) W.q_next[dup_tail] = d;
+        W.q[d].next = -1;
+        if (dup_tail >= 0) W.q[dup_tail].next = d;
         else dup_head = d;
         dup_tail = d;
         n_dup++;
@@ -1832,24 +1851,32 @@ __device__ __noinline__ int acc_visit(BoxDesc *boxes, const Arrays &A, const PW 
     }
   }
   if (warn) flags |= RF_WARN;
-  W.r_rdhead[rec] = reads.head;
-  W.r_nrd[rec] = reads.n;
+  W.ev[rec].rdhead = reads.head;
+  W.ev[rec].nrd = reads.n;
   if (n_coag == 0 && n_rm == 0 && err_code == 0) {
     *tns = n_samp | (warn ? ACC_WARN : 0);
     return 0;
   }
   if (flags & RF_MERGED) pool_store(W, ns, rec, np);
-  W.r_nsamp[rec] = n_samp;
-  W.r_ncoag[rec] = n_coag;
-  W.r_nrm[rec] = n_rm;
-  W.r_nchain[rec] = chain.n;
-  W.r_head[rec] = chain.head;
-  W.r_ndup[rec] = n_dup;
-  W.r_dhead[rec] = dup_head;
-  W.r_flags[rec] = flags;
-  W.r_err[rec] = err_code;
+  W.ev[rec].nsamp = n_samp;
+  W.ev[rec].ncoag = n_coag;
+  W.ev[rec].nrm = n_rm;
+  W.ev[rec].nchain = chain.n;
+  W.ev[rec].head = chain.head;
+  W.ev[rec].ndup = n_dup;
+  W.ev[rec].dhead = dup_head;
+  W.ev[rec].flags = flags;
+  W.ev[rec].err = err_code;
   if (claim) claim_write(W, p, t);
   return 1;
+}
+
+__device__ inline int run_visit(BoxDesc *boxes, const Arrays &A, int64_t k, uint32_t t, int rec,
+                                int type, uint64_t seed, uint32_t step, double del_t, bool claim,
+                                int *p_out, int *tns) {
+  return A.n_spec <= FEW_SPEC
+             ? acc_visit<FEW_SPEC>(boxes, k, t, rec, type, seed, step, del_t, claim, p_out, tns)
+             : acc_visit<MAX_SPEC>(boxes, k, t, rec, type, seed, step, del_t, claim, p_out, tns);
 }
 
 // visits per wavefront: each is one lane's serial sample loop, and fewer a
@@ -1881,12 +1908,12 @@ __device__ inline void acc_test(BoxDesc *boxes, const Arrays &A, const PW &W, in
   W.tp2[i] = -1;
   W.trec[i] = rec;
   int p, tns;
-  const int r = acc_visit(boxes, A, W, k, t, rec, type, seed, step, del_t, true, &p, &tns);
+  const int r = run_visit(boxes, A, k, t, rec, type, seed, step, del_t, true, &p, &tns);
   W.tp1[i] = p;
   W.tns[i] = tns;
   if (r == 1) W.acc[i] = 1;
   // the visit's samples, for the algorithmic traffic of this kernel
-  const int ns = (r == 1) ? W.r_nsamp[rec] : (tns & (TNS_SIDE2 - 1));
+  const int ns = (r == 1) ? W.ev[rec].nsamp : (tns & (TNS_SIDE2 - 1));
   if (ns > 0) atomicAdd(W.acc_samp, (unsigned long long)ns);
 }
 
@@ -1898,8 +1925,10 @@ k_par_acc_tests(BoxDesc *boxes, Arrays A, PW W, int n_box, int type, uint64_t se
   // every lane takes one; over the first round's target slots, ACC_LANES a
   // wavefront
   const int lanes = pend ? 64 : ACC_LANES;
-  if ((int)threadIdx.x >= lanes) return;
   const int count = pend ? W.rc[RC_N] : n_acc;
+  if ((int)blockIdx.x * lanes >= count) return;
+  step_ctx_fill(A, W);
+  if ((int)threadIdx.x >= lanes) return;
   for (int idx = blockIdx.x * lanes + threadIdx.x; idx < count; idx += gridDim.x * lanes)
     acc_test(boxes, A, W, n_box, type, seed, step, t0, pend, del_t, acc_base, idx);
 }
@@ -1956,12 +1985,12 @@ __device__ inline void resolve_event(BoxDesc *boxes, const Arrays &A, const PW &
     bool win = W.slot[p1].claim == t;
     rm_walk(W, r, [&](int q) { win = win && W.slot[q].claim == t; });
     rd_walk(W, r, [&](int q) { win = win && W.slot[q].claim_wr >= t; });
-    const int died = (W.r_flags[r] & RF_DIED) ? 1 : 0;
+    const int died = (W.ev[r].flags & RF_DIED) ? 1 : 0;
     W.ev_out[e] = win ? O_WIN : 0;
-    W.f_app[e] = win ? W.r_ndup[r] : 0;
-    W.f_id[e] = win ? W.r_ndup[r] : 0;
-    W.f_info[e] = win ? W.r_nrm[r] + died : 0;
-    W.f_hole[e] = win ? W.r_nrm[r] + died : 0;
+    W.f_app[e] = win ? W.ev[r].ndup : 0;
+    W.f_id[e] = win ? W.ev[r].ndup : 0;
+    W.f_info[e] = win ? W.ev[r].nrm + died : 0;
+    W.f_hole[e] = win ? W.ev[r].nrm + died : 0;
     W.f_lose[e] = win ? 0 : 1;
     return;
   }
@@ -1973,7 +2002,7 @@ __device__ inline void resolve_event(BoxDesc *boxes, const Arrays &A, const PW &
   Stream s;
   s.open(seed, m.box, step, pair_site(nb, nc, m.b1, m.b2, m.c1, m.c2), m.j, RNG_MERGE);
   int g;
-  const int d = merge_decide(A, W, B, s, p1, p2, m.c1, m.c2, cc, &g);
+  const int d = merge_decide(A, W, B, s, p1, p2, m.c1, m.c2, cc, &g, B->w);
   const bool win = ((d & O_RM1) ? W.slot[p1].claim == t : W.slot[p1].claim_wr > t) &&
                    ((d & O_RM2) ? W.slot[p2].claim == t : W.slot[p2].claim_wr > t);
   int o = 0;
@@ -2000,29 +2029,78 @@ __global__ void k_par_box_first(PW W) {
   }
 }
 
+// A particle's components, all MAX_COMP of them in wide loads that go out
+// together (a particle's 80 and 160 bytes are 16-byte aligned).  A load under
+// `if (c < n)` becomes a branch, and the compiler waits for every load in
+// flight at each one, one memory round trip per component.
+__device__ inline void load_comps(const int *csrc, const double *ctime, int64_t p, int *s,
+                                  double *t) {
+  static_assert(MAX_COMP % 4 == 0, "whole 16-byte words");
+  const int4 *ps = (const int4 *)(csrc + comp_at(p, 0));
+  const double2 *pt = (const double2 *)(ctime + comp_at(p, 0));
+#pragma unroll
+  for (int c = 0; c < MAX_COMP / 4; ++c) {
+    const int4 x = ps[c];
+    s[4 * c] = x.x;
+    s[4 * c + 1] = x.y;
+    s[4 * c + 2] = x.z;
+    s[4 * c + 3] = x.w;
+  }
+#pragma unroll
+  for (int c = 0; c < MAX_COMP / 2; ++c) {
+    const double2 x = pt[c];
+    t[2 * c] = x.x;
+    t[2 * c + 1] = x.y;
+  }
+}
+__device__ inline void load_comps(const Arrays &A, int64_t p, int *s, double *t) {
+  load_comps(A.csrc, A.ctime, p, s, t);
+}
+
+// Pool entry i written as the particle of class klass and identifier id in a
+// slot: its old particle leaves its list at t_leave, the new one joins at
+// t_join.  The slot's bookkeeping and the entry are read together.
 __device__ inline void write_new_particle(const Arrays &A, const PW &W, BoxDesc *B, int box,
                                           uint32_t t_leave, uint32_t t_join, int64_t slot,
-                                          bool appended, const Rec &r, int nb, int type,
-                                          int want_terms) {
+                                          bool appended, int i, int klass, int64_t id, int nb,
+                                          int type, int want_terms, const SlotView &sv) {
+  const PoolRec q = W.q[i];
+  int cs[MAX_COMP];
+  double ct[MAX_COMP];
+  load_comps(W.q_csrc, W.q_ctime, i, cs, ct);
   double v = 0.0;
   double m = 0.0;
-  for (int s = 0; s < A.n_spec; ++s) {
-    A.vol[(int64_t)s * A.total_cap + slot] = r.vol[s];
-    v += r.vol[s];
-    m += r.vol[s] * A.density[s];
+  const int ns = A.n_spec;
+  for (int s0 = 0; s0 < ns; s0 += SPEC_CHUNK) {
+    double x[SPEC_CHUNK], rho[SPEC_CHUNK];
+#pragma unroll
+    for (int u = 0; u < SPEC_CHUNK; ++u) {
+      const int s = s0 + u < ns ? s0 + u : ns - 1;
+      x[u] = W.q_vol[(int64_t)i * ns + s];
+      rho[u] = A.density[s];
+    }
+#pragma unroll
+    for (int u = 0; u < SPEC_CHUNK; ++u)
+      if (s0 + u < ns) {
+        A.vol[(int64_t)(s0 + u) * A.total_cap + slot] = x[u];
+        v += x[u];
+        m += x[u] * rho[u];
+      }
   }
   A.vtot[slot] = v;
-  A.id[slot] = r.id;
-  A.group[slot] = r.group;
-  A.klass[slot] = r.klass;
-  A.nprim[slot] = r.nprim;
-  A.ncomp[slot] = r.ncomp;
-  for (int c = 0; c < r.ncomp; ++c) {
-    A.csrc[comp_at(slot, c)] = r.csrc[c];
-    A.ctime[comp_at(slot, c)] = r.ctime[c];
-  }
-  A.least[slot] = r.least;
-  A.greatest[slot] = r.greatest;
+  A.id[slot] = id;
+  A.group[slot] = q.group;
+  A.klass[slot] = klass;
+  A.nprim[slot] = q.nprim;
+  A.ncomp[slot] = q.ncomp;
+#pragma unroll
+  for (int c = 0; c < MAX_COMP; ++c)
+    if (c < q.ncomp) {
+      A.csrc[comp_at(slot, c)] = cs[c];
+      A.ctime[comp_at(slot, c)] = ct[c];
+    }
+  A.least[slot] = q.least;
+  A.greatest[slot] = q.greatest;
   int b = bin_find_log(nb, B->log_lo, B->log_hi, vol2rad(v));
   if (b < 1 || b > nb) {
     atomicExch(&B->error, 134572570);
@@ -2030,9 +2108,9 @@ __device__ inline void write_new_particle(const Arrays &A, const PW &W, BoxDesc 
     W.key[slot] = 0;
     return;
   }
-  int k = par_key(b, r.klass, nb);
+  int k = par_key(b, klass, nb);
   if (appended) slot_append(W, B, box, slot, t_join, k);
-  else slot_write(W, B, box, slot, t_leave, t_join, k, slot_load(W, slot));
+  else slot_write(W, B, box, slot, t_leave, t_join, k, sv);
   st_set(W, slot, ST_NEW);
   W.key[slot] = k;
   if (want_terms) W.terms[slot] = particle_terms(type, v, m / v, B->env);
@@ -2162,30 +2240,6 @@ __device__ inline void put_info(const Arrays &A, BoxDesc *B, Alloc &al, int64_t 
     A.info_id[B->info_off + k] = id;
     A.info_action[B->info_off + k] = action;
     A.info_other[B->info_off + k] = other;
-  }
-}
-
-// A particle's components, all MAX_COMP of them in wide loads that go out
-// together (a particle's 80 and 160 bytes are 16-byte aligned).  A load under
-// `if (c < n)` becomes a branch, and the compiler waits for every load in
-// flight at each one, one memory round trip per component.
-__device__ inline void load_comps(const Arrays &A, int64_t p, int *s, double *t) {
-  static_assert(MAX_COMP % 4 == 0, "whole 16-byte words");
-  const int4 *ps = (const int4 *)(A.csrc + comp_at(p, 0));
-  const double2 *pt = (const double2 *)(A.ctime + comp_at(p, 0));
-#pragma unroll
-  for (int c = 0; c < MAX_COMP / 4; ++c) {
-    const int4 x = ps[c];
-    s[4 * c] = x.x;
-    s[4 * c + 1] = x.y;
-    s[4 * c + 2] = x.z;
-    s[4 * c + 3] = x.w;
-  }
-#pragma unroll
-  for (int c = 0; c < MAX_COMP / 2; ++c) {
-    const double2 x = pt[c];
-    t[2 * c] = x.x;
-    t[2 * c + 1] = x.y;
   }
 }
 
@@ -2424,7 +2478,7 @@ __device__ inline void perset_merge(BoxDesc *B, const Arrays &A, const PW &W, in
     s = *post;
   } else if (P.n1 + P.n2 > MAX_COMP && !resampled) {
     s.open(seed, box, step, pair_site(nb, nc, b1, b2, c1, c2), t - W.pair_exc[k], RNG_MERGE);
-    (void)merge_decide(A, W, B, s, p1, p2, c1, c2, cc, &new_group);
+    (void)merge_decide(A, W, B, s, p1, p2, c1, c2, cc, &new_group, B->w);
   }
   int64_t info_other = 0;
   int64_t slot = -1;
@@ -2524,17 +2578,19 @@ __device__ inline bool wave_resamplings(const Arrays &A, const BoxDesc *B, bool 
 // are appended with new identifiers in creation order, and a target or
 // copy that kept no copy of itself is removed with a weighting record.
 template <class Alloc>
-__device__ __noinline__ void acc_apply(BoxDesc *B, const Arrays &A, const PW &W, int box, uint32_t t,
-                                 int r, int64_t p, int type, int want_terms, int rid, Alloc &al,
-                                 bool chain_elsewhere = false) {
-  const int ns = A.n_spec;
+__device__ __noinline__ void acc_apply(BoxDesc *B, int box, uint32_t t, int r, int64_t p, int type,
+                                       int want_terms, int rid, Alloc &al,
+                                       bool chain_elsewhere = false) {
+  const Arrays &A = s_ctx.A;
+  const PW &W = s_ctx.W;
   const int nb = B->n_bin;
   const int64_t target_id = A.id[p];
   const int klass = A.klass[p];
-  const int flags = W.r_flags[r];
+  const EventRec ev = W.ev[r];
+  const int flags = ev.flags;
   // copy identifiers in creation order, drawn before any record names them
   int64_t id_first = 0;
-  for (int kk = 0; kk < W.r_ndup[r]; ++kk) {
+  for (int kk = 0; kk < ev.ndup; ++kk) {
     int64_t v = al.new_id();
     if (kk == 0) id_first = v;
   }
@@ -2542,8 +2598,8 @@ __device__ __noinline__ void acc_apply(BoxDesc *B, const Arrays &A, const PW &W,
   if (chain_elsewhere) {
     // the removed sources are applied by a wavefront (k_par_apply_chains)
     // at this event's first hole and record ranks
-    al.hole += W.r_nrm[r];
-    al.info += W.r_nrm[r];
+    al.hole += ev.nrm;
+    al.info += ev.nrm;
   } else {
     int64_t owner = target_id;
     chain_walk(W, r, [&](int q) {
@@ -2560,19 +2616,18 @@ __device__ __noinline__ void acc_apply(BoxDesc *B, const Arrays &A, const PW &W,
       put_info(A, B, al, A.id[q], 2, owner);
     });
   }
-  const unsigned long long n_samp = (unsigned long long)W.r_nsamp[r];
-  const unsigned long long n_coag = (unsigned long long)W.r_ncoag[r];
+  const unsigned long long n_samp = (unsigned long long)ev.nsamp;
+  const unsigned long long n_coag = (unsigned long long)ev.ncoag;
   al.count((int64_t)n_samp, (int64_t)n_coag, (flags & RF_WARN) ? 1 : 0);
   atomicAdd((unsigned long long *)&B->n_acc_samp, n_samp);
   if (n_coag) atomicAdd((unsigned long long *)&B->n_acc_coag, n_coag);
-  if (W.r_err[r]) atomicExch(&B->error, W.r_err[r]);
+  if (ev.err) atomicExch(&B->error, ev.err);
   if (!(flags & RF_MERGED)) return;
-  Rec np;
-  pool_load(W, ns, r, klass, target_id, np);
+  const SlotView sv = slot_load(W, p);
   W.slot[p].dead_t = t;
   W.slot[p].dead_r = rid;
-  al.live_add(W.key[p], -1);
-  write_new_particle(A, W, B, box, t, t, p, false, np, nb, type, want_terms);
+  al.live_add(sv.key, -1);
+  write_new_particle(A, W, B, box, t, t, p, false, r, klass, target_id, nb, type, want_terms, sv);
   if (flags & RF_DIED) {
     slot_leave(W, p, t);
     st_set(W, p, ST_HOLE);
@@ -2582,15 +2637,15 @@ __device__ __noinline__ void acc_apply(BoxDesc *B, const Arrays &A, const PW &W,
     al.live_add(W.key[p], 1);
   }
   int kk = 0;
-  for (int d = W.r_dhead[r]; d >= 0; d = W.q_next[d]) {
+  for (int d = ev.dhead; d >= 0; d = W.q[d].next) {
     ++kk;
-    pool_load(W, ns, d, klass, copy_id(kk), np);
     const int64_t slot = al.append_slot();
     if (slot < 0) {
       atomicExch(&B->error, ERR_CAPACITY);
       return;
     }
-    write_new_particle(A, W, B, box, t, t, slot, true, np, nb, type, want_terms);
+    write_new_particle(A, W, B, box, t, t, slot, true, d, klass, copy_id(kk), nb, type, want_terms,
+                       SlotView{});
     al.live_add(W.key[slot], 1);
   }
 }
@@ -2617,8 +2672,8 @@ __device__ inline void apply_event(BoxDesc *boxes, const Arrays &A, const PW &W,
     al.n_samp = al.n_coag = al.n_warn = 0;
     al.nl = 0;
     if (W.ev_rec[e] >= 0) {
-      acc_apply(B, A, W, box, t, W.ev_rec[e], W.ev_p1[e], type, want_terms, rid, al,
-                W.r_nchain[W.ev_rec[e]] > CHAIN_WAVE_MIN);
+      acc_apply(B, box, t, W.ev_rec[e], W.ev_p1[e], type, want_terms, rid, al,
+                W.ev[W.ev_rec[e]].nchain > CHAIN_WAVE_MIN);
     } else {
       const int64_t k = test_pair(W, (int64_t)n_box * W.P_stride, t);
       perset_merge(B, A, W, box, k, k - (int64_t)box * W.P_stride, t, W.ev_p1[e], W.ev_p2[e], seed,
@@ -2644,6 +2699,8 @@ __global__ void __launch_bounds__(256)
 k_par_apply(BoxDesc *boxes, Arrays A, PW W, int n_box, uint64_t seed, uint32_t step,
             int type, int want_terms, int rid) {
   const int E = W.rc[RC_E];
+  if ((int)(blockIdx.x * blockDim.x) >= E) return;
+  step_ctx_fill(A, W);
   const int64_t hole_base = (int64_t)*W.hole_top;
   // the loop bound is uniform over the workgroup: every lane reaches the
   // wavefront flushes of each pass
@@ -2662,7 +2719,7 @@ __device__ inline void apply_chain(BoxDesc *boxes, const Arrays &A, const PW &W,
                                    int64_t hole_base, int rid) {
   if (!(W.ev_out[e] & O_WIN)) return;
   const int r = W.ev_rec[e];
-  if (r < 0 || W.r_nchain[r] <= CHAIN_WAVE_MIN) return;
+  if (r < 0 || W.ev[r].nchain <= CHAIN_WAVE_MIN) return;
   const uint32_t t = W.ev_t[e];
   const int box = W.ev_box[e];
   BoxDesc *B = &boxes[box];
@@ -2674,8 +2731,8 @@ __device__ inline void apply_chain(BoxDesc *boxes, const Arrays &A, const PW &W,
   int *live = W.live + (int64_t)box * W.K_stride;
   int64_t owner = A.id[W.ev_p1[e]];
   int done = 0;  // removed sources before this chunk
-  int left = W.r_nchain[r];
-  for (int ch = W.r_head[r]; ch >= 0 && left > 0; ch = W.rm_buf[ch]) {
+  int left = W.ev[r].nchain;
+  for (int ch = W.ev[r].head; ch >= 0 && left > 0; ch = W.rm_buf[ch]) {
     const int m = left < RM_CHUNK - 1 ? left : RM_CHUNK - 1;
     const bool here = lane < m;
     const int q = here ? W.rm_buf[ch + 1 + lane] : 0;
@@ -2979,6 +3036,7 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
   const int lo = lower_bound_u32(pend, n, W.pair_exc[pb]);
   const int hi = lower_bound_u32(pend, n, W.pair_exc[pb + W.P_stride]);
   if (lo >= hi) return;
+  step_ctx_fill(A, W);
   __shared__ scan_storage<TAIL_THREADS, int> scan_tmp;
   __shared__ scan_storage<TAIL_THREADS, uint32_t> scan_tmp3;
   __shared__ uint32_t s_carry;
@@ -3039,13 +3097,14 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
     if (active && (fl & TF_RUN)) {
       fl &= ~(TF_RUN | TF_EFFECT | TF_WARN | TF_ATHIN | TF_SIDE2 | TF_WAIT);
       if (is_acc) {
-        const int r = acc_visit(boxes, A, W, k, t, rec, type, seed, step, del_t, false, &p1, &tns);
+        const int r = run_visit(boxes, A, k, t, rec, type, seed, step, del_t, false, &p1, &tns);
         if (r == 1) fl |= TF_EFFECT;
         if (tns & TNS_ATHIN) fl |= TF_ATHIN;
         p2 = -1;
       } else {
         TestOut o;
-        perset_test(B, A, W, box, k, k - pb, t, type, seed, step, precision, band, 0, o, &s_w);
+        perset_test(B, A, W, box, k, k - pb, t, type, seed, step, precision, band, 0, o,
+                    s_w);
         p1 = o.p1;
         p2 = o.p2;
         W.thin[t - batch_t0] = o.thin ? 1 : 0;
@@ -3067,7 +3126,7 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
       const int cc = A.cc[table_index(A, box, nb, nc, b1, b2, c1, c2)];
       ms.open(seed, box, step, pair_site(nb, nc, b1, b2, c1, c2), t - W.pair_exc[k], RNG_MERGE);
       int g;
-      o_win = merge_decide(A, W, B, ms, p1, p2, c1, c2, cc, &g, &s_w) | (g << 16);
+      o_win = merge_decide(A, W, B, ms, p1, p2, c1, c2, cc, &g, s_w) | (g << 16);
     }
     // 2. claims
     if (effect) {
@@ -3095,11 +3154,11 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
         rm_walk(W, rec, [&](int q) { win = win && claim_load(W, q) == t; });
         rd_walk(W, rec, [&](int q) { win = win && claim_wr_load(W, q) >= t; });
         if (win) {
-          const int died = (W.r_flags[rec] & RF_DIED) ? 1 : 0;
-          c_app = W.r_ndup[rec];
-          c_id = W.r_ndup[rec];
-          c_info = W.r_nrm[rec] + died;
-          c_hole = W.r_nrm[rec] + died;
+          const int died = (W.ev[rec].flags & RF_DIED) ? 1 : 0;
+          c_app = W.ev[rec].ndup;
+          c_id = W.ev[rec].ndup;
+          c_info = W.ev[rec].nrm + died;
+          c_hole = W.ev[rec].nrm + died;
         }
       } else {
         const int o = o_win & 0xFFFF;
@@ -3144,7 +3203,7 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
       al.live = nullptr;
       al.s_live = s_live;
       al.n_samp = al.n_coag = al.n_warn = 0;
-      if (is_acc) acc_apply(B, A, W, box, t, rec, p1, type, want_terms, rid, al);
+      if (is_acc) acc_apply(B, box, t, rec, p1, type, want_terms, rid, al);
       else perset_merge(B, A, W, box, k, k - pb, t, p1, p2, seed, step, type, want_terms, rid, al,
                         o_win, &ms, resampled, par);
       c_samp += al.n_samp;
@@ -3434,16 +3493,13 @@ inline int parallel_init(ParallelWork &W, int n_box, int max_bin) {
 // the accelerated path's records, allocated when a step first has target slots
 inline void parallel_free_records(ParallelWork &W) {
   PW &d = W.d;
-  void *ptrs[] = {d.r_rdhead, d.r_nrd, d.r_nsamp, d.r_ncoag, d.r_nrm, d.r_nchain, d.r_head, d.r_ndup,
-                  d.r_dhead, d.r_flags, d.r_err, d.q_vol, d.q_group, d.q_nprim, d.q_ncomp,
-                  d.q_next, d.q_csrc, d.q_ctime, d.q_least,
-                  d.q_greatest, d.dup_top, d.rm_buf, d.rm_top};
+  void *ptrs[] = {d.ev, d.q_vol, d.q, d.q_csrc, d.q_ctime, d.dup_top, d.rm_buf, d.rm_top};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
-  d.r_nsamp = d.r_ncoag = d.r_nrm = d.r_nchain = d.r_head = d.r_ndup = nullptr;
-  d.r_dhead = d.r_flags = d.r_err = d.r_rdhead = d.r_nrd = nullptr;
-  d.q_vol = d.q_ctime = d.q_least = d.q_greatest = nullptr;
-  d.q_group = d.q_nprim = d.q_ncomp = d.q_next = d.q_csrc = nullptr;
+  d.ev = nullptr;
+  d.q = nullptr;
+  d.q_vol = d.q_ctime = nullptr;
+  d.q_csrc = nullptr;
   d.dup_top = d.rm_buf = d.rm_top = nullptr;
   d.acc_cap = d.pool_cap = d.rm_cap = 0;
 }
@@ -3451,16 +3507,11 @@ inline void parallel_free_records(ParallelWork &W) {
 inline int parallel_alloc_records(ParallelWork &W, int n_spec) {
   PW &d = W.d;
   const int64_t c = ACC_CAP, pc = (int64_t)ACC_CAP + DUP_CAP;
-  int **rv[] = {&d.r_nsamp, &d.r_ncoag, &d.r_nrm, &d.r_nchain, &d.r_head, &d.r_ndup,
-                &d.r_dhead, &d.r_flags, &d.r_err, &d.r_rdhead, &d.r_nrd};
-  for (int **q : rv) PCHECK(pmalloc(q, c));
+  PCHECK(pmalloc(&d.ev, c));
+  PCHECK(pmalloc(&d.q, pc));
   PCHECK(pmalloc(&d.q_vol, (size_t)n_spec * pc));
   PCHECK(pmalloc(&d.q_csrc, (size_t)MAX_COMP * pc));
   PCHECK(pmalloc(&d.q_ctime, (size_t)MAX_COMP * pc));
-  int **qv[] = {&d.q_group, &d.q_nprim, &d.q_ncomp, &d.q_next};
-  for (int **q : qv) PCHECK(pmalloc(q, pc));
-  PCHECK(pmalloc(&d.q_least, pc));
-  PCHECK(pmalloc(&d.q_greatest, pc));
   PCHECK(pmalloc(&d.dup_top, 1));
   PCHECK(pmalloc(&d.rm_buf, RM_CAP));
   PCHECK(pmalloc(&d.rm_top, 1));
@@ -3761,7 +3812,7 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
     scan_incl_max(scan_job(d.tp_in, d.tpair, d.scan_part, (int64_t)T), (int64_t)T, st);
     d.tpair_ok = 1;
   }
-  if (T_acc > 0 && d.r_nsamp == nullptr) {
+  if (T_acc > 0 && d.ev == nullptr) {
     int e = parallel_alloc_records(W, A.n_spec);
     if (e) return e;
   }
