@@ -192,6 +192,7 @@ static int alloc_tables(pmc_gpu *h, int classes) {
 // particles already uploaded, their bin lists (the list order is state the
 // next step depends on) and the removal logs.
 static int layout(pmc_gpu *h, const std::vector<int64_t> &new_cap) {
+  h->work.clean_type = 0;
   std::vector<BoxDesc> hb(h->n_box);
   HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
   Arrays old = h->A;
@@ -300,6 +301,11 @@ static int set_field(pmc_gpu *h, int box, size_t offset, const T &v) {
   return 0;
 }
 #define SET_FIELD(h, box, field, v) set_field(h, box, offsetof(BoxDesc, field), v)
+
+// Called by every entry point that changes a box's particles, weights,
+// environment, grid or layout: the next parallel step looks for stale keys,
+// terms and tables again.
+static void boxes_changed(pmc_gpu *h) { h->work.clean_type = 0; }
 
 static int check_box(pmc_gpu *h, int box) {
   if (!h) return fail(ERR_ARG, "null handle");
@@ -454,6 +460,7 @@ int pmc_gpu_destroy(pmc_gpu *h) {
 int pmc_gpu_set_env(pmc_gpu *h, int box, double temp, double pressure, double additive_coeff) {
   int e = check_box(h, box);
   if (e) return e;
+  boxes_changed(h);
   Env env = make_env(temp, pressure, additive_coeff);
   HIPCHECK(hipSetDevice(h->device));
   HIPCHECK(hipStreamSynchronize(h->stream));
@@ -466,6 +473,7 @@ int pmc_gpu_set_weights(pmc_gpu *h, int box, int n_group, int n_class, const int
                         const double *magnitude, const double *exponent) {
   int e = check_box(h, box);
   if (e) return e;
+  boxes_changed(h);
   if (n_group < 1 || n_group > MAX_GROUP || n_class < 1 || n_class > MAX_CLASS || !type ||
       !magnitude || !exponent)
     return fail(ERR_ARG, "set_weights: n_group %d / n_class %d outside 1..%d/1..%d", n_group,
@@ -512,6 +520,7 @@ int pmc_gpu_set_next_id(pmc_gpu *h, int box, int64_t next_id, int64_t id_stride,
                         int64_t id_offset) {
   int e = check_box(h, box);
   if (e) return e;
+  boxes_changed(h);
   if (id_stride < 1) return fail(ERR_ARG, "id_stride must be >= 1");
   HIPCHECK(hipSetDevice(h->device));
   if ((e = SET_FIELD(h, box, next_id, next_id))) return e;
@@ -606,6 +615,7 @@ int pmc_gpu_upload(pmc_gpu *h, int box, int n_part, int capacity, const double *
                    const double *least, const double *greatest) {
   int e = check_box(h, box);
   if (e) return e;
+  boxes_changed(h);
   if (n_part < 0 || (n_part > 0 && (!vol || !id || !group || !klass)))
     return fail(ERR_ARG, "upload: bad arguments");
   if (n_comp && (!comp_source || !comp_time))
@@ -693,6 +703,7 @@ static int enqueue_prep_lists(pmc_gpu *h, int only_box) {
 int pmc_gpu_set_bin_grid(pmc_gpu *h, int box, int n_bin, double r_min, double r_max) {
   int e = check_box(h, box);
   if (e) return e;
+  boxes_changed(h);
   if (n_bin < 0 || n_bin > h->max_bin)
     return fail(ERR_ARG, "set_bin_grid: n_bin %d outside 0..%d", n_bin, h->max_bin);
   if (n_bin > 0 && !(r_min > 0.0 && r_min < r_max))
@@ -843,6 +854,7 @@ int pmc_gpu_mc_coag_async(pmc_gpu *h, int kernel_type, double del_t) {
       if (h->tape_buf[b])
         return fail(ERR_STATE, "box %d records or replays a tape: that is the exact mode's", b);
   if (h->mode == PMC_MODE_EXACT) {
+    boxes_changed(h);
     hipEvent_t ev;
     timing_begin(h, "k_prepare", &ev);
     hipLaunchKernelGGL(k_prep_radii, dim3(PREP_RADII_WG, h->n_box), dim3(256), 0, h->stream,
@@ -1236,6 +1248,7 @@ static int run_removal(pmc_gpu *h, const std::vector<BoxDesc> &hb, const std::ve
 // twice its ideal number.
 int pmc_gpu_rebalance(pmc_gpu *h, int allow_doubling, int allow_halving) {
   if (!h) return fail(ERR_ARG, "null handle");
+  boxes_changed(h);
   if ((int)h->n_part_ideal.size() != h->n_box)
     return fail(ERR_STATE, "rebalance: set_n_part_ideal first");
   for (int b = 0; b < h->n_box; ++b)
@@ -1381,6 +1394,7 @@ int pmc_gpu_rebalance(pmc_gpu *h, int allow_doubling, int allow_halving) {
 // A removal pass of every box with a per-box parameter (dilution
 // probability or mixing height) after the usual checks.
 static int removal_all(pmc_gpu *h, Removal X, const double *per_box) {
+  boxes_changed(h);
   HIPCHECK(hipSetDevice(h->device));
   HIPCHECK(hipStreamSynchronize(h->stream));
   int e = rebal_ensure(h, true);
@@ -1443,6 +1457,7 @@ int pmc_gpu_append(pmc_gpu *h, int box, int n, const double *vol, const int64_t 
                    const double *greatest) {
   int e = check_box(h, box);
   if (e) return e;
+  boxes_changed(h);
   if (n < 0 || (n > 0 && (!vol || !group || !klass)))
     return fail(ERR_ARG, "append: bad arguments");
   if (n_comp && (!comp_source || !comp_time))
@@ -1494,6 +1509,7 @@ int pmc_gpu_append(pmc_gpu *h, int box, int n, const double *vol, const int64_t 
 int pmc_gpu_scale_weights(pmc_gpu *h, int box, double factor) {
   int e = check_box(h, box);
   if (e) return e;
+  boxes_changed(h);
   if (!(factor > 0.0)) return fail(ERR_ARG, "scale_weights: factor must be > 0");
   HIPCHECK(hipSetDevice(h->device));
   HIPCHECK(hipStreamSynchronize(h->stream));

@@ -88,6 +88,7 @@ struct PW {  // device view of the parallel work arrays
   int *key;         // [total_cap] list key, -1 for no key
   SlotRec *slot;    // [total_cap]
   int epoch;        // this step's status epoch, 1..63
+  int tag;          // this step's tag (RC_REGRID)
   float4 *terms;    // [total_cap]
   int *perm;        // [total_cap] global slots sorted by (box, key)
   int *tile_box, *tile_start, *tiles_in_box;
@@ -99,8 +100,8 @@ struct PW {  // device view of the parallel work arrays
   uint32_t *tid, *pend;
   uint32_t *ev_t;
   int *ev_p1, *ev_p2, *ev_box, *ev_out;
-  int *f_app, *f_id, *f_info, *f_hole, *f_lose, *f_pend, *s_pend;
-  int *s_app, *s_id, *s_info, *s_hole, *s_lose;
+  int *f_app, *f_id, *f_info, *f_hole, *f_pend, *s_pend;
+  int *s_app, *s_id, *s_info, *s_hole;
   int *box_first;
   uint64_t *holes, *holes_sorted;  // (box << 32 | slot)
   int *cmp_lo, *cmp_hi, *cmp_head;
@@ -125,10 +126,9 @@ struct PW {  // device view of the parallel work arrays
   int *rm_buf;                 // chunks: [0] next chunk or -1, [1..RM_CHUNK) removed slots
   int *rm_top;                 // [1] chunk allocator of the round
   int rm_cap;
-  uint32_t *misc;              // [8] batch bounds from k_batch_end
   unsigned long long *hole_top;  // [8] hole counter; then tail_rounds and rstat
   int *pend_k;                 // [T_cap] pair of each pending test entering the tail
-  uint32_t *tp_in, *tpair;     // [T_cap] pair of every test of a single-batch step
+  uint32_t *tpair;             // [T_cap] pair of every test of a single-batch step
   int tpair_ok;                // tpair is current for this step
   unsigned long long *tail_rounds;  // [1] claim rounds run by the tail, summed over boxes
   // Particles that join a list within the step ("arrivals": a merged
@@ -159,7 +159,8 @@ struct PW {  // device view of the parallel work arrays
   // The counts that drive a batch's claim rounds, kept on the device so the
   // host launches every round without reading them back: RC_N tests of the
   // current device-wide round (0: the round does not run), RC_E its events,
-  // RC_TAIL the tests left to the tail.
+  // RC_TAIL the tests left to the tail; RC_REGRID the tag of the last step
+  // that gave a box a new grid.
   int *rc;                      // [RC_SIZE]
   unsigned long long *pstat;    // [2] device-wide rounds run, tests left to the tail
   // the batch's round sizes, read back with the hole count after the tail to
@@ -169,7 +170,7 @@ struct PW {  // device view of the parallel work arrays
   unsigned long long *rstat;    // [4]
 };
 
-constexpr int RC_N = 0, RC_E = 1, RC_TAIL = 2, RC_SIZE = 4;
+constexpr int RC_N = 0, RC_E = 1, RC_TAIL = 2, RC_REGRID = 3, RC_SIZE = 4;
 
 constexpr int ACC_CAP = 1 << 18;
 constexpr int DUP_CAP = 1 << 18;
@@ -213,6 +214,11 @@ struct ParallelWork {
   // the last batch's round 0 events, round 1 tests and events, tail tests
   // (-1: none yet): the grids of the next step's rounds are sized from them
   int64_t est[4] = {-1, -1, -1, -1};
+  // The last step left every box's keys, terms and tables current for this
+  // kernel type and precision (0: not, or a call changed a box since), with
+  // grids of at most mb_step bins.
+  int clean_type = 0, clean_terms = 0, mb_step = 0;
+  int tag = 0;                // the last step's tag (RC_REGRID)
 };
 
 #define PLAUNCH(W, name, ...)                                   \
@@ -342,14 +348,42 @@ __global__ void k_par_reset_minmax(BoxDesc *boxes, int n_box) {
   boxes[box].rmax_bits = 0ull;
 }
 
-// aero_sorted_remake_if_needed, src/aero_sorted.F90:214-373, one thread
-// per box, occupancy from the live counts
-__global__ void k_par_remake(BoxDesc *boxes, Arrays A, PW W, int n_box) {
-  int box = blockIdx.x * blockDim.x + threadIdx.x;
-  if (box >= n_box) return;
+// The start of a step, one wavefront a box: its counters, the round state it
+// owns cleared, and aero_sorted_remake_if_needed
+// (src/aero_sorted.F90:214-373) with the occupancy from the live counts.  A
+// box that gets a new grid tags the step: what was launched behind this
+// kernel for the old grid then does nothing, and the host starts over from
+// the keys.  (One thread a box walked the live counts and made the grid:
+// 25 us for 160 bins, 4 here.)
+__global__ void __launch_bounds__(64) k_step_front(BoxDesc *boxes, Arrays A, PW W, int64_t NP) {
+  const int box = blockIdx.x, lane = threadIdx.x;
   BoxDesc *B = &boxes[box];
-  B->regridded = 0;
-  B->rekey = 0;
+  for (int k = lane; k < W.K_stride; k += 64) {
+    // at the start of the first round every event of the batch is pending
+    W.minpend[(int64_t)box * W.K_stride + k] = 0u;
+    W.minpend_next[(int64_t)box * W.K_stride + k] = UNCLAIMED;
+  }
+  if (lane == 0) {
+    W.box_first[box] = -1;
+    B->step_samp = 0;
+    B->step_coag = 0;
+    B->part_steps += B->n_part;
+    B->regridded = 0;
+    B->rekey = 0;
+    if (box == 0) {
+      *W.hole_top = 0ull;
+      *W.tail_rounds = 0ull;
+      *W.ap_top = 0u;
+      if (W.ev) {
+        *W.rm_top = 0;
+        *W.dup_top = 0;
+      }
+      if (NP > 0) {  // what the pair scans read as their last input
+        W.pair_n[NP] = 0;
+        W.pair_accn[NP] = 0;
+      }
+    }
+  }
   if (B->error) return;
   double *edges = A.edges + (int64_t)box * (A.max_bin + 1);
   double *centers = A.centers + (int64_t)box * A.max_bin;
@@ -359,23 +393,27 @@ __global__ void k_par_remake(BoxDesc *boxes, Arrays A, PW W, int n_box) {
   double rmin = 0.0, rmax = 0.0;
   if (use_counts) {
     const int *live = W.live + (int64_t)box * W.K_stride;
-    int i_min = 0, i_max = 0;
-    for (int b = 1; b <= nb; ++b) {
+    int first = nb + 1, last = 0;
+    for (int b = 1 + lane; b <= nb; b += 64) {
       int tot = 0;
       for (int c = 1; c <= nc; ++c) tot += live[par_key(b, c, nb)];
       if (tot > 0) {
-        if (i_min == 0) i_min = b;
-        i_max = b;
+        first = min(first, b);
+        last = max(last, b);
       }
     }
-    if (i_min == 0) {
+    for (int o = 32; o > 0; o >>= 1) {
+      first = min(first, __shfl_xor(first, o));
+      last = max(last, __shfl_xor(last, o));
+    }
+    if (last == 0) {
       if (nb > 0) {
         rmin = edges[nb];
         rmax = edges[0];
       }
     } else {
-      rmin = edges[i_min - 1];
-      rmax = edges[i_max];
+      rmin = edges[first - 1];
+      rmax = edges[last];
     }
   } else if (B->valid_sort && nb > 0) {
     // a valid sort whose keys were dropped (population control moved
@@ -395,41 +433,45 @@ __global__ void k_par_remake(BoxDesc *boxes, Arrays A, PW W, int n_box) {
     rmax = __longlong_as_double((long long)B->rmax_bits);
   }
   if (rmax == 0.0) {
-    if (!use_counts) {
-      B->n_bin = 0;
-      B->bounds_valid = 0;
-      B->tables_valid = 0;
+    if (lane == 0) {
+      if (!use_counts) {
+        B->n_bin = 0;
+        B->bounds_valid = 0;
+        B->tables_valid = 0;
+      }
+      B->valid_sort = 1;
+      B->pkeys_valid = 1;
     }
-    B->valid_sort = 1;
-    B->pkeys_valid = 1;
     return;
   }
-  bool need = (nb < 1) || (rmin / edges[0] < 3.0) || (edges[nb] / rmax < 3.0);
+  const bool need = (nb < 1) || (rmin / edges[0] < 3.0) || (edges[nb] / rmax < 3.0);
   if (need) {
-    double gmin = rmin / 10.0, gmax = rmax * 10.0;
-    double nbf = ceil((log10(gmax) - log10(gmin)) * 10.0);
-    if (nbf < 0.0) {
-      B->error = 538534122;
+    const double gmin = rmin / 10.0, gmax = rmax * 10.0;
+    const double nbf = ceil((log10(gmax) - log10(gmin)) * 10.0);
+    if (nbf < 0.0 || nbf > (double)A.max_bin) {
+      if (lane == 0) B->error = nbf < 0.0 ? 538534122 : ERR_CAPACITY;
       return;
     }
-    if (nbf > (double)A.max_bin) {
-      B->error = ERR_CAPACITY;
-      return;
+    const int nn = (int)nbf;
+    make_log_grid_wave(nn, gmin, gmax, edges, centers, widths);
+    if (lane == 0) {
+      B->n_bin = nn;
+      B->log_lo = log(gmin);
+      B->log_hi = log(gmax);
+      B->bounds_valid = 0;
+      B->tables_valid = 0;
+      B->regridded = 1;
+      B->rekey = 1;
+      W.rc[RC_REGRID] = W.tag;
     }
-    int nn = (int)nbf;
-    make_log_grid(nn, gmin, gmax, edges, centers, widths);
-    B->n_bin = nn;
-    B->log_lo = log(edges[0]);
-    B->log_hi = log(edges[nn]);
-    B->bounds_valid = 0;
-    B->tables_valid = 0;
-    B->regridded = 1;
+  } else if (!use_counts && lane == 0) {
     B->rekey = 1;
-  } else if (!use_counts) {
-    B->rekey = 1;
+    W.rc[RC_REGRID] = W.tag;
   }
-  B->valid_sort = 1;
-  B->xlists_valid = 0;
+  if (lane == 0) {
+    B->valid_sort = 1;
+    B->xlists_valid = 0;
+  }
 }
 
 // tile histogram of keys into hist[box][key][tile]
@@ -453,24 +495,6 @@ k_par_hist(BoxDesc *boxes, PW W) {
   const int nt = W.tiles_in_box[box];
   uint32_t *h = W.hist + (int64_t)K * W.tile_first[box];
   for (int k = threadIdx.x; k < K; k += TILE_THREADS) h[(int64_t)k * nt + t_in_box] = (uint32_t)s_h[k];
-}
-
-// list starts and counts of every (box, key) from the scanned histogram
-__global__ void k_par_lists(BoxDesc *boxes, PW W, int n_box) {
-  const int box = blockIdx.y;
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= W.K_stride) return;
-  const int nt = W.tiles_in_box[box];
-  const int K = W.K_hist;
-  const int64_t o = (int64_t)K * W.tile_first[box];
-  const uint32_t base = W.hist_scan[o];
-  // keys beyond the step's grid hold no particle: their lists start at the
-  // end of the box's, as the last key's list ends
-  const int kk = k < K ? k : K - 1;
-  const uint32_t e = W.hist_scan[o + (int64_t)kk * nt + nt - 1] + W.hist[o + (int64_t)kk * nt + nt - 1];
-  const uint32_t s = k < K ? W.hist_scan[o + (int64_t)k * nt] : e;
-  W.lstart[(int64_t)box * W.K_stride + k] = (int)(s - base);
-  W.lcnt[(int64_t)box * W.K_stride + k] = (int)(e - s);
 }
 
 // Stable scatter.  The tile's keys are loaded coalesced and transposed to a
@@ -705,7 +729,7 @@ __global__ void k_par_pairs(BoxDesc *boxes, Arrays A, PW W, double del_t, uint64
                             uint32_t step) {
   const int box = blockIdx.y;
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= W.P_stride) return;
+  if (q >= W.P_stride || W.rc[RC_REGRID] == W.tag) return;
   BoxDesc *B = &boxes[box];
   uint32_t ns = 0;
   int acc = 0;
@@ -774,11 +798,32 @@ __device__ inline int64_t test_pair(const PW &W, int64_t NP, uint32_t t) {
   return W.tpair_ok ? (int64_t)W.tpair[t] : find_pair(W.pair_exc, NP, t);
 }
 
-// the first test of every non-empty pair marks that pair; a max-scan then
-// gives every test its pair
-__global__ void k_mark_pair_starts(PW W, int64_t NP) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < NP && W.pair_n[k] > 0) W.tp_in[W.pair_exc[k]] = (uint32_t)k;
+// The pair of every test of a single-batch step, and the first batch's
+// counts: each wavefront takes 64 pairs, a lane writes the tests of a pair
+// with few, the wavefront together those of one with many.
+constexpr int FEW_TESTS = 8;
+__device__ inline void batch_begin(const PW &W, int n_batch) {
+  W.rc[RC_N] = n_batch;
+  W.rc[RC_E] = 0;
+  W.rc[RC_TAIL] = 0;
+  for (int q = 0; q < 4; ++q) W.rstat[q] = 0ull;
+}
+__global__ void __launch_bounds__(256) k_expand_pairs(PW W, int64_t NP, int table, int n_batch) {
+  const int lane = threadIdx.x & 63;
+  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (k == 0) batch_begin(W, n_batch);
+  if (!table) return;
+  const uint32_t n = k < NP ? W.pair_n[k] : 0u, t0 = k < NP ? W.pair_exc[k] : 0u;
+  if (n <= (uint32_t)FEW_TESTS)
+    for (uint32_t i = 0; i < n; ++i) W.tpair[t0 + i] = (uint32_t)k;
+  uint64_t many = __ballot(n > (uint32_t)FEW_TESTS);
+  while (many) {
+    const int src = __ffsll((long long)many) - 1;
+    many &= many - 1;
+    const uint32_t nn = __shfl(n, src), tt = __shfl(t0, src);
+    const uint32_t kk = (uint32_t)(k - lane + src);
+    for (uint32_t i = lane; i < nn; i += 64) W.tpair[tt + i] = kk;
+  }
 }
 
 __device__ inline void atomic_max_double(double *addr, double v) {
@@ -1035,48 +1080,50 @@ __device__ inline int draw_entry(const PW &W, int64_t base, int64_t L, int key, 
   return drawable_as(W, stv, kp, key) ? p : DRAW_AGAIN;
 }
 
-// reserved arrival entries and a fresh arrival log for every list: lists
-// at most ARR_REACH bins above an occupied one (particles only grow)
-// reserve 2 + n/64, and a list that received arrivals in the previous step
-// (on the same grid) at least twice as many as it received then
-__global__ void k_par_acap(BoxDesc *boxes, PW W) {
-  const int box = blockIdx.y;
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= W.K_stride) return;
+// List starts and counts of every (box, key) from the scanned histogram, then
+// the lists' reserved arrival entries and a fresh arrival log, one workgroup
+// a box: lists at most ARR_REACH bins above an occupied one (particles only
+// grow) reserve 2 + n/64, and a list that received arrivals in the previous
+// step (on the same grid) at least twice as many as it received then.
+__global__ void __launch_bounds__(256) k_par_lists(BoxDesc *boxes, PW W) {
+  if (W.rc[RC_REGRID] == W.tag) return;  // laid out for another grid
+  const int box = blockIdx.x;
+  const int nt = W.tiles_in_box[box];
+  const int K = W.K_hist;
+  const int64_t o = (int64_t)K * W.tile_first[box];
+  const uint32_t base = W.hist_scan[o];
+  int *cnt = W.lcnt + (int64_t)box * W.K_stride;
+  for (int k = threadIdx.x; k < W.K_stride; k += blockDim.x) {
+    // keys beyond the step's grid hold no particle: their lists start at the
+    // end of the box's, as the last key's list ends
+    const int kk = k < K ? k : K - 1;
+    const uint32_t e = W.hist_scan[o + (int64_t)kk * nt + nt - 1] + W.hist[o + (int64_t)kk * nt + nt - 1];
+    const uint32_t s = k < K ? W.hist_scan[o + (int64_t)k * nt] : e;
+    W.lstart[(int64_t)box * W.K_stride + k] = (int)(s - base);
+    cnt[k] = (int)(e - s);
+  }
+  __syncthreads();
   const BoxDesc *B = &boxes[box];
-  const int64_t L = (int64_t)box * W.K_stride + k;
   const int nb = B->n_bin, nc = B->w.n_class;
-  const int prev = (B->regridded || B->rekey) ? 0 : W.arr_n[L];
-  int cap = 0;
-  if (!B->error && nb > 0 && k < nb * nc) {
-    const int b = k % nb + 1;
-    const int *cnt = W.lcnt + (int64_t)box * W.K_stride;
-    bool near = false;
-    for (int c = 1; c <= nc && !near; ++c)
-      for (int bb = max(1, b - ARR_REACH); bb <= b && !near; ++bb) near = cnt[par_key(bb, c, nb)] > 0;
-    if (near) cap = 2 + cnt[k] / 64;
-    if (prev > 0) cap = max(cap, 2 * prev + 2);
-    cap = min(A_MAX, cap);
-  }
-  W.acap[L] = cap;
-  W.arr_n[L] = 0;
-  W.arr_head[L] = -1;
-  if (box == 0 && k == 0) *W.ap_top = 0u;
-}
-
-// arrivals of the step beyond their list's reserved entries (not seen by
-// the list's later pairs)
-__global__ void k_par_arr_over(BoxDesc *boxes, PW W) {
-  const int box = blockIdx.y;
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  int over = 0;
-  if (k < W.K_stride) {
+  const bool fresh = B->regridded || B->rekey;
+  for (int k = threadIdx.x; k < W.K_stride; k += blockDim.x) {
     const int64_t L = (int64_t)box * W.K_stride + k;
-    over = max(0, W.arr_n[L] - W.acap[L]);
+    const int prev = fresh ? 0 : W.arr_n[L];
+    int cap = 0;
+    if (!B->error && nb > 0 && k < nb * nc) {
+      const int b = k % nb + 1;
+      bool near = false;
+      for (int c = 1; c <= nc && !near; ++c)
+        for (int bb = max(1, b - ARR_REACH); bb <= b && !near; ++bb)
+          near = cnt[par_key(bb, c, nb)] > 0;
+      if (near) cap = 2 + cnt[k] / 64;
+      if (prev > 0) cap = max(cap, 2 * prev + 2);
+      cap = min(A_MAX, cap);
+    }
+    W.acap[L] = cap;
+    W.arr_n[L] = 0;
+    W.arr_head[L] = -1;
   }
-  for (int off = 32; off > 0; off >>= 1) over += __shfl_xor(over, off);
-  if ((threadIdx.x & 63) == 0 && over)
-    atomicAdd((unsigned long long *)&boxes[box].n_arr_over, (unsigned long long)over);
 }
 
 // find_rand_pair + maybe_coag_pair (src/coagulation.F90:712-803) for test t
@@ -1337,6 +1384,7 @@ __device__ __forceinline__ void par_test(BoxDesc *boxes, const Arrays &A, const 
   const uint32_t t = pend ? pend[i] : t0 + (uint32_t)i;
   const int64_t NP = (int64_t)n_box * W.P_stride;
   const int64_t k = test_pair(W, NP, t);
+  if (!pend) W.thin[i] = 0;
   if (W.pair_acc[k]) return;  // a target slot: k_par_acc_tests
   W.acc[i] = 0;
   W.tid[i] = t;
@@ -1934,7 +1982,9 @@ k_par_acc_tests(BoxDesc *boxes, Arrays A, PW W, int n_box, int type, uint64_t se
 }
 
 // the largest batch end t1 <= min(T, t0 + T_cap) whose target slots fit the
-// records; out[0] = t1, out[1] = acc_count(t0), out[2] = acc_count(t1)
+// records; out[0] = t1, out[1] = acc_count(t0), out[2] = acc_count(t1),
+// out[3] and [4] the step's tests and target slots, out[5] whether a box got
+// a new grid (then nothing else)
 __device__ inline uint32_t acc_count(const PW &W, int64_t NP, uint32_t T, uint32_t t) {
   if (t >= T) return W.acc_exc[NP];
   int64_t k = test_pair(W, NP, t);
@@ -1944,6 +1994,9 @@ __device__ inline uint32_t acc_count(const PW &W, int64_t NP, uint32_t T, uint32
 __global__ void k_batch_end(PW W, int64_t NP, uint32_t t0, uint32_t t_cap, uint32_t a_cap,
                             uint32_t *out) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  const bool regrid = W.rc[RC_REGRID] == W.tag;
+  out[5] = regrid ? 1u : 0u;
+  if (regrid) return;
   const uint32_t T = W.pair_exc[NP];
   const uint32_t a0 = acc_count(W, NP, T, t0);
   uint32_t lo = t0 + 1, hi = (T - t0 < t_cap) ? T : t0 + t_cap;
@@ -1959,18 +2012,18 @@ __global__ void k_batch_end(PW W, int64_t NP, uint32_t t0, uint32_t t_cap, uint3
   out[4] = W.acc_exc[NP];
 }
 
-// compact accepted tests into the event list (in test order)
-__global__ void k_par_gather(PW W) {
-  const int n = W.rc[RC_N];
-  PAR_FOR(i, n) {
-    if (!W.acc[i]) continue;
-    int e = W.acc_scan[i];
+// compact accepted tests into the event list (in test order), as the scan of
+// their flags places them
+struct GatherEvents {
+  PW W;
+  __device__ void operator()(int64_t i, uint32_t acc, uint32_t e) const {
+    if (!acc) return;
     W.ev_t[e] = W.tid[i];
     W.ev_p1[e] = W.tp1[i];
     W.ev_p2[e] = W.tp2[i];
     W.ev_rec[e] = W.trec[i];
   }
-}
+};
 
 __device__ inline void resolve_event(BoxDesc *boxes, const Arrays &A, const PW &W, int n_box,
                                      uint64_t seed, uint32_t step, int e) {
@@ -1978,6 +2031,14 @@ __device__ inline void resolve_event(BoxDesc *boxes, const Arrays &A, const PW &
   int p1 = W.ev_p1[e], p2 = W.ev_p2[e];
   MergeCtx m = merge_ctx(boxes, W, n_box, t);
   W.ev_box[e] = m.box;
+  // the first event of its box (events are in test order, so box-major)
+  if (e == 0) {
+    W.box_first[m.box] = 0;
+  } else {
+    int64_t q;
+    if (pair_box(W, test_pair(W, (int64_t)n_box * W.P_stride, W.ev_t[e - 1]), &q) != m.box)
+      W.box_first[m.box] = e;
+  }
   const int r = W.ev_rec[e];
   if (r >= 0) {
     // a target event wins when it holds the target and every removed source
@@ -1991,7 +2052,6 @@ __device__ inline void resolve_event(BoxDesc *boxes, const Arrays &A, const PW &
     W.f_id[e] = win ? W.ev[r].ndup : 0;
     W.f_info[e] = win ? W.ev[r].nrm + died : 0;
     W.f_hole[e] = win ? W.ev[r].nrm + died : 0;
-    W.f_lose[e] = win ? 0 : 1;
     return;
   }
   // the decisions say which parents the merge changes (removes); a parent
@@ -2012,21 +2072,12 @@ __device__ inline void resolve_event(BoxDesc *boxes, const Arrays &A, const PW &
   W.f_id[e] = (o & O_NEWID) ? 1 : 0;
   W.f_info[e] = ((o & O_INFO1) ? 1 : 0) + ((o & O_INFO2) ? 1 : 0);
   W.f_hole[e] = ((o & O_RM1) && !(o & O_SLOT1) ? 1 : 0) + ((o & O_RM2) && !(o & O_SLOT2) ? 1 : 0);
-  W.f_lose[e] = win ? 0 : 1;
 }
 
 __global__ void k_par_resolve(BoxDesc *boxes, Arrays A, PW W, int n_box, uint64_t seed,
                               uint32_t step) {
   const int E = W.rc[RC_E];
   PAR_FOR(e, E) resolve_event(boxes, A, W, n_box, seed, step, e);
-}
-
-// first event of every box (events are in test order, so box-major)
-__global__ void k_par_box_first(PW W) {
-  const int E = W.rc[RC_E];
-  PAR_FOR(e, E) {
-    if (e == 0 || W.ev_box[e - 1] != W.ev_box[e]) W.box_first[W.ev_box[e]] = e;
-  }
 }
 
 // A particle's components, all MAX_COMP of them in wide loads that go out
@@ -2779,28 +2830,19 @@ k_par_apply_chains(BoxDesc *boxes, Arrays A, PW W, int rid) {
 }
 
 // per-box totals of a round: appended slots, new ids, records, winners
-__global__ void k_par_box_totals(BoxDesc *boxes, PW W, int n_box) {
-  int box = blockIdx.x * blockDim.x + threadIdx.x;
-  if (box >= n_box) return;
-  const int E = W.rc[RC_E];
-  int first = W.box_first[box];
+__device__ inline void box_totals(BoxDesc *boxes, const PW &W, int E, int box) {
+  const int first = W.box_first[box];
   if (first < 0) return;
-  int last = first;
-  {
-    int lo = first, hi = E - 1;  // last event of the box (ev_box sorted)
-    while (lo < hi) {
-      int mid = (lo + hi + 1) >> 1;
-      if (W.ev_box[mid] == box) lo = mid; else hi = mid - 1;
-    }
-    last = lo;
+  int lo = first, hi = E - 1;  // last event of the box (ev_box sorted)
+  while (lo < hi) {
+    int mid = (lo + hi + 1) >> 1;
+    if (W.ev_box[mid] == box) lo = mid; else hi = mid - 1;
   }
+  const int last = lo;
   BoxDesc *B = &boxes[box];
-  int app = W.s_app[last] + W.f_app[last] - W.s_app[first];
-  int ids = W.s_id[last] + W.f_id[last] - W.s_id[first];
-  int info = W.s_info[last] + W.f_info[last] - W.s_info[first];
-  B->n_part += app;
-  B->next_id += ids;
-  B->n_info += info;
+  B->n_part += W.s_app[last] + W.f_app[last] - W.s_app[first];
+  B->next_id += W.s_id[last] + W.f_id[last] - W.s_id[first];
+  B->n_info += W.s_info[last] + W.f_info[last] - W.s_info[first];
 }
 
 __device__ inline void release_event(const PW &W, int e) {
@@ -2816,11 +2858,6 @@ __device__ inline void release_event(const PW &W, int e) {
     W.slot[W.ev_p2[e]].claim = UNCLAIMED;
     W.slot[W.ev_p2[e]].claim_wr = UNCLAIMED;
   }
-}
-
-__global__ void k_par_release(PW W) {
-  const int E = W.rc[RC_E];
-  PAR_FOR(e, E) release_event(W, e);
 }
 
 // Tests of the round that must be drawn again: accepted tests that lost a
@@ -2894,15 +2931,39 @@ __device__ inline void pending_test(BoxDesc *boxes, const PW &W, int n_box, int 
   W.f_pend[i] = f;
 }
 
-__global__ void k_par_pending(BoxDesc *boxes, PW W, int n_box, int rid) {
-  const int n = W.rc[RC_N];
+// What follows the round's merges, in one launch: the boxes' totals, the
+// claims released, and which tests stay pending (none of which reads what
+// another writes).
+__global__ void k_par_settle(BoxDesc *boxes, PW W, int n_box, int rid) {
+  const int n = W.rc[RC_N], E = W.rc[RC_E];
+  if (n == 0) return;
+  PAR_FOR(b, n_box) box_totals(boxes, W, E, b);
+  PAR_FOR(e, E) release_event(W, e);
   PAR_FOR(i, n) pending_test(boxes, W, n_box, rid, i);
 }
 
-// the running minimum over each box's bins of the next round's minima
-// (one workgroup per box), and this round's cleared for the round after
+// the pending tests in order, with their pairs (which the tail reads)
+struct GatherPending {
+  PW W;
+  int64_t NP;
+  __device__ void operator()(int64_t i, uint32_t f, uint32_t at) const {
+    if (!f) return;
+    const uint32_t t = W.tid[i];
+    W.pend[at] = t;
+    W.pend_k[at] = (int)test_pair(W, NP, t);
+  }
+};
+
+// The end of a device-wide round, one workgroup per box: the running minimum
+// over the box's bins of the next round's minima, this round's cleared for
+// the round after.  And, if the round ran, its holes join the step's count,
+// and its pending tests go to another device-wide round while that settles
+// most of the batch (at most half of it still pending, and not the last
+// round), else to the tail.  A round without events leaves nothing
+// pending: with no winner no test's inputs changed, and a test on an empty
+// arrival entry stays thinned, as no particle arrived.
 constexpr int PREFIX_THREADS = 256;
-__global__ void __launch_bounds__(PREFIX_THREADS) k_minpend_prefix(PW W) {
+__global__ void __launch_bounds__(PREFIX_THREADS) k_round_end(PW W, int n_batch, int round) {
   __shared__ scan_storage<PREFIX_THREADS, uint32_t> tmp;
   __shared__ uint32_t carry;
   const int tid = threadIdx.x;
@@ -2921,35 +2982,15 @@ __global__ void __launch_bounds__(PREFIX_THREADS) k_minpend_prefix(PW W) {
     if (tid == PREFIX_THREADS - 1) carry = r;
     __syncthreads();
   }
-}
-
-__global__ void k_par_gather_pending(PW W) {
-  const int n = W.rc[RC_N];
-  PAR_FOR(i, n) {
-    if (W.f_pend[i]) W.pend[W.s_pend[i]] = W.tid[i];
-  }
-}
-
-// The tests of a batch's first round: all of them.
-__global__ void k_batch_begin(PW W, int n_batch) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    W.rc[RC_N] = n_batch;
-    W.rc[RC_E] = 0;
-    W.rc[RC_TAIL] = 0;
-    for (int q = 0; q < 4; ++q) W.rstat[q] = 0ull;
-  }
-}
-
-// The end of a device-wide round that ran: its holes join the step's count,
-// and its pending tests go to another device-wide round while that settles
-// most of the batch (at most half of it still pending, and not the last
-// round), else to the tail.  A round without events leaves nothing
-// pending: with no winner no test's inputs changed, and a test on an empty
-// arrival entry stays thinned, as no particle arrived.
-__global__ void k_round_end(PW W, int n_batch, int round) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  if (tid != 0) return;
+  W.box_first[blockIdx.x] = -1;
+  if (blockIdx.x != 0) return;
   const int n = W.rc[RC_N];
   if (n == 0) return;  // the round did not run
+  if (W.ev) {
+    *W.rm_top = 0;
+    *W.dup_top = 0;
+  }
   const int E = W.rc[RC_E];
   const int p = E > 0 ? W.s_pend[n] : 0;
   *W.hole_top += (unsigned long long)W.s_hole[E];
@@ -3330,15 +3371,8 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
   }
 }
 
-// the pair of every pending test, found in parallel before the tail
-__global__ void k_pend_pairs(PW W, int64_t NP, const uint32_t *pend) {
-  const int n = W.rc[RC_TAIL];
-  PAR_FOR(i, n) W.pend_k[i] = (int)test_pair(W, NP, pend[i]);
-}
-
-// the largest bin count among the boxes (their pair space for this step);
-// also clears the two entries after that pair space, which the pair scans
-// read as their last input
+// the largest bin count among the boxes (their pair space for this step),
+// to the host
 __global__ void __launch_bounds__(256) k_max_nbin(const BoxDesc *boxes, int n_box, uint32_t *out) {
   __shared__ scan_storage<256, int> tr;
   int m = 1;
@@ -3348,25 +3382,25 @@ __global__ void __launch_bounds__(256) k_max_nbin(const BoxDesc *boxes, int n_bo
   if (threadIdx.x == 0) out[0] = (uint32_t)r;
 }
 
-__global__ void k_clear_pair_ends(PW W, int64_t NP) {
-  if (threadIdx.x == 0) {
-    W.pair_n[NP] = 0;
-    W.pair_accn[NP] = 0;
+// Round state of a batch after the first (k_step_front clears the first's),
+// and the entries after the pair space when its size is new.
+__global__ void k_batch_reset(PW W, int n_box, int64_t NP, int n_batch) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < (int64_t)n_box * W.K_stride) {
+    W.minpend[i] = 0u;
+    W.minpend_next[i] = UNCLAIMED;
   }
+  if (i != 0) return;
+  batch_begin(W, n_batch);
+  *W.tail_rounds = 0ull;
+  if (W.ev) {
+    *W.rm_top = 0;
+    *W.dup_top = 0;
+  }
+  W.pair_n[NP] = 0;
+  W.pair_accn[NP] = 0;
 }
 
-__global__ void k_set_u64(unsigned long long *p, unsigned long long v) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
-}
-
-__global__ void k_fill_int(int *p, int64_t n, int v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-__global__ void k_fill_u32(uint32_t *p, int64_t n, uint32_t v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
 __global__ void k_init_slots(SlotRec *p, int64_t n) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = SlotRec{UNCLAIMED, UNCLAIMED, 0u, 0, 0, 0u, 0, ST_LIVE};
@@ -3375,20 +3409,6 @@ __global__ void k_clear_status(SlotRec *p, int64_t n) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i].st = ST_LIVE;
 }
-__global__ void k_fill_u8(uint8_t *p, int64_t n, uint8_t v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
-__global__ void k_step_begin(BoxDesc *boxes, int n_box) {
-  int box = blockIdx.x * blockDim.x + threadIdx.x;
-  if (box >= n_box) return;
-  BoxDesc *B = &boxes[box];
-  B->step_samp = 0;
-  B->step_coag = 0;
-  B->part_steps += B->n_part;
-}
-
 // Tail-fill compaction over all holes at once.  Per box: the range of its
 // holes in the sorted list and how many lie below the final count.  Then
 // the j-th such head hole receives the j-th live slot of the tail
@@ -3396,13 +3416,12 @@ __global__ void k_step_begin(BoxDesc *boxes, int n_box) {
 // tail's holes below v, found by binary search over those holes.  Sources
 // lie at or above n_final and destinations below it, so the moves run in
 // place.  Live particles of the tail keep their slot order.
-__global__ void k_compact_ranges(BoxDesc *boxes, PW W, int n_box, int n_holes) {
-  const int box = blockIdx.x * blockDim.x + threadIdx.x;
-  if (box >= n_box) return;
+__device__ inline void compact_range(const BoxDesc *boxes, const PW &W, const uint64_t *sorted,
+                                     int box, int n_holes) {
   auto lower = [&](uint64_t key, int lo, int hi) {
     while (lo < hi) {
       const int mid = (lo + hi) >> 1;
-      if (W.holes_sorted[mid] < key) lo = mid + 1; else hi = mid;
+      if (sorted[mid] < key) lo = mid + 1; else hi = mid;
     }
     return lo;
   };
@@ -3412,6 +3431,33 @@ __global__ void k_compact_ranges(BoxDesc *boxes, PW W, int n_box, int n_holes) {
   W.cmp_lo[box] = lo;
   W.cmp_hi[box] = hi;
   W.cmp_head[box] = lower(((uint64_t)box << 32) | (uint64_t)(uint32_t)n_final, lo, hi) - lo;
+}
+
+__global__ void k_compact_ranges(BoxDesc *boxes, PW W, int n_box, int n_holes) {
+  const int box = blockIdx.x * blockDim.x + threadIdx.x;
+  if (box < n_box) compact_range(boxes, W, W.holes_sorted, box, n_holes);
+}
+
+// Few holes are sorted and cut into the boxes' ranges by one workgroup: each
+// thread counts the holes below its own in LDS, n reads a hole, 2 us for 1000
+// of them (the device radix sort and the ranges: 14 + 4 us).  Beyond
+// FEW_HOLES the quadratic count loses.
+constexpr int FEW_HOLES = 2048;
+__global__ void __launch_bounds__(1024) k_compact_few(BoxDesc *boxes, PW W, int n_box,
+                                                      int n_holes) {
+  __shared__ uint64_t s_in[FEW_HOLES], s_out[FEW_HOLES];
+  for (int i = threadIdx.x; i < n_holes; i += 1024) s_in[i] = W.holes[i];
+  __syncthreads();
+  for (int i = threadIdx.x; i < n_holes; i += 1024) {
+    const uint64_t h = s_in[i];
+    int rank = 0;
+    for (int j = 0; j < n_holes; ++j) rank += s_in[j] < h ? 1 : 0;
+    s_out[rank] = h;
+    W.holes_sorted[rank] = h;
+  }
+  __syncthreads();
+  for (int box = threadIdx.x; box < n_box; box += 1024)
+    compact_range(boxes, W, s_out, box, n_holes);
 }
 
 __global__ void k_compact_move(BoxDesc *boxes, Arrays A, PW W, int n_holes) {
@@ -3441,12 +3487,6 @@ __global__ void k_compact_move(BoxDesc *boxes, Arrays A, PW W, int n_holes) {
   W.slot[pt].st = W.slot[pf].st;
 }
 
-__global__ void k_compact_finish(BoxDesc *boxes, PW W, int n_box) {
-  const int box = blockIdx.x * blockDim.x + threadIdx.x;
-  if (box >= n_box) return;
-  boxes[box].n_part -= W.cmp_hi[box] - W.cmp_lo[box];
-}
-
 __global__ void k_par_invalidate(BoxDesc *boxes, int n_box) {
   int box = blockIdx.x * blockDim.x + threadIdx.x;
   if (box >= n_box) return;
@@ -3454,10 +3494,22 @@ __global__ void k_par_invalidate(BoxDesc *boxes, int n_box) {
   boxes[box].terms_kernel = 0;
 }
 
-__global__ void k_par_end(BoxDesc *boxes, int n_box) {
-  int box = blockIdx.x * blockDim.x + threadIdx.x;
-  if (box >= n_box) return;
+// The end of a step, one workgroup a box: the slots the compaction freed, the
+// sort's flags, and the arrivals of the step beyond their list's reserved
+// entries (not seen by the list's later pairs).
+__global__ void __launch_bounds__(256) k_step_end(BoxDesc *boxes, PW W, int compacted) {
+  const int box = blockIdx.x;
   BoxDesc *B = &boxes[box];
+  int over = 0;
+  for (int k = threadIdx.x; k < W.K_stride; k += 256) {
+    const int64_t L = (int64_t)box * W.K_stride + k;
+    over += max(0, W.arr_n[L] - W.acap[L]);
+  }
+  for (int off = 32; off > 0; off >>= 1) over += __shfl_xor(over, off);
+  if ((threadIdx.x & 63) == 0 && over)
+    atomicAdd((unsigned long long *)&B->n_arr_over, (unsigned long long)over);
+  if (threadIdx.x != 0) return;
+  if (compacted) B->n_part -= W.cmp_hi[box] - W.cmp_lo[box];
   B->valid_sort = 1;
   B->xlists_valid = 0;
 }
@@ -3465,9 +3517,12 @@ __global__ void k_par_end(BoxDesc *boxes, int n_box) {
 // ------------------------------------------------------------ host side
 // The reference's tot_n_samp counts each pair's Poisson draw over the
 // members present when the loop reaches it (src/coagulation.F90:627): the
-// batch's thinned tests come off the counts drawn over the bound.
-__global__ void __launch_bounds__(256) k_thin_counts(BoxDesc *boxes, PW W, int64_t NP, uint32_t t0,
-                                                     int n) {
+// batch's thinned tests come off the counts drawn over the bound.  The
+// step's holes, the tail's rounds and the batch's round sizes go to the host.
+__global__ void __launch_bounds__(256) k_batch_finish(BoxDesc *boxes, PW W, int64_t NP,
+                                                      uint32_t t0, int n,
+                                                      unsigned long long *to_host) {
+  if (blockIdx.x == 0 && threadIdx.x < 6) to_host[threadIdx.x] = W.hole_top[threadIdx.x];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   int box = -1;
   int64_t q;
@@ -3515,6 +3570,8 @@ inline int parallel_alloc_records(ParallelWork &W, int n_spec) {
   PCHECK(pmalloc(&d.dup_top, 1));
   PCHECK(pmalloc(&d.rm_buf, RM_CAP));
   PCHECK(pmalloc(&d.rm_top, 1));
+  PCHECK(hipMemset(d.dup_top, 0, sizeof(int)));
+  PCHECK(hipMemset(d.rm_top, 0, sizeof(int)));
   d.acc_cap = (int)c;
   d.pool_cap = (int)pc;
   d.rm_cap = RM_CAP;
@@ -3527,12 +3584,12 @@ inline void parallel_free_arrays(ParallelWork &W) {
                   d.tiles_in_box, d.tile_first, d.hist, d.hist_scan, d.lstart, d.lcnt, d.live,
                   d.pair_n, d.pair_exc, d.acc, d.acc_scan, d.tp1, d.tp2, d.tid, d.pend, d.ev_t,
                   d.ev_p1, d.ev_p2, d.ev_box, d.ev_out, d.f_app, d.f_id, d.f_info, d.f_hole,
-                  d.f_lose, d.f_pend, d.s_pend, d.s_app, d.s_id, d.s_info, d.s_hole,
-                  d.s_lose, d.box_first,
+                  d.f_pend, d.s_pend, d.s_app, d.s_id, d.s_info, d.s_hole,
+                  d.box_first,
                   d.holes, d.holes_sorted, d.cmp_lo, d.cmp_hi, d.cmp_head, d.acc_samp,
                   d.scan_part, W.sort_tmp, d.rc,
-                  d.pair_acc, d.pair_accn, d.acc_exc, d.trec, d.tns, d.ev_rec, d.misc,
-                  d.hole_top, d.pend_k, d.tp_in, d.tpair,
+                  d.pair_acc, d.pair_accn, d.acc_exc, d.trec, d.tns, d.ev_rec,
+                  d.hole_top, d.pend_k, d.tpair,
                   d.acap, d.arr_n, d.arr_head, d.ap_p, d.ap_t, d.ap_dep, d.ap_next, d.ap_top,
                   d.thin, d.minpend, d.minpend_next};
   for (void *p : ptrs)
@@ -3644,7 +3701,6 @@ inline int parallel_layout(ParallelWork &W, const Arrays &A, int n_box,
   PCHECK(pmalloc(&d.pair_accn, W.NP + 1));
   PCHECK(pmalloc(&d.acc_exc, W.NP + 1));
   PCHECK(hipMemset(d.pair_accn, 0, sizeof(uint32_t) * (W.NP + 1)));
-  PCHECK(pmalloc(&d.misc, 8));
   PCHECK(pmalloc(&d.rc, RC_SIZE));
   PCHECK(hipMemset(d.rc, 0, sizeof(int) * RC_SIZE));
   d.pstat = W.pstat;
@@ -3665,7 +3721,6 @@ inline int parallel_layout(ParallelWork &W, const Arrays &A, int n_box,
   PCHECK(pmalloc(&d.ev_out, T));
   PCHECK(pmalloc(&d.trec, T));
   PCHECK(pmalloc(&d.pend_k, T));
-  PCHECK(pmalloc(&d.tp_in, T));
   PCHECK(pmalloc(&d.tpair, T));
   PCHECK(pmalloc(&d.tns, T));
   PCHECK(pmalloc(&d.thin, T));
@@ -3684,8 +3739,8 @@ inline int parallel_layout(ParallelWork &W, const Arrays &A, int n_box,
   PCHECK(pmalloc(&d.ap_next, d.ap_ovf + d.ap_cap));
   PCHECK(pmalloc(&d.ap_top, 1));
   PCHECK(pmalloc(&d.ev_rec, T));
-  int **fl[] = {&d.f_app, &d.f_id, &d.f_info, &d.f_hole, &d.f_lose, &d.f_pend,
-                &d.s_app, &d.s_id, &d.s_info, &d.s_hole, &d.s_lose, &d.s_pend};
+  int **fl[] = {&d.f_app, &d.f_id, &d.f_info, &d.f_hole, &d.f_pend,
+                &d.s_app, &d.s_id, &d.s_info, &d.s_hole, &d.s_pend};
   for (int **f : fl) PCHECK(pmalloc(f, T + 1));
   PCHECK(pmalloc(&d.box_first, n_box));
   int64_t total_cap = 0;
@@ -3720,45 +3775,104 @@ inline int parallel_classes(ParallelWork &W, int n_box, int classes) {
   return 0;
 }
 
-// the whole parallel step; the host reads back the test and event counts
+// the sort of the step's keys into lists, and the pairs' test counts laid out
+// in reference order; d.P_stride and W.NP are set for grids of mb_step bins
+inline void parallel_sort_and_pairs(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n_box,
+                                    hipStream_t st, double del_t, uint64_t seed, uint32_t step) {
+  PW &d = W.d;
+  const dim3 gt(W.n_tiles), bt(TILE_THREADS);
+  // stable counting sort of the keys; the histogram spans the step's grid:
+  // keys are below mb_step * classes
+  d.K_hist = W.mb_step * d.tab_classes;
+  PLAUNCH(W, "k_par_hist", k_par_hist, gt, bt, d.K_hist * sizeof(int), st, d_box, d);
+  const int64_t nh = (int64_t)d.K_hist * W.n_tiles;
+  scan_excl_sum(scan_job(d.hist, d.hist_scan, d.scan_part, nh), nh, st);
+  hipLaunchKernelGGL(k_par_lists, dim3(n_box), dim3(256), 0, st, d_box, d);
+  // the sentinel 2^key_bits - 1 lies above the keys
+  int key_bits = 1;
+  while ((1 << key_bits) <= d.K_hist) key_bits++;
+  PLAUNCH(W, "k_par_scatter", k_par_scatter, gt, bt, 2 * d.K_stride * sizeof(int), st, d_box, d,
+          key_bits);
+  // Poisson test counts per bin pair
+  PLAUNCH(W, "k_par_pairs", k_par_pairs, dim3((unsigned)((d.P_stride + 255) / 256), n_box),
+          dim3(256), 0, st, d_box, A, d, del_t, seed, step);
+  // both in one pass; each writes its total after the pair space
+  ScanJob J = scan_job(d.pair_n, d.pair_exc, d.scan_part, W.NP);
+  J.in[1] = d.pair_accn;
+  J.out[1] = d.acc_exc;
+  J.cols = 2;
+  scan_excl_sum(J, W.NP, st);
+  // the step's test count, its target slots and the first batch's bounds
+  hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, d, W.NP, 0u, (uint32_t)W.T_cap,
+                     (uint32_t)ACC_CAP, W.h_u32 + 4);
+}
+
+// the pair space of grids of up to mb bins
+inline void parallel_pair_space(ParallelWork &W, int n_box, int mb) {
+  W.mb_step = mb;
+  W.d.max_bin = mb;
+  W.d.P_stride = (int64_t)W.d.tab_classes * W.d.tab_classes * mb * mb;
+  W.NP = (int64_t)n_box * W.d.P_stride;
+}
+
+// The whole parallel step.  The host waits twice: for the test counts, which
+// size the claim rounds, and for the hole count, which sizes the compaction.
+// A step that follows another with no call between that changes a box finds
+// keys, terms and tables current: it launches straight through to the test
+// counts on the last step's grids, and starts over from the keys only if a
+// box turns out to need a new grid.  (About 35 dispatches a step; 83 with
+// every pass a launch of its own and the checks for stale state in each
+// step.)
 inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n_box,
                          const std::vector<int64_t> &cap, int max_bin, hipStream_t st, int type,
                          double del_t, uint64_t seed, uint32_t step, int precision, double band,
                          int validation) {
   PW &d = W.d;
+  const int want_terms = (precision != 0) ? 1 : 0;
+  bool clean = W.clean_type == type && W.clean_terms == want_terms;
+  W.clean_type = 0;  // set again at the end of a step that went through
   if (d.key == nullptr || d.K_stride != max_bin * d.tab_classes || W.NP != (int64_t)n_box * d.P_stride) {
     int e = parallel_layout(W, A, n_box, cap, max_bin);
     if (e) return e;
     hipLaunchKernelGGL(k_par_invalidate, dim3((n_box + 63) / 64), dim3(64), 0, st, d_box, n_box);
+    clean = false;
   }
-  const int want_terms = (precision != 0) ? 1 : 0;
   const dim3 gb((n_box + 63) / 64), bb(64);
   const dim3 gt(W.n_tiles), bt(TILE_THREADS);
   d.tpair_ok = 0;  // built once the step's tests are laid out
-  hipLaunchKernelGGL(k_step_begin, gb, bb, 0, st, d_box, n_box);
+  if (++W.tag == INT32_MAX) W.tag = 1;
+  d.tag = W.tag;
   // 1. keys for boxes with a valid grid but stale keys, radius extremes for
   // unsorted boxes, the remake test, and keys again after a new grid
-  hipLaunchKernelGGL(k_par_zero_live, dim3(1, n_box), dim3(256), 0, st, d_box, d, n_box, 0);
-  hipLaunchKernelGGL(k_par_rekey, gt, bt, 0, st, d_box, A, d, type, want_terms, 0);
-  hipLaunchKernelGGL(k_par_finish_rekey, gb, bb, 0, st, d_box, n_box, type, want_terms, 0);
-  hipLaunchKernelGGL(k_par_reset_minmax, gb, bb, 0, st, d_box, n_box);
-  hipLaunchKernelGGL(k_par_minmax, gt, bt, 0, st, d_box, A, d);
-  hipLaunchKernelGGL(k_par_remake, gb, bb, 0, st, d_box, A, d, n_box);
-  hipLaunchKernelGGL(k_par_zero_live, dim3(1, n_box), dim3(256), 0, st, d_box, d, n_box, 1);
-  hipLaunchKernelGGL(k_par_rekey, gt, bt, 0, st, d_box, A, d, type, 0, 1);
-  hipLaunchKernelGGL(k_par_finish_rekey, gb, bb, 0, st, d_box, n_box, type, 0, 1);
-  // The largest grid among the boxes this step: the pair space spans it
-  // (not the allocation's max_bin) and the sort keys need only its bits.
-  hipLaunchKernelGGL(k_max_nbin, dim3(1), dim3(256), 0, st, d_box, n_box, d.misc);
-  PCHECK(hipMemcpyAsync(W.h_u32 + 8, d.misc, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-  PCHECK(hipStreamSynchronize(st));
-  const int mb_step = std::max(1, std::min((int)W.h_u32[8], max_bin));
-  d.max_bin = mb_step;
-  d.P_stride = (int64_t)d.tab_classes * d.tab_classes * mb_step * mb_step;
-  W.NP = (int64_t)n_box * d.P_stride;
-  hipLaunchKernelGGL(k_clear_pair_ends, dim3(1), dim3(64), 0, st, d, W.NP);
-  // 2. majorant and pair tables (shared with the exact mode)
-  {
+  if (!clean) {
+    hipLaunchKernelGGL(k_par_zero_live, dim3(1, n_box), dim3(256), 0, st, d_box, d, n_box, 0);
+    hipLaunchKernelGGL(k_par_rekey, gt, bt, 0, st, d_box, A, d, type, want_terms, 0);
+    hipLaunchKernelGGL(k_par_finish_rekey, gb, bb, 0, st, d_box, n_box, type, want_terms, 0);
+    hipLaunchKernelGGL(k_par_reset_minmax, gb, bb, 0, st, d_box, n_box);
+    hipLaunchKernelGGL(k_par_minmax, gt, bt, 0, st, d_box, A, d);
+  }
+  hipLaunchKernelGGL(k_step_front, dim3(n_box), dim3(64), 0, st, d_box, A, d, clean ? W.NP : 0);
+  if (clean) {
+    // 2.-4. on the last step's grids; W.h_u32[9] tells whether they still hold
+    parallel_sort_and_pairs(W, A, d_box, n_box, st, del_t, seed, step);
+    PCHECK(hipStreamSynchronize(st));
+    clean = W.h_u32[9] == 0;
+  }
+  if (!clean) {
+    if (++W.tag == INT32_MAX) W.tag = 1;
+    d.tag = W.tag;
+    hipLaunchKernelGGL(k_par_zero_live, dim3(1, n_box), dim3(256), 0, st, d_box, d, n_box, 1);
+    hipLaunchKernelGGL(k_par_rekey, gt, bt, 0, st, d_box, A, d, type, 0, 1);
+    hipLaunchKernelGGL(k_par_finish_rekey, gb, bb, 0, st, d_box, n_box, type, 0, 1);
+    // The largest grid among the boxes this step: the pair space spans it
+    // (not the allocation's max_bin) and the sort keys need only its bits.
+    hipLaunchKernelGGL(k_max_nbin, dim3(1), dim3(256), 0, st, d_box, n_box, W.h_u32 + 12);
+    PCHECK(hipStreamSynchronize(st));
+    parallel_pair_space(W, n_box, std::max(1, std::min((int)W.h_u32[12], max_bin)));
+    hipLaunchKernelGGL(k_batch_reset,
+                       dim3((unsigned)(((int64_t)n_box * d.K_stride + 255) / 256)), dim3(256), 0,
+                       st, d, n_box, W.NP, 0);
+    // 2. majorant and pair tables (shared with the exact mode)
     const int mb = max_bin;
     hipLaunchKernelGGL(k_kbounds, dim3((mb * mb + 255) / 256, n_box), dim3(256), 0, st, d_box, A, type);
     hipLaunchKernelGGL(k_mark_bounds, gb, bb, 0, st, d_box, n_box, type);
@@ -3766,52 +3880,12 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
                        dim3((d.tab_classes * d.tab_classes * mb * mb + 255) / 256, n_box), dim3(256),
                        0, st, d_box, A);
     hipLaunchKernelGGL(k_mark_tables, gb, bb, 0, st, d_box, n_box);
+    // 3. and 4.
+    parallel_sort_and_pairs(W, A, d_box, n_box, st, del_t, seed, step);
+    PCHECK(hipStreamSynchronize(st));
   }
-  // 3. stable counting sort of the keys
-  // the histogram spans the step's grid: keys are below mb_step * classes
-  d.K_hist = mb_step * d.tab_classes;
-  PLAUNCH(W, "k_par_hist", k_par_hist, gt, bt, d.K_hist * sizeof(int), st, d_box, d);
-  {
-    const int64_t nh = (int64_t)d.K_hist * W.n_tiles;
-    scan_excl_sum(scan_job(d.hist, d.hist_scan, d.scan_part, nh), nh, st);
-  }
-  hipLaunchKernelGGL(k_par_lists, dim3((d.K_stride + 255) / 256, n_box), dim3(256), 0, st, d_box, d,
-                     n_box);
-  hipLaunchKernelGGL(k_par_acap, dim3((d.K_stride + 255) / 256, n_box), dim3(256), 0, st, d_box, d);
-  // keys are below mb_step * classes; the sentinel 2^key_bits - 1 above them
-  int key_bits = 1;
-  while ((1 << key_bits) <= mb_step * d.tab_classes) key_bits++;
-  PLAUNCH(W, "k_par_scatter", k_par_scatter, gt, bt, 2 * d.K_stride * sizeof(int), st, d_box, d,
-          key_bits);
-  // 4. Poisson test counts per bin pair, laid out in reference order
-  PLAUNCH(W, "k_par_pairs", k_par_pairs, dim3((unsigned)((d.P_stride + 255) / 256), n_box),
-          dim3(256), 0, st, d_box, A, d, del_t, seed, step);
-  {
-    // both in one pass; each writes its total after the pair space
-    ScanJob J = scan_job(d.pair_n, d.pair_exc, d.scan_part, W.NP);
-    J.in[1] = d.pair_accn;
-    J.out[1] = d.acc_exc;
-    J.cols = 2;
-    scan_excl_sum(J, W.NP, st);
-  }
-  // the step's test count, its target slots and the first batch's bounds,
-  // in one read
-  hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, d, W.NP, 0u, (uint32_t)W.T_cap,
-                     (uint32_t)ACC_CAP, d.misc);
-  PCHECK(hipMemcpyAsync(W.h_u32 + 4, d.misc, 5 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-  PCHECK(hipStreamSynchronize(st));
   const uint32_t T = W.h_u32[7];
   const uint32_t T_acc = W.h_u32[8];
-  // the test-to-pair table, when the step is one batch
-  d.tpair_ok = 0;
-  if (T > 0 && (int64_t)T <= W.T_cap) {
-    hipLaunchKernelGGL(k_fill_u32, dim3((T + 255) / 256), dim3(256), 0, st, d.tp_in, (int64_t)T,
-                       0u);
-    hipLaunchKernelGGL(k_mark_pair_starts, dim3((unsigned)((W.NP + 255) / 256)), dim3(256), 0, st,
-                       d, W.NP);
-    scan_incl_max(scan_job(d.tp_in, d.tpair, d.scan_part, (int64_t)T), (int64_t)T, st);
-    d.tpair_ok = 1;
-  }
   if (T_acc > 0 && d.ev == nullptr) {
     int e = parallel_alloc_records(W, A.n_spec);
     if (e) return e;
@@ -3830,36 +3904,33 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
   // Grids are sized from the previous batch's counts, and the kernels stride
   // over any excess.
   int64_t n_holes = 0;
-  hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(64), 0, st, d.hole_top, 0ull);
   for (uint32_t t0 = 0; t0 < T;) {
     uint32_t t1, a0, a1;
-    if (t0 == 0) {
-      t1 = W.h_u32[4];
-      a0 = W.h_u32[5];
-      a1 = W.h_u32[6];
-    } else {
+    const bool first = t0 == 0;
+    if (!first) {
       // the batch ends where its target slots would overflow the records
       hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, d, W.NP, t0, (uint32_t)W.T_cap,
-                         (uint32_t)d.acc_cap, d.misc);
-      PCHECK(hipMemcpyAsync(W.h_u32 + 4, d.misc, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+                         (uint32_t)d.acc_cap, W.h_u32 + 4);
       PCHECK(hipStreamSynchronize(st));
-      t1 = W.h_u32[4];
-      a0 = W.h_u32[5];
-      a1 = W.h_u32[6];
     }
+    t1 = W.h_u32[4];
+    a0 = W.h_u32[5];
+    a1 = W.h_u32[6];
     const int n_acc = (int)(a1 - a0);
     const int n_batch = (int)(t1 - t0);
     const uint32_t batch_t0 = t0;
     t0 = t1;
-    if (n_batch > 0)
-      hipLaunchKernelGGL(k_fill_u8, dim3((n_batch + 255) / 256), dim3(256), 0, st, d.thin,
-                         (int64_t)n_batch, (uint8_t)0);
-    // at the start of the first round every event of the batch is pending
-    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)(((int64_t)n_box * d.K_stride + 255) / 256)),
-                       dim3(256), 0, st, d.minpend, (int64_t)n_box * d.K_stride, 0u);
-    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)(((int64_t)n_box * d.K_stride + 255) / 256)),
-                       dim3(256), 0, st, d.minpend_next, (int64_t)n_box * d.K_stride, UNCLAIMED);
-    hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(64), 0, st, d, n_batch);
+    if (first) {
+      // the batch's counts, and the test-to-pair table when the step is one batch
+      const int table = (int64_t)T <= W.T_cap ? 1 : 0;
+      hipLaunchKernelGGL(k_expand_pairs, dim3(table ? (unsigned)((W.NP + 255) / 256) : 1u),
+                         dim3(256), 0, st, d, W.NP, table, n_batch);
+      d.tpair_ok = table;
+    } else {
+      hipLaunchKernelGGL(k_batch_reset,
+                         dim3((unsigned)(((int64_t)n_box * d.K_stride + 255) / 256)), dim3(256), 0,
+                         st, d, n_box, W.NP, n_batch);
+    }
     const uint32_t *pend = nullptr;
     // a grid for at most `bound` items, `per` a workgroup, sized from the
     // last batch's count with a margin (the kernels stride over any excess)
@@ -3875,11 +3946,7 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
       const unsigned g_n = round == 0 ? (unsigned)((nb + 255) / 256) : grid(nb, W.est[1], 256);
       const unsigned g_e = grid(nb, W.est[round == 0 ? 0 : 2], 256);
       W.rid++;
-      if (n_acc > 0) {
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, d.rm_top, 1, 0);
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, d.dup_top, 1, 0);
-      }
-      // the target walks run on the second stream beside the per-set tests
+      // the target visits run on the second stream beside the per-set tests
       // (disjoint slots; both only claim with atomics)
       if (n_acc > 0) {
         PCHECK(hipEventRecord(W.ev_fork, st));
@@ -3898,59 +3965,44 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
         PLAUNCH(W, "k_par_tests", k_par_tests<true>, dim3(g_n), dim3(256), 0, st, d_box, A, d,
                 n_box, type, seed, step, batch_t0, pend, precision, band, validation);
       if (n_acc > 0) PCHECK(hipStreamWaitEvent(st, W.ev_join, 0));
-      scan_excl_sum(scan_job(d.acc, d.acc_scan, d.scan_part, 0, d.rc + RC_N, d.rc + RC_E), nb, st);
-      hipLaunchKernelGGL(k_par_gather, dim3(g_n), dim3(256), 0, st, d);
-      hipLaunchKernelGGL(k_fill_int, dim3((n_box + 255) / 256), dim3(256), 0, st, d.box_first,
-                         (int64_t)n_box, -1);
+      scan_excl_sum(scan_job(d.acc, d.acc_scan, d.scan_part, 0, d.rc + RC_N, d.rc + RC_E), nb, st,
+                    GatherEvents{d});
       hipLaunchKernelGGL(k_par_resolve, dim3(g_e), dim3(256), 0, st, d_box, A, d, n_box, seed, step);
-      hipLaunchKernelGGL(k_par_box_first, dim3(g_e), dim3(256), 0, st, d);
       {
-        // the winners' ranks: the five flag arrays in one pass
-        const int *fs[5] = {d.f_app, d.f_id, d.f_info, d.f_hole, d.f_lose};
-        int *ss[5] = {d.s_app, d.s_id, d.s_info, d.s_hole, d.s_lose};
+        // the winners' ranks: the flag arrays in one pass
+        const int *fs[4] = {d.f_app, d.f_id, d.f_info, d.f_hole};
+        int *ss[4] = {d.s_app, d.s_id, d.s_info, d.s_hole};
         ScanJob J = scan_job(fs[0], ss[0], d.scan_part, 0, d.rc + RC_E);
-        for (int q = 1; q < 5; ++q) {
+        for (int q = 1; q < 4; ++q) {
           J.in[q] = (const uint32_t *)fs[q];
           J.out[q] = (uint32_t *)ss[q];
         }
-        J.cols = 5;
+        J.cols = 4;
         scan_excl_sum(J, nb, st);
       }
       // one wavefront per event, a few events each: most have no long chain
-      hipLaunchKernelGGL(k_par_apply_chains, dim3(std::min(grid(nb, W.est[round == 0 ? 0 : 2], 16), 4096u)),
-                         dim3(256), 0, st, d_box, A, d, (int)W.rid);
+      if (n_acc > 0)
+        hipLaunchKernelGGL(k_par_apply_chains, dim3(std::min(grid(nb, W.est[round == 0 ? 0 : 2], 16), 4096u)),
+                           dim3(256), 0, st, d_box, A, d, (int)W.rid);
       PLAUNCH(W, "k_par_apply", k_par_apply, dim3(g_e), dim3(256), 0, st, d_box, A, d,
               n_box, seed, step, type, want_terms, (int)W.rid);
-      hipLaunchKernelGGL(k_par_box_totals, gb, bb, 0, st, d_box, d, n_box);
-      hipLaunchKernelGGL(k_par_release, dim3(g_e), dim3(256), 0, st, d);
-      hipLaunchKernelGGL(k_par_pending, dim3(g_n), dim3(256), 0, st, d_box, d, n_box, (int)W.rid);
-      hipLaunchKernelGGL(k_minpend_prefix, dim3(n_box), dim3(PREFIX_THREADS), 0, st, d);
+      hipLaunchKernelGGL(k_par_settle, dim3(g_n), dim3(256), 0, st, d_box, d, n_box, (int)W.rid);
+      scan_excl_sum(scan_job(d.f_pend, d.s_pend, d.scan_part, 0, d.rc + RC_N), nb, st,
+                    GatherPending{d, W.NP});
+      hipLaunchKernelGGL(k_round_end, dim3(n_box), dim3(PREFIX_THREADS), 0, st, d, n_batch, round);
       std::swap(d.minpend, d.minpend_next);
-      scan_excl_sum(scan_job(d.f_pend, d.s_pend, d.scan_part, 0, d.rc + RC_N), nb, st);
-      hipLaunchKernelGGL(k_par_gather_pending, dim3(g_n), dim3(256), 0, st, d);
-      hipLaunchKernelGGL(k_round_end, dim3(1), dim3(64), 0, st, d, n_batch, round);
       // the next round and the tail read the pending tests from d.pend: the
       // tests kernels copy them into tid before the round writes d.pend
       pend = d.pend;
     }
     // the rest per box, one workgroup each
-    if (n_acc > 0) {
-      hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, d.rm_top, 1, 0);
-      hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, d.dup_top, 1, 0);
-    }
-    hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(64), 0, st, d.tail_rounds, 0ull);
-    hipLaunchKernelGGL(k_pend_pairs, dim3(grid(n_batch, W.est[3], 256)), dim3(256), 0, st, d,
-                       W.NP, d.pend);
     PLAUNCH(W, "k_par_tail", k_par_tail, dim3(n_box), dim3(TAIL_THREADS),
             2 * d.K_stride * sizeof(int), st, d_box, A, d,
             n_box, d.pend, type, seed, step, precision, band, del_t, a0,
             want_terms, (int)W.rid + 1, d.tail_rounds, batch_t0);
-    if (n_batch > 0)
-      hipLaunchKernelGGL(k_thin_counts, dim3((n_batch + 255) / 256), dim3(256), 0, st, d_box, d,
-                         W.NP, batch_t0, n_batch);
-    // the holes, the tail's rounds and the batch's round sizes in one read
-    PCHECK(hipMemcpyAsync(W.h_u64, d.hole_top, 6 * sizeof(unsigned long long),
-                          hipMemcpyDeviceToHost, st));
+    // the holes, the tail's rounds and the batch's round sizes, to the host
+    hipLaunchKernelGGL(k_batch_finish, dim3((n_batch + 255) / 256), dim3(256), 0, st, d_box, d,
+                       W.NP, batch_t0, n_batch, W.h_u64);
     PCHECK(hipStreamSynchronize(st));
     n_holes = (int64_t)W.h_u64[0];
     W.n_tail_rounds += (int64_t)W.h_u64[1];
@@ -3959,17 +4011,20 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
   }
   // 6. compaction
   if (n_holes > 0) {
-    PCHECK(rocprim::radix_sort_keys(W.sort_tmp, W.sort_tmp_bytes, d.holes, d.holes_sorted,
-                                    (unsigned)n_holes, 0u, 64u, st));
-    hipLaunchKernelGGL(k_compact_ranges, gb, bb, 0, st, d_box, d, n_box, (int)n_holes);
+    if (n_holes <= FEW_HOLES) {
+      hipLaunchKernelGGL(k_compact_few, dim3(1), dim3(1024), 0, st, d_box, d, n_box, (int)n_holes);
+    } else {
+      PCHECK(rocprim::radix_sort_keys(W.sort_tmp, W.sort_tmp_bytes, d.holes, d.holes_sorted,
+                                      (unsigned)n_holes, 0u, 64u, st));
+      hipLaunchKernelGGL(k_compact_ranges, gb, bb, 0, st, d_box, d, n_box, (int)n_holes);
+    }
     PLAUNCH(W, "k_par_compact", k_compact_move, dim3((unsigned)((n_holes + 255) / 256)), dim3(256),
             0, st, d_box, A, d, (int)n_holes);
-    hipLaunchKernelGGL(k_compact_finish, gb, bb, 0, st, d_box, d, n_box);
   }
-  hipLaunchKernelGGL(k_par_arr_over, dim3((d.K_stride + 255) / 256, n_box), dim3(256), 0, st, d_box,
-                     d);
-  hipLaunchKernelGGL(k_par_end, gb, bb, 0, st, d_box, n_box);
+  hipLaunchKernelGGL(k_step_end, dim3(n_box), dim3(256), 0, st, d_box, d, n_holes > 0 ? 1 : 0);
   PCHECK(hipGetLastError());
+  W.clean_type = type;
+  W.clean_terms = want_terms;
   return 0;
 }
 

@@ -58,10 +58,10 @@ __device__ inline T block_reduce(T v, Op op, scan_storage<BLOCK, T> &st) {
 
 // ------------------------------------------------------- device-wide scans
 // Up to SCAN_COLS arrays of 32-bit elements of one length n are scanned in
-// the same launches (a claim round's five event flags).  Sums wrap modulo
+// the same launches (a claim round's four event flags).  Sums wrap modulo
 // 2^32, so int and uint32_t arrays scan alike.  An exclusive sum also
 // writes its total at out[n] and, when total_dst is set, there.
-constexpr int SCAN_COLS = 5;
+constexpr int SCAN_COLS = 4;
 constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_UNROLL = 4;            // segments of SCAN_THREADS elements loaded together
 constexpr int SCAN_MIN_SEGS = 8;          // segments a workgroup handles at least
@@ -105,8 +105,16 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_chunks(ScanJob J, Op op, 
   }
 }
 
-template <typename Op, bool EXCL>
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(ScanJob J, Op op, uint32_t ident) {
+// What a scan does with each element of its first column besides writing the
+// result (a compaction of flagged items, one launch less than a pass of its
+// own).
+struct ScanOnly {
+  __device__ void operator()(int64_t, uint32_t, uint32_t) const {}
+};
+
+template <typename Op, bool EXCL, typename F>
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(ScanJob J, Op op, uint32_t ident,
+                                                             F each) {
   __shared__ scan_storage<SCAN_THREADS, uint32_t> s;
   const int64_t n = scan_n(J);
   const int g = gridDim.x, b = blockIdx.x;
@@ -141,7 +149,11 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(ScanJob J, Op op, u
         const int64_t i = (sg + u) * SCAN_THREADS + threadIdx.x;
         uint32_t tot;
         const uint32_t r = block_scan_incl<SCAN_THREADS>(v[u], op, s, &tot);
-        if (i < n) out[i] = EXCL ? carry + (r - v[u]) : op(carry, r);
+        if (i < n) {
+          const uint32_t res = EXCL ? carry + (r - v[u]) : op(carry, r);
+          out[i] = res;
+          if (c == 0) each(i, v[u], res);
+        }
         carry = op(carry, tot);
       }
     }
@@ -161,17 +173,12 @@ inline int scan_blocks(int64_t n_bound) {
 }
 
 // exclusive sums (out[0..n]) of J's columns; n at most n_bound
-inline void scan_excl_sum(const ScanJob &J, int64_t n_bound, hipStream_t st) {
+template <typename F = ScanOnly>
+inline void scan_excl_sum(const ScanJob &J, int64_t n_bound, hipStream_t st, F each = F()) {
   const int g = scan_blocks(n_bound);
   if (g > 1) hipLaunchKernelGGL(k_scan_chunks<OpSum>, dim3(g), dim3(SCAN_THREADS), 0, st, J, OpSum(), 0u);
-  hipLaunchKernelGGL((k_scan_apply<OpSum, true>), dim3(g), dim3(SCAN_THREADS), 0, st, J, OpSum(), 0u);
-}
-
-// inclusive running maximum (out[0..n)) of J's columns
-inline void scan_incl_max(const ScanJob &J, int64_t n_bound, hipStream_t st) {
-  const int g = scan_blocks(n_bound);
-  if (g > 1) hipLaunchKernelGGL(k_scan_chunks<OpMax>, dim3(g), dim3(SCAN_THREADS), 0, st, J, OpMax(), 0u);
-  hipLaunchKernelGGL((k_scan_apply<OpMax, false>), dim3(g), dim3(SCAN_THREADS), 0, st, J, OpMax(), 0u);
+  hipLaunchKernelGGL((k_scan_apply<OpSum, true, F>), dim3(g), dim3(SCAN_THREADS), 0, st, J,
+                     OpSum(), 0u, each);
 }
 
 // a job over one array
