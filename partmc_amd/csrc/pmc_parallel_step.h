@@ -914,14 +914,7 @@ __device__ inline void record_arrival(const PW &W, BoxDesc *B, int box, int key,
   W.slot[p].arr_of = (int)e;
   atomicAdd((unsigned long long *)&B->n_arrivals, 1ull);
   if (i < A_MAX) return;
-  int old = __hip_atomic_load(&W.arr_head[L], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  for (;;) {
-    W.ap_next[e] = old;
-    __threadfence();
-    const int prev = atomicCAS(&W.arr_head[L], old, (int)e);
-    if (prev == old) break;
-    old = prev;
-  }
+  W.ap_next[e] = atomicExch(&W.arr_head[L], (int)e);
 }
 
 // visit every arrival entry of list L: the array, then the overflow chain
