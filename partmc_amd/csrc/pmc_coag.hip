@@ -1231,10 +1231,9 @@ static int run_removal(pmc_gpu *h, const std::vector<BoxDesc> &hb, const std::ve
   }
   HIPCHECK(hipMemcpyAsync(R.plan, plan.data(), sizeof(int) * 2 * nb, hipMemcpyHostToDevice,
                           h->stream));
-  const dim3 bb(64), gb((nb + 63) / 64);
   if (any_lists)
-    hipLaunchKernelGGL(k_remove_lists, gb, bb, 0, h->stream, h->d_box, h->A, nb, R.plan + nb, X,
-                       h->seed, h->step);
+    hipLaunchKernelGGL(k_remove_lists, dim3(nb), dim3(LIST_THREADS), 0, h->stream, h->d_box, h->A,
+                       R.plan + nb, X, h->seed, h->step);
   if (any_tiles)
     return run_removal_tiles(h, X, n_max, X.kind == RM_HALVE ? INFO_HALVED : INFO_DILUTION);
   HIPCHECK(hipGetLastError());
