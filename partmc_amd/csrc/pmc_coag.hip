@@ -57,6 +57,7 @@ __constant__ double HALL_ECOLL[315] = {
 #include "pmc_parallel.h"
 #include "pmc_stats.h"
 #include "pmc_rebalance.h"
+#include "pmc_transfer.h"
 
 using namespace pmc;
 
@@ -110,6 +111,13 @@ struct pmc_gpu {
   std::vector<Timed> pending;
   std::vector<std::pair<std::string, std::pair<double, int64_t>>> totals;
   std::vector<double *> tape_buf;  // per box: device values of its tape, or null
+  std::vector<int64_t> off;     // per-box first slot
+  // pinned memory between the host's arrays and the device: a ring for
+  // particles (pmc_transfer.h) and a copy of the descriptors
+  char *stage = nullptr;
+  hipEvent_t stage_done[STAGE_PARTS] = {};  // the kernel that uses a part has ended
+  BoxDesc *box_copy = nullptr;
+  std::mutex stage_lock;
 };
 
 static void timing_begin(pmc_gpu *h, const char *name, hipEvent_t *start) {
@@ -176,6 +184,16 @@ static hipError_t dmalloc(T **p, size_t n) {
   return hipMalloc((void **)p, std::max<size_t>(n, 1) * sizeof(T));
 }
 
+// the descriptors of boxes [first, first + n) once the stream's work is done
+static hipError_t read_boxes(pmc_gpu *h, BoxDesc *dst, int first, int n) {
+  std::lock_guard<std::mutex> lock(h->stage_lock);
+  hipError_t e = hipMemcpyAsync(h->box_copy, h->d_box + first, sizeof(BoxDesc) * n,
+                                hipMemcpyDeviceToHost, h->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  if (e == hipSuccess) memcpy((void *)dst, h->box_copy, sizeof(BoxDesc) * n);
+  return e;
+}
+
 static int alloc_tables(pmc_gpu *h, int classes) {
   Arrays &A = h->A;
   if (A.kw) (void)hipFree(A.kw);
@@ -194,7 +212,7 @@ static int alloc_tables(pmc_gpu *h, int classes) {
 static int layout(pmc_gpu *h, const std::vector<int64_t> &new_cap) {
   h->work.clean_type = 0;
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   Arrays old = h->A;
   int64_t total = 0, pool_total = 0, info_total = 0;
   std::vector<int64_t> off(h->n_box), poff(h->n_box), ioff(h->n_box), phalf(h->n_box);
@@ -290,6 +308,7 @@ static int layout(pmc_gpu *h, const std::vector<int64_t> &new_cap) {
   free_particles(h);
   h->A = A;
   h->cap = new_cap;
+  h->off = off;
   HIPCHECK(hipMemcpy(h->d_box, hb.data(), sizeof(BoxDesc) * h->n_box, hipMemcpyHostToDevice));
   parallel_free_arrays(h->work);  // re-laid out lazily by the next parallel step
   return 0;
@@ -428,6 +447,11 @@ int pmc_gpu_create(pmc_gpu **out, int device, int n_box, int n_spec, const doubl
   HIPCHECK(dmalloc(&h->d_box, n_box));
   HIPCHECK(hipMemcpy(h->d_box, hb.data(), sizeof(BoxDesc) * n_box, hipMemcpyHostToDevice));
   h->cap.assign(n_box, 0);
+  h->off.assign(n_box, 0);
+  HIPCHECK(hipHostMalloc((void **)&h->stage, STAGE_PARTS * STAGE_BYTES));
+  HIPCHECK(hipHostMalloc((void **)&h->box_copy, sizeof(BoxDesc) * n_box));
+  for (hipEvent_t &ev : h->stage_done)
+    HIPCHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   err = parallel_init(h->work, n_box, max_bin);
   if (err) return fail(err, "parallel work allocation failed");
   h->work.tbegin = [](void *c, const char *n, hipEvent_t *e) { timing_begin((pmc_gpu *)c, n, e); };
@@ -452,6 +476,10 @@ int pmc_gpu_destroy(pmc_gpu *h) {
   parallel_free(h->work);
   for (double *t : h->tape_buf)
     if (t) (void)hipFree(t);
+  if (h->stage) (void)hipHostFree(h->stage);
+  if (h->box_copy) (void)hipHostFree(h->box_copy);
+  for (hipEvent_t ev : h->stage_done)
+    if (ev) (void)hipEventDestroy(ev);
   (void)hipStreamDestroy(h->stream);
   delete h;
   return 0;
@@ -463,10 +491,9 @@ int pmc_gpu_set_env(pmc_gpu *h, int box, double temp, double pressure, double ad
   boxes_changed(h);
   Env env = make_env(temp, pressure, additive_coeff);
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
-  if ((e = SET_FIELD(h, box, env, env))) return e;
-  int zero = 0;
-  return SET_FIELD(h, box, terms_kernel, zero);
+  hipLaunchKernelGGL(k_set_env, dim3(1), dim3(64), 0, h->stream, h->d_box + box, env);
+  HIPCHECK(hipGetLastError());
+  return 0;
 }
 
 int pmc_gpu_set_weights(pmc_gpu *h, int box, int n_group, int n_class, const int *type,
@@ -489,24 +516,18 @@ int pmc_gpu_set_weights(pmc_gpu *h, int box, int n_group, int n_class, const int
     w.expo[i] = exponent[i];
   }
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
-  e = SET_FIELD(h, box, w, w);
-  if (e) return e;
-  int zero = 0;
-  e = SET_FIELD(h, box, tables_valid, zero);
-  if (e) return e;
-  // class count changes the key space of the lists
-  if ((e = SET_FIELD(h, box, xlists_valid, zero))) return e;
-  if ((e = SET_FIELD(h, box, pkeys_valid, zero))) return e;
+  hipLaunchKernelGGL(k_set_weights, dim3(1), dim3(64), 0, h->stream, h->d_box + box, w);
+  HIPCHECK(hipGetLastError());
   if (n_class > h->tab_classes) {
+    HIPCHECK(hipStreamSynchronize(h->stream));
     if ((e = alloc_tables(h, n_class))) return e;
     if ((e = parallel_classes(h->work, h->n_box, n_class))) return fail(e, "%s", parallel_last_error());
     std::vector<BoxDesc> hb(h->n_box);
-    HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+    HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
     for (auto &B : hb) B.tables_valid = 0;
     HIPCHECK(hipMemcpy(h->d_box, hb.data(), sizeof(BoxDesc) * h->n_box, hipMemcpyHostToDevice));
   }
-  return SET_FIELD(h, box, valid_sort, zero);
+  return 0;
 }
 
 int pmc_gpu_set_rng(pmc_gpu *h, uint64_t seed, uint32_t step) {
@@ -523,9 +544,10 @@ int pmc_gpu_set_next_id(pmc_gpu *h, int box, int64_t next_id, int64_t id_stride,
   boxes_changed(h);
   if (id_stride < 1) return fail(ERR_ARG, "id_stride must be >= 1");
   HIPCHECK(hipSetDevice(h->device));
-  if ((e = SET_FIELD(h, box, next_id, next_id))) return e;
-  if ((e = SET_FIELD(h, box, id_stride, id_stride))) return e;
-  return SET_FIELD(h, box, id_offset, id_offset);
+  hipLaunchKernelGGL(k_set_next_id, dim3(1), dim3(64), 0, h->stream, h->d_box + box, next_id,
+                     id_stride, id_offset);
+  HIPCHECK(hipGetLastError());
+  return 0;
 }
 
 int pmc_gpu_get_next_id(pmc_gpu *h, int box, int64_t *next_id) {
@@ -537,74 +559,96 @@ int pmc_gpu_get_next_id(pmc_gpu *h, int box, int64_t *next_id) {
   return 0;
 }
 
-__global__ void k_default_components(Arrays A, int64_t base, int n, int set_comp, int set_ct) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int64_t p = base + i;
-  if (set_comp) {
-    A.ncomp[p] = 1;
-    for (int c = 0; c < MAX_COMP; ++c) {
-      A.csrc[comp_at(p, c)] = 0;
-      A.ctime[comp_at(p, c)] = 0.0;
+// Particle records into the slots from base on: volumes particle-major
+// vol[i * n_spec + s] as aero_particle_t%vol, the optional component and
+// create-time arrays defaulted when absent.  Returns once the host's arrays
+// are copied; flag (or null) is a device word to clear on the way.
+static int put_particles(pmc_gpu *h, int64_t base, int n_part, const double *vol,
+                         const int64_t *id, const int *group, const int *klass,
+                         const int *n_primary, const int *n_comp, const int *comp_source,
+                         const double *comp_time, const double *least, const double *greatest,
+                         int *flag) {
+  const int ns = h->n_spec;
+  const bool times = least && greatest;
+  const unsigned fields = REC_VOL | REC_GROUP | REC_KLASS | (id ? REC_ID : 0) |
+                          (n_primary ? REC_NPRIM : 0) |
+                          (n_comp ? REC_NCOMP | REC_CSRC | REC_CTIME : 0) |
+                          (times ? REC_LEAST | REC_GREATEST : 0);
+  const int64_t chunk = (int64_t)(STAGE_BYTES / record_bytes(fields, ns));
+  std::lock_guard<std::mutex> lock(h->stage_lock);
+  for (int64_t i0 = 0, c = 0; i0 < n_part; i0 += chunk, ++c) {
+    const int part = (int)(c % STAGE_PARTS);
+    const size_t m = (size_t)std::min<int64_t>(chunk, n_part - i0);
+    HIPCHECK(hipEventSynchronize(h->stage_done[part]));
+    const Records R = records_at(h->stage + part * STAGE_BYTES, fields, (int64_t)m, ns);
+    memcpy(R.vol, vol + i0 * ns, m * ns * sizeof(double));
+    if (R.id) memcpy(R.id, id + i0, m * sizeof(int64_t));
+    memcpy(R.group, group + i0, m * sizeof(int));
+    memcpy(R.klass, klass + i0, m * sizeof(int));
+    if (R.nprim) memcpy(R.nprim, n_primary + i0, m * sizeof(int));
+    if (R.ncomp) {
+      // the caller's [n_part][MAX_COMP] arrays are the device layout
+      memcpy(R.ncomp, n_comp + i0, m * sizeof(int));
+      memcpy(R.csrc, comp_source + i0 * MAX_COMP, m * MAX_COMP * sizeof(int));
+      memcpy(R.ctime, comp_time + i0 * MAX_COMP, m * MAX_COMP * sizeof(double));
     }
+    if (times) {
+      memcpy(R.least, least + i0, m * sizeof(double));
+      memcpy(R.greatest, greatest + i0, m * sizeof(double));
+    }
+    hipLaunchKernelGGL(k_put_records, dim3((unsigned)((m + XFER_THREADS - 1) / XFER_THREADS)),
+                       dim3(XFER_THREADS), XFER_THREADS * ns * sizeof(double), h->stream, h->A,
+                       base + i0, (int)m, R, i0 == 0 ? flag : nullptr);
+    HIPCHECK(hipGetLastError());
+    HIPCHECK(hipEventRecord(h->stage_done[part], h->stream));
   }
-  if (set_ct) {
-    A.least[p] = 0.0;
-    A.greatest[p] = 0.0;
-  }
+  return 0;
 }
 
-// Particle records n_part .. into the box's slots [first, first + n_part):
-// volumes particle-major vol[i * n_spec + s] as aero_particle_t%vol, the
-// optional component and create-time arrays defaulted when absent.
-static int put_particles(pmc_gpu *h, const BoxDesc &hb, int64_t first, int n_part,
-                         const double *vol, const int64_t *id, const int *group, const int *klass,
-                         const int *n_primary, const int *n_comp, const int *comp_source,
-                         const double *comp_time, const double *least, const double *greatest) {
-  Arrays &A = h->A;
-  const int64_t base = hb.off + first, tc = A.total_cap;
+// The records of n slots from base on into the host's arrays (null: not
+// asked for).
+static int get_particles(pmc_gpu *h, int64_t base, int n, double *vol, int64_t *id, int *group,
+                         int *klass, int *n_primary, int *n_comp, int *comp_source,
+                         double *comp_time, double *least, double *greatest) {
   const int ns = h->n_spec;
-  if (n_part > 0) {
-    std::vector<double> row(n_part);
-    for (int s = 0; s < ns; ++s) {
-      for (int i = 0; i < n_part; ++i) row[i] = vol[(size_t)i * ns + s];
-      HIPCHECK(hipMemcpy(A.vol + s * tc + base, row.data(), n_part * sizeof(double),
-                         hipMemcpyHostToDevice));
-    }
-    for (int i = 0; i < n_part; ++i) {
-      double v = 0.0;
-      for (int s = 0; s < ns; ++s) v += vol[(size_t)i * ns + s];
-      row[i] = v;
-    }
-    HIPCHECK(hipMemcpy(A.vtot + base, row.data(), n_part * sizeof(double), hipMemcpyHostToDevice));
-    if (id) HIPCHECK(hipMemcpy(A.id + base, id, n_part * sizeof(int64_t), hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(A.group + base, group, n_part * sizeof(int), hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(A.klass + base, klass, n_part * sizeof(int), hipMemcpyHostToDevice));
-    if (n_primary) {
-      HIPCHECK(hipMemcpy(A.nprim + base, n_primary, n_part * sizeof(int), hipMemcpyHostToDevice));
-    } else {
-      std::vector<int> ones(n_part, 1);
-      HIPCHECK(hipMemcpy(A.nprim + base, ones.data(), n_part * sizeof(int), hipMemcpyHostToDevice));
-    }
-    if (n_comp) {
-      HIPCHECK(hipMemcpy(A.ncomp + base, n_comp, n_part * sizeof(int), hipMemcpyHostToDevice));
-      // the caller's [n_part][MAX_COMP] arrays are the device layout
-      HIPCHECK(hipMemcpy(A.csrc + comp_at(base, 0), comp_source,
-                         (size_t)n_part * MAX_COMP * sizeof(int), hipMemcpyHostToDevice));
-      HIPCHECK(hipMemcpy(A.ctime + comp_at(base, 0), comp_time,
-                         (size_t)n_part * MAX_COMP * sizeof(double), hipMemcpyHostToDevice));
-    }
-    if (least && greatest) {
-      HIPCHECK(hipMemcpy(A.least + base, least, n_part * sizeof(double), hipMemcpyHostToDevice));
-      HIPCHECK(hipMemcpy(A.greatest + base, greatest, n_part * sizeof(double),
-                         hipMemcpyHostToDevice));
-    }
-    if (!n_comp || !(least && greatest)) {
-      hipLaunchKernelGGL(k_default_components, dim3((n_part + 255) / 256), dim3(256), 0, h->stream,
-                         A, base, n_part, n_comp ? 0 : 1, (least && greatest) ? 0 : 1);
-      HIPCHECK(hipGetLastError());
-      HIPCHECK(hipStreamSynchronize(h->stream));
-    }
+  const unsigned fields = (vol ? REC_VOL : 0) | (id ? REC_ID : 0) | (group ? REC_GROUP : 0) |
+                          (klass ? REC_KLASS : 0) | (n_primary ? REC_NPRIM : 0) |
+                          (n_comp ? REC_NCOMP : 0) | (comp_source ? REC_CSRC : 0) |
+                          (comp_time ? REC_CTIME : 0) | (least ? REC_LEAST : 0) |
+                          (greatest ? REC_GREATEST : 0);
+  if (!fields) return 0;
+  const int64_t chunk = (int64_t)(STAGE_BYTES / record_bytes(fields, ns));
+  const int64_t chunks = (n + chunk - 1) / chunk;
+  std::lock_guard<std::mutex> lock(h->stage_lock);
+  auto records = [&](int64_t c) {
+    return records_at(h->stage + (c % STAGE_PARTS) * STAGE_BYTES, fields,
+                      std::min<int64_t>(chunk, n - c * chunk), ns);
+  };
+  auto enqueue = [&](int64_t c) -> hipError_t {
+    const int m = (int)std::min<int64_t>(chunk, n - c * chunk);
+    hipLaunchKernelGGL(k_get_records, dim3((m + XFER_THREADS - 1) / XFER_THREADS),
+                       dim3(XFER_THREADS), vol ? XFER_THREADS * ns * sizeof(double) : 0, h->stream,
+                       h->A, base + c * chunk, m, records(c));
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : hipEventRecord(h->stage_done[c % STAGE_PARTS], h->stream);
+  };
+  for (int64_t c = 0; c < std::min<int64_t>(chunks, STAGE_PARTS); ++c) HIPCHECK(enqueue(c));
+  for (int64_t c = 0; c < chunks; ++c) {
+    HIPCHECK(hipEventSynchronize(h->stage_done[c % STAGE_PARTS]));
+    const Records R = records(c);
+    const int64_t i0 = c * chunk;
+    const size_t m = (size_t)std::min<int64_t>(chunk, n - i0);
+    if (vol) memcpy(vol + i0 * ns, R.vol, m * ns * sizeof(double));
+    if (id) memcpy(id + i0, R.id, m * sizeof(int64_t));
+    if (group) memcpy(group + i0, R.group, m * sizeof(int));
+    if (klass) memcpy(klass + i0, R.klass, m * sizeof(int));
+    if (n_primary) memcpy(n_primary + i0, R.nprim, m * sizeof(int));
+    if (n_comp) memcpy(n_comp + i0, R.ncomp, m * sizeof(int));
+    if (comp_source) memcpy(comp_source + i0 * MAX_COMP, R.csrc, m * MAX_COMP * sizeof(int));
+    if (comp_time) memcpy(comp_time + i0 * MAX_COMP, R.ctime, m * MAX_COMP * sizeof(double));
+    if (least) memcpy(least + i0, R.least, m * sizeof(double));
+    if (greatest) memcpy(greatest + i0, R.greatest, m * sizeof(double));
+    if (c + STAGE_PARTS < chunks) HIPCHECK(enqueue(c + STAGE_PARTS));
   }
   return 0;
 }
@@ -621,27 +665,19 @@ int pmc_gpu_upload(pmc_gpu *h, int box, int n_part, int capacity, const double *
   if (n_comp && (!comp_source || !comp_time))
     return fail(ERR_ARG, "upload: n_comp given without comp_source/comp_time");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   int64_t want = std::max<int64_t>(capacity, n_part);
   if (want < 16) want = 16;
   if (want > h->cap[box]) {
+    HIPCHECK(hipStreamSynchronize(h->stream));
     std::vector<int64_t> nc = h->cap;
     nc[box] = want;
     if ((e = layout(h, nc))) return e;
   }
-  BoxDesc hb;
-  HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
-  if ((e = put_particles(h, hb, 0, n_part, vol, id, group, klass, n_primary, n_comp, comp_source,
-                         comp_time, least, greatest)))
+  if ((e = put_particles(h, h->off[box], n_part, vol, id, group, klass, n_primary, n_comp,
+                         comp_source, comp_time, least, greatest, nullptr)))
     return e;
-  hb.n_part = n_part;
-  hb.valid_sort = 0;
-  hb.xlists_valid = 0;
-  hb.pkeys_valid = 0;
-  hb.terms_kernel = 0;
-  hb.n_info = 0;
-  hb.error = 0;
-  HIPCHECK(hipMemcpy(h->d_box + box, &hb, sizeof(BoxDesc), hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(k_set_uploaded, dim3(1), dim3(64), 0, h->stream, h->d_box + box, n_part);
+  HIPCHECK(hipGetLastError());
   return 0;
 }
 
@@ -710,15 +746,13 @@ int pmc_gpu_set_bin_grid(pmc_gpu *h, int box, int n_bin, double r_min, double r_
     return fail(711537859, "bin_grid requires 0 < min < max");
   if (h->cap[box] == 0) return fail(ERR_STATE, "set_bin_grid: upload particles first");
   HIPCHECK(hipSetDevice(h->device));
-  if ((e = SET_FIELD(h, box, grid_req_n_bin, n_bin))) return e;
-  if ((e = SET_FIELD(h, box, grid_req_min, r_min))) return e;
-  if ((e = SET_FIELD(h, box, grid_req_max, r_max))) return e;
+  hipLaunchKernelGGL(k_set_grid_req, dim3(1), dim3(64), 0, h->stream, h->d_box + box, n_bin, r_min,
+                     r_max);
   hipLaunchKernelGGL(k_prep_plan, dim3(1), dim3(64), 0, h->stream, h->d_box, h->A, box);
   HIPCHECK(hipGetLastError());
   if ((e = enqueue_prep_keys(h, box))) return e;
   BoxDesc B;
-  HIPCHECK(hipMemcpyAsync(&B, h->d_box + box, sizeof(B), hipMemcpyDeviceToHost, h->stream));
-  HIPCHECK(hipStreamSynchronize(h->stream));
+  HIPCHECK(read_boxes(h, &B, box, 1));
   std::vector<int> plan(h->n_box, 0);
   if (!B.error && B.prep_outside > 0) {
     // particles outside the grid leave in the reference's swap-last order,
@@ -733,9 +767,8 @@ int pmc_gpu_set_bin_grid(pmc_gpu *h, int box, int n_bin, double r_min, double r_
     if ((e = enqueue_prep_keys(h, box))) return e;
   }
   if ((e = enqueue_prep_lists(h, box))) return e;
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   return check_box_errors(h, hb);
 }
 
@@ -755,50 +788,14 @@ int pmc_gpu_download(pmc_gpu *h, int box, int max_part, int *n_part, double *vol
   int e = check_box(h, box);
   if (e) return e;
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   BoxDesc hb;
-  HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, &hb, box, 1));
   if (n_part) *n_part = hb.n_part;
   int n = hb.n_part;
   if (n > max_part) return fail(ERR_CAPACITY, "download: box holds %d particles, room for %d", n, max_part);
   if (n == 0) return 0;
-  const Arrays &A = h->A;
-  const int64_t base = hb.off, tc = A.total_cap;
-  const int ns = h->n_spec;
-  if (vol) {
-    std::vector<double> row(n);
-    for (int s = 0; s < ns; ++s) {
-      HIPCHECK(hipMemcpy(row.data(), A.vol + s * tc + base, n * sizeof(double), hipMemcpyDeviceToHost));
-      for (int i = 0; i < n; ++i) vol[(size_t)i * ns + s] = row[i];
-    }
-  }
-  if (id) HIPCHECK(hipMemcpy(id, A.id + base, n * sizeof(int64_t), hipMemcpyDeviceToHost));
-  if (group) HIPCHECK(hipMemcpy(group, A.group + base, n * sizeof(int), hipMemcpyDeviceToHost));
-  if (klass) HIPCHECK(hipMemcpy(klass, A.klass + base, n * sizeof(int), hipMemcpyDeviceToHost));
-  if (n_primary) HIPCHECK(hipMemcpy(n_primary, A.nprim + base, n * sizeof(int), hipMemcpyDeviceToHost));
-  if (n_comp) HIPCHECK(hipMemcpy(n_comp, A.ncomp + base, n * sizeof(int), hipMemcpyDeviceToHost));
-  if (comp_source || comp_time) {
-    // the device keeps only the first n_comp entries of a particle; the
-    // rest read as zero
-    std::vector<int> nco(n);
-    HIPCHECK(hipMemcpy(nco.data(), A.ncomp + base, n * sizeof(int), hipMemcpyDeviceToHost));
-    // the device layout is the caller's [n][MAX_COMP]
-    if (comp_source) {
-      HIPCHECK(hipMemcpy(comp_source, A.csrc + comp_at(base, 0), (size_t)n * MAX_COMP * sizeof(int),
-                         hipMemcpyDeviceToHost));
-      for (int64_t i = 0; i < n; ++i)
-        for (int c = nco[i] > 0 ? nco[i] : 0; c < MAX_COMP; ++c) comp_source[(size_t)i * MAX_COMP + c] = 0;
-    }
-    if (comp_time) {
-      HIPCHECK(hipMemcpy(comp_time, A.ctime + comp_at(base, 0), (size_t)n * MAX_COMP * sizeof(double),
-                         hipMemcpyDeviceToHost));
-      for (int64_t i = 0; i < n; ++i)
-        for (int c = nco[i] > 0 ? nco[i] : 0; c < MAX_COMP; ++c) comp_time[(size_t)i * MAX_COMP + c] = 0.0;
-    }
-  }
-  if (least) HIPCHECK(hipMemcpy(least, A.least + base, n * sizeof(double), hipMemcpyDeviceToHost));
-  if (greatest) HIPCHECK(hipMemcpy(greatest, A.greatest + base, n * sizeof(double), hipMemcpyDeviceToHost));
-  return 0;
+  return get_particles(h, hb.off, n, vol, id, group, klass, n_primary, n_comp, comp_source,
+                       comp_time, least, greatest);
 }
 
 int pmc_gpu_set_mode(pmc_gpu *h, int mode, int precision, double band) {
@@ -885,9 +882,8 @@ int pmc_gpu_mc_coag_async(pmc_gpu *h, int kernel_type, double del_t) {
 int pmc_gpu_sync(pmc_gpu *h) {
   if (!h) return fail(ERR_ARG, "null handle");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   return check_box_errors(h, hb);
 }
 
@@ -895,9 +891,8 @@ int pmc_gpu_mc_coag(pmc_gpu *h, int kernel_type, double del_t, int64_t *tot_n_sa
                     int64_t *tot_n_coag) {
   int e = pmc_gpu_mc_coag_async(h, kernel_type, del_t);
   if (e) return e;
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   for (int b = 0; b < h->n_box; ++b) {
     if (tot_n_samp) tot_n_samp[b] = hb[b].step_samp;
     if (tot_n_coag) tot_n_coag[b] = hb[b].step_coag;
@@ -909,9 +904,8 @@ int pmc_gpu_get_counters(pmc_gpu *h, int64_t *n_samp, int64_t *n_coag, int64_t *
                          int64_t *n_recheck, int64_t *n_flip, double *max_rel_err) {
   if (!h) return fail(ERR_ARG, "null handle");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   for (int b = 0; b < h->n_box; ++b) {
     if (n_samp) n_samp[b] = hb[b].n_samp;
     if (n_coag) n_coag[b] = hb[b].n_coag;
@@ -926,9 +920,8 @@ int pmc_gpu_get_counters(pmc_gpu *h, int64_t *n_samp, int64_t *n_coag, int64_t *
 int pmc_gpu_reset_counters(pmc_gpu *h) {
   if (!h) return fail(ERR_ARG, "null handle");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   for (auto &B : hb) {
     B.n_samp = B.n_coag = B.n_warn = B.n_recheck = B.n_flip = 0;
     B.max_rel_err = 0.0;
@@ -950,9 +943,8 @@ int pmc_gpu_reset_counters(pmc_gpu *h) {
 int pmc_gpu_get_error_stats(pmc_gpu *h, double *max_p_err) {
   if (!h || !max_p_err) return fail(ERR_ARG, "get_error_stats: bad arguments");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   for (int b = 0; b < h->n_box; ++b) max_p_err[b] = hb[b].max_p_err;
   return 0;
 }
@@ -962,9 +954,8 @@ int pmc_gpu_get_path_stats(pmc_gpu *h, int64_t *n_accel_pairs, int64_t *n_droppe
   if (!h || !n_accel_pairs || !n_dropped || !rounds)
     return fail(ERR_ARG, "get_path_stats: bad arguments");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   for (int b = 0; b < h->n_box; ++b) {
     n_accel_pairs[b] = hb[b].n_accel_pairs;
     n_dropped[b] = hb[b].n_dropped;
@@ -1055,7 +1046,7 @@ int pmc_gpu_get_step_lists(pmc_gpu *h, int box, int *counts) {
   const PW &d = h->work.d;
   if (d.lcnt == nullptr) return fail(ERR_STATE, "get_step_lists: no parallel-mode step has run");
   BoxDesc hb;
-  HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, &hb, box, 1));
   const int K = hb.n_bin * hb.w.n_class;
   if (K <= 0) return 0;
   if (K > d.K_stride) return fail(ERR_STATE, "get_step_lists: lists not laid out for this grid");
@@ -1068,9 +1059,8 @@ int pmc_gpu_get_step_lists(pmc_gpu *h, int box, int *counts) {
 int pmc_gpu_get_arrival_stats(pmc_gpu *h, int64_t *n_arrivals, int64_t *n_overflow) {
   if (!h || !n_arrivals || !n_overflow) return fail(ERR_ARG, "get_arrival_stats: bad arguments");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   for (int b = 0; b < h->n_box; ++b) {
     n_arrivals[b] = hb[b].n_arrivals;
     n_overflow[b] = hb[b].n_arr_over;
@@ -1081,9 +1071,8 @@ int pmc_gpu_get_arrival_stats(pmc_gpu *h, int64_t *n_arrivals, int64_t *n_overfl
 int pmc_gpu_get_accel_counts(pmc_gpu *h, int64_t *n_samp, int64_t *n_coag) {
   if (!h || !n_samp || !n_coag) return fail(ERR_ARG, "get_accel_counts: bad arguments");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   for (int b = 0; b < h->n_box; ++b) {
     n_samp[b] = hb[b].n_acc_samp;
     n_coag[b] = hb[b].n_acc_coag;
@@ -1259,7 +1248,7 @@ int pmc_gpu_rebalance(pmc_gpu *h, int allow_doubling, int allow_halving) {
   RebalWork &R = h->rw;
   const int nb = h->n_box, stride = GC_KEYS + 1;
   std::vector<BoxDesc> hb(nb);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * nb, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   e = check_box_errors(h, hb);
   if (e) return e;
   std::vector<int> gc((size_t)nb * stride), plan(2 * nb);
@@ -1373,7 +1362,7 @@ int pmc_gpu_rebalance(pmc_gpu *h, int allow_doubling, int allow_halving) {
             return fail(ERR_STATE, "rebalance: class (%d, %d) still above twice its ideal after 64 halvings", g, c);
           if (!fresh) {
             // doubling passes may have dropped the sort: flags as they are now
-            HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * nb, hipMemcpyDeviceToHost));
+            HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
             fresh = true;
           }
           Removal X{};
@@ -1385,8 +1374,7 @@ int pmc_gpu_rebalance(pmc_gpu *h, int allow_doubling, int allow_halving) {
           HIPCHECK(count());
         }
   }
-  HIPCHECK(hipStreamSynchronize(h->stream));
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * nb, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   return check_box_errors(h, hb);
 }
 
@@ -1400,7 +1388,7 @@ static int removal_all(pmc_gpu *h, Removal X, const double *per_box) {
   if (e) return e;
   const int nb = h->n_box;
   std::vector<BoxDesc> hb(nb);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * nb, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   if ((e = check_box_errors(h, hb))) return e;
   if (per_box) {
     HIPCHECK(hipMemcpyAsync(h->rw.bval, per_box, sizeof(double) * nb, hipMemcpyHostToDevice,
@@ -1415,8 +1403,7 @@ static int removal_all(pmc_gpu *h, Removal X, const double *per_box) {
     n_max = std::max<int64_t>(n_max, hb[b].n_part);
   }
   if ((e = run_removal(h, hb, want, X, n_max))) return e;
-  HIPCHECK(hipStreamSynchronize(h->stream));
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * nb, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   return check_box_errors(h, hb);
 }
 
@@ -1463,12 +1450,11 @@ int pmc_gpu_append(pmc_gpu *h, int box, int n, const double *vol, const int64_t 
     return fail(ERR_ARG, "append: n_comp given without comp_source/comp_time");
   if (n == 0) return 0;
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   BoxDesc hb;
-  HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, &hb, box, 1));
   if (hb.error) {
     std::vector<BoxDesc> all(h->n_box);
-    HIPCHECK(hipMemcpy(all.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+    HIPCHECK(read_boxes(h, all.data(), 0, h->n_box));
     return check_box_errors(h, all);
   }
   for (int i = 0; i < n; ++i)
@@ -1480,26 +1466,24 @@ int pmc_gpu_append(pmc_gpu *h, int box, int n, const double *vol, const int64_t 
     std::vector<int64_t> nc = h->cap;
     nc[box] = std::max<int64_t>(2 * h->cap[box], (int64_t)first + n);
     if ((e = layout(h, nc))) return e;
-    HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
+    HIPCHECK(read_boxes(h, &hb, box, 1));
   }
-  if ((e = put_particles(h, hb, first, n, vol, id, group, klass, n_primary, n_comp, comp_source,
-                         comp_time, least, greatest)))
-    return e;
   if ((e = rebal_ensure(h, false))) return e;
+  if ((e = put_particles(h, hb.off + first, n, vol, id, group, klass, n_primary, n_comp,
+                         comp_source, comp_time, least, greatest, h->rw.box_tot)))
+    return e;
   if (!id)
     hipLaunchKernelGGL(k_assign_ids, dim3((n + 255) / 256), dim3(256), 0, h->stream, h->d_box,
                        h->A, box, first, n);
-  HIPCHECK(hipMemsetAsync(h->rw.box_tot, 0, sizeof(int), h->stream));
   hipLaunchKernelGGL(k_append_check, dim3((n + 255) / 256), dim3(256), 0, h->stream, h->d_box,
                      h->A, box, first, n, h->rw.box_tot);
   hipLaunchKernelGGL(k_append_finish, dim3(1), dim3(64), 0, h->stream, h->d_box, h->A, box, first,
                      n, h->rw.box_tot, id ? 0 : n);
   HIPCHECK(hipGetLastError());
-  HIPCHECK(hipStreamSynchronize(h->stream));
-  HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, &hb, box, 1));
   if (hb.error) {
     std::vector<BoxDesc> all(h->n_box);
-    HIPCHECK(hipMemcpy(all.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+    HIPCHECK(read_boxes(h, all.data(), 0, h->n_box));
     return check_box_errors(h, all);
   }
   return 0;
@@ -1511,22 +1495,16 @@ int pmc_gpu_scale_weights(pmc_gpu *h, int box, double factor) {
   boxes_changed(h);
   if (!(factor > 0.0)) return fail(ERR_ARG, "scale_weights: factor must be > 0");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
-  Weights w;
-  HIPCHECK(hipMemcpy(&w, (char *)(h->d_box + box) + offsetof(BoxDesc, w), sizeof(Weights),
-                     hipMemcpyDeviceToHost));
-  for (int i = 0; i < w.n_group * w.n_class; ++i) w.mag[i] *= factor;
-  if ((e = SET_FIELD(h, box, w, w))) return e;
-  int zero = 0;
-  return SET_FIELD(h, box, tables_valid, zero);
+  hipLaunchKernelGGL(k_scale_weights, dim3(1), dim3(64), 0, h->stream, h->d_box + box, factor);
+  HIPCHECK(hipGetLastError());
+  return 0;
 }
 
 int pmc_gpu_get_part_steps(pmc_gpu *h, int64_t *part_steps) {
   if (!h || !part_steps) return fail(ERR_ARG, "get_part_steps: bad arguments");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(hipMemcpy(hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box, hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
   for (int b = 0; b < h->n_box; ++b) part_steps[b] = hb[b].part_steps;
   return 0;
 }
@@ -1578,9 +1556,8 @@ int pmc_gpu_get_grid(pmc_gpu *h, int box, int *n_bin, double *edges, double *cen
   int e = check_box(h, box);
   if (e) return e;
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   BoxDesc hb;
-  HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, &hb, box, 1));
   if (n_bin) *n_bin = hb.n_bin;
   int nb = hb.n_bin;
   if (nb <= 0) return 0;
@@ -1594,9 +1571,8 @@ int pmc_gpu_get_lists(pmc_gpu *h, int box, int *counts, int *entries) {
   int e = check_box(h, box);
   if (e) return e;
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   BoxDesc hb;
-  HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, &hb, box, 1));
   int K = hb.n_bin * hb.w.n_class;
   if (K <= 0) return 0;
   std::vector<int> st(K), ln(K);
@@ -1618,9 +1594,8 @@ int pmc_gpu_get_kbounds(pmc_gpu *h, int box, double *kmin, double *kmax) {
   int e = check_box(h, box);
   if (e) return e;
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   BoxDesc hb;
-  HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, &hb, box, 1));
   size_t nn = (size_t)hb.n_bin * hb.n_bin;
   size_t o = (size_t)box * h->max_bin * h->max_bin;
   if (kmin) HIPCHECK(hipMemcpy(kmin, h->A.kmin + o, nn * sizeof(double), hipMemcpyDeviceToHost));
@@ -1633,17 +1608,32 @@ int pmc_gpu_get_removed(pmc_gpu *h, int box, int max_n, int *n, int64_t *id, int
   int e = check_box(h, box);
   if (e) return e;
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   BoxDesc hb;
-  HIPCHECK(hipMemcpy(&hb, h->d_box + box, sizeof(BoxDesc), hipMemcpyDeviceToHost));
+  HIPCHECK(read_boxes(h, &hb, box, 1));
   int64_t cnt = std::min<int64_t>(hb.n_info, hb.info_cap);
   if (n) *n = (int)hb.n_info;
   if (hb.n_info > hb.info_cap) return fail(ERR_CAPACITY, "removal log overflow (%lld records)", (long long)hb.n_info);
   if (cnt > max_n) return fail(ERR_CAPACITY, "removal log holds %lld records, room for %d", (long long)cnt, max_n);
   if (cnt == 0) return 0;
-  if (id) HIPCHECK(hipMemcpy(id, h->A.info_id + hb.info_off, cnt * sizeof(int64_t), hipMemcpyDeviceToHost));
-  if (action) HIPCHECK(hipMemcpy(action, h->A.info_action + hb.info_off, cnt * sizeof(int), hipMemcpyDeviceToHost));
-  if (other_id) HIPCHECK(hipMemcpy(other_id, h->A.info_other + hb.info_off, cnt * sizeof(int64_t), hipMemcpyDeviceToHost));
+  // through the pinned ring, all of it at a time
+  std::lock_guard<std::mutex> lock(h->stage_lock);
+  const int64_t chunk = (int64_t)(STAGE_PARTS * STAGE_BYTES / (2 * sizeof(int64_t) + sizeof(int)));
+  int64_t *s_id = (int64_t *)h->stage, *s_other = s_id + chunk;
+  int *s_action = (int *)(s_other + chunk);
+  for (int64_t i0 = 0; i0 < cnt; i0 += chunk) {
+    const size_t m = (size_t)std::min<int64_t>(chunk, cnt - i0);
+    const int64_t o = hb.info_off + i0;
+    auto get = [&](void *dst, const void *src, size_t bytes) {
+      return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream);
+    };
+    if (id) HIPCHECK(get(s_id, h->A.info_id + o, m * sizeof(int64_t)));
+    if (action) HIPCHECK(get(s_action, h->A.info_action + o, m * sizeof(int)));
+    if (other_id) HIPCHECK(get(s_other, h->A.info_other + o, m * sizeof(int64_t)));
+    HIPCHECK(hipStreamSynchronize(h->stream));
+    if (id) memcpy(id + i0, s_id, m * sizeof(int64_t));
+    if (action) memcpy(action + i0, s_action, m * sizeof(int));
+    if (other_id) memcpy(other_id + i0, s_other, m * sizeof(int64_t));
+  }
   return 0;
 }
 
