@@ -2457,7 +2457,7 @@ __device__ inline MergeParents load_parents(const Arrays &A, const PW &W, int64_
 __device__ inline int direct_merge(const Arrays &A, const PW &W, BoxDesc *B, int box, uint32_t t,
                                    int64_t p1, int64_t p2, int64_t dst, bool appended, int64_t id,
                                    int group, int klass, int type, int want_terms, Stream *rs,
-                                   const MergeParents &P, bool resampled, int *key) {
+                                   const MergeParents &P, bool in_place, int *key) {
   const int64_t tc = A.total_cap;
   const int n1 = P.n1, n2 = P.n2;
   *key = 0;
@@ -2469,7 +2469,7 @@ __device__ inline int direct_merge(const Arrays &A, const PW &W, BoxDesc *B, int
   const bool all = n1 + n2 <= MAX_COMP;
   int s1[MAX_COMP], s2[MAX_COMP];
   double t1[MAX_COMP], t2[MAX_COMP];
-  if (all) {
+  if (all && !in_place) {
     load_comps(A, p2, s2, t2);
     if (dst != p1) load_comps(A, p1, s1, t1);
   }
@@ -2505,7 +2505,9 @@ __device__ inline int direct_merge(const Arrays &A, const PW &W, BoxDesc *B, int
   }
   const int nb = B->n_bin;
   const int b = bin_find_log(nb, B->log_lo, B->log_hi, vol2rad(v));
-  if (all) {
+  if (in_place) {
+    // the components are in place
+  } else if (all) {
     if (dst != p1) {
 #pragma unroll
       for (int c = 0; c < MAX_COMP; ++c)
@@ -2520,7 +2522,7 @@ __device__ inline int direct_merge(const Arrays &A, const PW &W, BoxDesc *B, int
         A.csrc[comp_at(dst, n1 + c)] = s2[c];
         A.ctime[comp_at(dst, n1 + c)] = t2[c];
       }
-  } else if (!resampled) {
+  } else {
     resample_components(A, *rs, p1, p2, dst, n1, n2, P.np1, P.np2);
   }
   A.vtot[dst] = v;
@@ -2551,13 +2553,13 @@ __device__ inline int direct_merge(const Arrays &A, const PW &W, BoxDesc *B, int
 // particle's group and class from bits 16 and 24 on: removals become
 // holes (or the slot the merged particle takes), the merged particle is
 // written, removal records follow the reference's order.  post: the merge
-// stream after the decisions, or null to find it again.  resampled: the
+// stream after the decisions, or null to find it again.  in_place: the
 // merged particle's components are in its slot already.
 template <class Alloc>
 __device__ inline void perset_merge(BoxDesc *B, const Arrays &A, const PW &W, int box, int n_box,
                                     uint32_t t, int64_t p1, int64_t p2, uint64_t seed,
                                     uint32_t step, int type, int want_terms, int rid, Alloc &al,
-                                    int o_group, const Stream *post, bool resampled,
+                                    int o_group, const Stream *post, bool in_place,
                                     const MergeParents &P) {
   al.count(0, 1, 0);
   const int cc = o_group >> 24;
@@ -2566,7 +2568,7 @@ __device__ inline void perset_merge(BoxDesc *B, const Arrays &A, const PW &W, in
   Stream s;
   if (post) {
     s = *post;
-  } else if (P.n1 + P.n2 > MAX_COMP && !resampled) {
+  } else if (P.n1 + P.n2 > MAX_COMP && !in_place) {
     const int64_t k = test_pair(W, (int64_t)n_box * W.P_stride, t);
     int c1, c2, b1, b2;
     decode_pair(k - (int64_t)box * W.P_stride, W.tab_classes, W.max_bin, &c1, &c2, &b1, &b2);
@@ -2591,7 +2593,7 @@ __device__ inline void perset_merge(BoxDesc *B, const Arrays &A, const PW &W, in
     }
     const bool appended = !(o & (O_SLOT1 | O_SLOT2));
     const int err = direct_merge(A, W, B, box, t, p1, p2, slot, appended, nid, new_group, cc, type,
-                                 want_terms, &s, P, resampled, &key);
+                                 want_terms, &s, P, in_place, &key);
     if (err) atomicExch(&B->error, err);
   }
   if (o & O_RM1) {
@@ -2619,17 +2621,23 @@ __device__ inline void perset_merge(BoxDesc *B, const Arrays &A, const PW &W, in
   if (o & O_INFO2) put_info(A, B, al, P.id2, 2, info_other);
 }
 
-// The resamplings among a wavefront's winning per-set merges, done together
-// while they are few: each takes the wavefront about 2 us, where all of them
-// side by side, a lane each, take 13.  win: this lane merges p1 and p2 with
-// decisions o into an existing slot or the append_rank-th new one; ms: its
-// merge stream after the decisions.  Returns whether this lane's components
-// are done.  Every lane of the wavefront takes part.
+// The components of a wavefront's winning per-set merges, by its lanes
+// together while the merges are few.  Resamplings: each takes the wavefront
+// about 2 us, where all of them side by side, a lane each, take 13.  The rest
+// join their parents' components, three merges at once with a lane a
+// component: one round trip, where a lane's own 40 conditional stores wait
+// for its loads (six boxes of 3e5 drops 43.0 -> 41.7 ms, a scenario
+// 16.7 -> 16.3); beyond JOIN_MOST, four such passes, the lanes side by side
+// do as well.  win: this lane merges p1 and p2 with decisions o into an
+// existing slot or the append_rank-th new one; ms: its merge stream after the
+// decisions.  Returns whether this lane's components are done.  Every lane of
+// the wavefront takes part.
 constexpr int RESAMPLE_MOST = 6;
-__device__ inline bool wave_resamplings(const Arrays &A, const BoxDesc *B, bool win, int o,
+constexpr int JOIN_AT_ONCE = 64 / MAX_COMP, JOIN_MOST = 12;
+__device__ inline bool wave_components(const Arrays &A, const BoxDesc *B, bool win, int o,
                                         int64_t p1, int64_t p2, int64_t append_rank,
                                         const Stream &ms, const MergeParents &P) {
-  bool mine = false;
+  bool mine = false, join = false;
   int64_t dst = 0;
   int n1 = 0, n2 = 0, np1 = 0, np2 = 0;
   if (win && (o & O_NEW)) {
@@ -2637,16 +2645,53 @@ __device__ inline bool wave_resamplings(const Arrays &A, const BoxDesc *B, bool 
     n2 = P.n2;
     np1 = P.np1;
     np2 = P.np2;
-    mine = n1 + n2 > MAX_COMP && np1 >= n1 && np2 >= n2;
-    if (mine) {
+    bool ok = np1 >= n1 && np2 >= n2;
+    if (ok) {
       if (o & O_SLOT1) dst = p1;
       else if (o & O_SLOT2) dst = p2;
       else if (B->n_part + append_rank < B->cap) dst = B->off + B->n_part + append_rank;
-      else mine = false;  // the merge fails
+      else ok = false;  // the merge fails
     }
+    mine = ok && n1 + n2 > MAX_COMP;
+    join = ok && !mine;
+  }
+  // components that only join, JOIN_AT_ONCE merges in a pass of the lanes
+  uint64_t cat = __ballot(join);
+  if (__popcll(cat) > JOIN_MOST) {
+    cat = 0;
+    join = false;
+  }
+  const int lane = threadIdx.x & 63, slice = lane / MAX_COMP, c = lane % MAX_COMP;
+  while (cat) {
+    uint64_t m = cat;
+    for (int q = 0; q < slice; ++q) m &= m - 1;
+    const bool on = slice < JOIN_AT_ONCE && m != 0;
+    const int src = on ? __ffsll((long long)m) - 1 : lane;
+    const int a = __shfl((int)p1, src), b = __shfl((int)p2, src), d = __shfl((int)dst, src);
+    const int na = __shfl(n1, src), nb = __shfl(n2, src);
+    const bool in_a = on && c < na && d != a, in_b = on && c < nb;
+    int sa = 0, sb = 0;
+    double ta = 0.0, tb = 0.0;
+    if (in_a) {
+      sa = A.csrc[comp_at(a, c)];
+      ta = A.ctime[comp_at(a, c)];
+    }
+    if (in_b) {
+      sb = A.csrc[comp_at(b, c)];
+      tb = A.ctime[comp_at(b, c)];
+    }
+    if (in_a) {
+      A.csrc[comp_at(d, c)] = sa;
+      A.ctime[comp_at(d, c)] = ta;
+    }
+    if (in_b) {
+      A.csrc[comp_at(d, na + c)] = sb;
+      A.ctime[comp_at(d, na + c)] = tb;
+    }
+    for (int q = 0; q < JOIN_AT_ONCE; ++q) cat &= cat - 1;
   }
   uint64_t todo = __ballot(mine);
-  if (__popcll(todo) > RESAMPLE_MOST) return false;
+  if (__popcll(todo) > RESAMPLE_MOST) return join;
   while (todo) {
     const int src = __ffsll((long long)todo) - 1;
     todo &= todo - 1;
@@ -2662,7 +2707,7 @@ __device__ inline bool wave_resamplings(const Arrays &A, const BoxDesc *B, bool 
                   __shfl((long long)dst, src), __shfl(n1, src), __shfl(n2, src),
                   __shfl(np1, src), __shfl(np2, src));
   }
-  return mine;
+  return mine || join;
 }
 
 // a winning target event (coag_target_with_source and
@@ -3320,8 +3365,8 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
     }
     __syncthreads();
     // 4. apply the winners at their ranks
-    const bool resampled =
-        wave_resamplings(A, B, win && !is_acc, o_win, p1, p2, r_app, ms, par);
+    const bool in_place =
+        wave_components(A, B, win && !is_acc, o_win, p1, p2, r_app, ms, par);
     if (win) {
       TailAlloc al;
       al.B = B;
@@ -3334,7 +3379,7 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
       al.n_samp = al.n_coag = al.n_warn = 0;
       if (is_acc) acc_apply(B, box, t, rec, p1, type, want_terms, rid, al);
       else perset_merge(B, A, W, box, n_box, t, p1, p2, seed, step, type, want_terms, rid, al,
-                        o_win, &ms, resampled, par);
+                        o_win, &ms, in_place, par);
       c_samp += al.n_samp;
       c_coag += al.n_coag;
       c_warn += al.n_warn;
