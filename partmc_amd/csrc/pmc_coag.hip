@@ -436,7 +436,6 @@ int pmc_gpu_create(pmc_gpu **out, int device, int n_box, int n_spec, const doubl
     memset(&B, 0, sizeof(B));
     B.next_id = 1;
     B.id_stride = 1;
-    B.grid_req_n_bin = -1;
     B.w.n_group = 1;
     B.w.n_class = 1;
     B.w.type[0] = WEIGHT_NONE;
@@ -710,14 +709,15 @@ static int run_removal_tiles(pmc_gpu *h, const Removal &X, int64_t n_max, int ac
 
 // The segment passes of a preparation (pmc_prepare.h): the list counters of
 // a wavefront sit in LDS while all of a workgroup's fit.
-static int enqueue_prep_keys(pmc_gpu *h, int only_box) {
+static int enqueue_prep_keys(pmc_gpu *h, int only_box, int explicit_grid) {
   const int keys = h->max_bin * h->tab_classes;
   const dim3 g(SORT_THREADS / PREP_WAVES, only_box >= 0 ? 1 : h->n_box), b(64 * PREP_WAVES);
   if (keys <= PREP_LDS_KEYS)
     hipLaunchKernelGGL(k_prep_keys<true>, g, b, PREP_WAVES * keys * sizeof(int), h->stream,
-                       h->d_box, h->A, only_box, keys);
+                       h->d_box, h->A, only_box, keys, explicit_grid);
   else
-    hipLaunchKernelGGL(k_prep_keys<false>, g, b, 0, h->stream, h->d_box, h->A, only_box, keys);
+    hipLaunchKernelGGL(k_prep_keys<false>, g, b, 0, h->stream, h->d_box, h->A, only_box, keys,
+                       explicit_grid);
   HIPCHECK(hipGetLastError());
   return 0;
 }
@@ -746,11 +746,10 @@ int pmc_gpu_set_bin_grid(pmc_gpu *h, int box, int n_bin, double r_min, double r_
     return fail(711537859, "bin_grid requires 0 < min < max");
   if (h->cap[box] == 0) return fail(ERR_STATE, "set_bin_grid: upload particles first");
   HIPCHECK(hipSetDevice(h->device));
-  hipLaunchKernelGGL(k_set_grid_req, dim3(1), dim3(64), 0, h->stream, h->d_box + box, n_bin, r_min,
-                     r_max);
-  hipLaunchKernelGGL(k_prep_plan, dim3(1), dim3(64), 0, h->stream, h->d_box, h->A, box);
+  hipLaunchKernelGGL(k_prep_plan, dim3(1), dim3(64), 0, h->stream, h->d_box, h->A, box,
+                     GridRequest{n_bin, r_min, r_max});
   HIPCHECK(hipGetLastError());
-  if ((e = enqueue_prep_keys(h, box))) return e;
+  if ((e = enqueue_prep_keys(h, box, 1))) return e;
   BoxDesc B;
   HIPCHECK(read_boxes(h, &B, box, 1));
   std::vector<int> plan(h->n_box, 0);
@@ -764,7 +763,7 @@ int pmc_gpu_set_bin_grid(pmc_gpu *h, int box, int n_bin, double r_min, double r_
     Removal X{};
     X.kind = RM_OUTSIDE;
     if ((e = run_removal_tiles(h, X, B.n_part, 0))) return e;
-    if ((e = enqueue_prep_keys(h, box))) return e;
+    if ((e = enqueue_prep_keys(h, box, 1))) return e;
   }
   if ((e = enqueue_prep_lists(h, box))) return e;
   std::vector<BoxDesc> hb(h->n_box);
@@ -856,9 +855,10 @@ int pmc_gpu_mc_coag_async(pmc_gpu *h, int kernel_type, double del_t) {
     timing_begin(h, "k_prepare", &ev);
     hipLaunchKernelGGL(k_prep_radii, dim3(PREP_RADII_WG, h->n_box), dim3(256), 0, h->stream,
                        h->d_box, h->A, -1);
-    hipLaunchKernelGGL(k_prep_plan, dim3(h->n_box), dim3(64), 0, h->stream, h->d_box, h->A, -1);
+    hipLaunchKernelGGL(k_prep_plan, dim3(h->n_box), dim3(64), 0, h->stream, h->d_box, h->A, -1,
+                       GridRequest{});
     HIPCHECK(hipGetLastError());
-    if ((e = enqueue_prep_keys(h, -1))) return e;
+    if ((e = enqueue_prep_keys(h, -1, 0))) return e;
     if ((e = enqueue_prep_lists(h, -1))) return e;
     timing_end(h, "k_prepare", ev);
     if ((e = enqueue_tables(h, kernel_type))) return e;

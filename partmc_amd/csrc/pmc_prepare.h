@@ -29,6 +29,15 @@
 
 namespace pmc {
 
+// An explicit grid for one box to be sorted on.  It is an argument of the
+// passes and never part of the box: a preparation that ends early (the box
+// holds an error, a class is out of range) leaves no grid behind for a later
+// step, which has no pass that discards.
+struct GridRequest {
+  int n_bin = -1;  // -1: none
+  double r_min = 0.0, r_max = 0.0;
+};
+
 constexpr int PREP_WAVES = 4;      // wavefronts a workgroup of the segment passes
 constexpr int PREP_RADII_WG = 32;  // workgroups a box of k_prep_radii
 constexpr int PREP_LDS_KEYS = 3072;  // list counters of a wavefront kept in LDS up to here
@@ -94,7 +103,7 @@ __global__ void __launch_bounds__(256)
 k_prep_radii(const BoxDesc *boxes, Arrays A, int only_box) {
   const int box = only_box >= 0 ? only_box : (int)blockIdx.y;
   const BoxDesc *B = &boxes[box];
-  if (B->error || B->grid_req_n_bin >= 0 || prep_use_lists(B)) return;
+  if (B->error || prep_use_lists(B)) return;
   double lo = 1e300, hi = -1e300;
   for (int i = blockIdx.x * 256 + threadIdx.x; i < B->n_part; i += gridDim.x * 256) {
     const double r = vol2rad(A.vtot[B->off + i]);
@@ -110,7 +119,8 @@ k_prep_radii(const BoxDesc *boxes, Arrays A, int only_box) {
   }
 }
 
-__global__ void __launch_bounds__(64) k_prep_plan(BoxDesc *boxes, Arrays A, int only_box) {
+__global__ void __launch_bounds__(64)
+k_prep_plan(BoxDesc *boxes, Arrays A, int only_box, GridRequest req) {
   const int box = only_box >= 0 ? only_box : (int)blockIdx.x;
   const int lane = threadIdx.x;
   BoxDesc *B = &boxes[box];
@@ -123,13 +133,13 @@ __global__ void __launch_bounds__(64) k_prep_plan(BoxDesc *boxes, Arrays A, int 
   // a new grid of nn bins, or none (-1)
   int nn = -1;
   double gmin = 0.0, gmax = 0.0;
-  if (B->grid_req_n_bin >= 0) {
-    if (B->grid_req_n_bin > A.max_bin) {
+  if (req.n_bin >= 0) {
+    if (req.n_bin > A.max_bin) {
       err = ERR_CAPACITY;
     } else {
-      nn = B->grid_req_n_bin;
-      gmin = B->grid_req_min;
-      gmax = B->grid_req_max;
+      nn = req.n_bin;
+      gmin = req.r_min;
+      gmax = req.r_max;
     }
   } else {
     const bool use_lists = prep_use_lists(B);
@@ -213,6 +223,11 @@ __global__ void __launch_bounds__(64) k_prep_plan(BoxDesc *boxes, Arrays A, int 
       B->bounds_valid = 0;
       B->tables_valid = 0;
       B->regridded = 1;
+      // the old grid's lists and keys end here, also when the passes after
+      // this one do not get as far as new ones
+      B->valid_sort = 0;
+      B->xlists_valid = 0;
+      B->pkeys_valid = 0;
     }
     if (err) B->error = err;
     B->prep_sort = sort;
@@ -245,11 +260,12 @@ __device__ inline void prep_counters_fence() {
 }
 
 // Bins and classes of the box's particles, and how many of each segment go
-// to each list.  Under an explicit grid, particles outside are counted (the
-// host discards them and repeats the pass); without one they are an error.
+// to each list.  Particles outside an explicit grid are counted (the host
+// discards them and repeats the pass); without one they are an error, so that
+// no particle without a list reaches k_prep_scatter.
 template <bool LDS>
 __global__ void __launch_bounds__(64 * PREP_WAVES)
-k_prep_keys(BoxDesc *boxes, Arrays A, int only_box, int lds_keys) {
+k_prep_keys(BoxDesc *boxes, Arrays A, int only_box, int lds_keys, int explicit_grid) {
   extern __shared__ int s_prep[];
   const int box = only_box >= 0 ? only_box : (int)blockIdx.y;
   BoxDesc *B = &boxes[box];
@@ -260,7 +276,6 @@ k_prep_keys(BoxDesc *boxes, Arrays A, int only_box, int lds_keys) {
   if (seg >= prep_segs(n)) return;
   const int nb = B->n_bin, nc = B->w.n_class, K = nb * nc;
   const int64_t base = B->off;
-  const bool request = B->grid_req_n_bin >= 0;
   int *row = A.sort_scratch + ((int64_t)box * SORT_THREADS + seg) * A.max_keys;
   int *cnt = prep_counters(A, box, seg, LDS ? s_prep : nullptr, lds_keys);
   for (int k = lane; k < K; k += 64) cnt[k] = 0;
@@ -273,7 +288,7 @@ k_prep_keys(BoxDesc *boxes, Arrays A, int only_box, int lds_keys) {
     A.fwd_bin[base + i] = b;
     A.fwd_class[base + i] = c;
     if (b < 1 || b > nb) {
-      if (request) outside++;
+      if (explicit_grid) outside++;
       else atomicExch(&B->error, 708651144);
     } else if (c < 1 || c > nc) {
       atomicExch(&B->error, 233133947);  // weight class out of range
@@ -340,7 +355,6 @@ k_prep_lists(BoxDesc *boxes, Arrays A, int only_box) {
   if (t != 0) return;
   B->pool_top = (int)pos;
   B->pool_cur = h;
-  B->grid_req_n_bin = -1;
   if (pos > B->pool_half) {
     B->error = ERR_CAPACITY;
     return;

@@ -38,8 +38,6 @@ struct BoxDesc {
   int64_t n_accel_pairs;     // parallel mode: pairs the per-particle path would take
   unsigned long long rmin_bits, rmax_bits;  // radius extremes (ordered bits)
   int bounds_kernel;         // kernel type the cached bounds were made for
-  int grid_req_n_bin;        // explicit grid request (-1 = none)
-  double grid_req_min, grid_req_max;
   int prep_sort;             // exact-mode preparation: the box sorts its particles
   int prep_outside;          // ... and its particles outside an explicit grid
   int error;

@@ -166,13 +166,6 @@ __global__ void k_set_next_id(BoxDesc *B, int64_t next_id, int64_t stride, int64
   B->id_offset = offset;
 }
 
-__global__ void k_set_grid_req(BoxDesc *B, int n_bin, double r_min, double r_max) {
-  if (threadIdx.x != 0) return;
-  B->grid_req_n_bin = n_bin;
-  B->grid_req_min = r_min;
-  B->grid_req_max = r_max;
-}
-
 // a box's particles were replaced by n_part new ones
 __global__ void k_set_uploaded(BoxDesc *B, int n_part) {
   if (threadIdx.x != 0) return;

@@ -1,0 +1,67 @@
+"""A box after a call that failed: once its particles are replaced, it steps
+as a box that never saw the failing call.  Whole numbers and list order are
+the oracle's, volumes are sums of the same doubles (relative 1e-12)."""
+import numpy as np
+import pytest
+
+from helpers import compare_state, oracle_box, small
+from partmc_amd import CoagError, CoagGPU, populations as P
+
+pytestmark = pytest.mark.gpu
+
+BAD_CLASS = 233133947  # weight class out of range
+
+
+def make_pop():
+    """5000 Brownian particles without a grid of their own."""
+    pop = small(P.config_c2(), 5000)
+    pop.grid = None
+    return pop
+
+
+def make_gpu(pop):
+    n = pop.n_part
+    g = CoagGPU(1, pop.density)
+    g.reserve([3 * n])
+    g.set_rng(11, 0)
+    g.set_env(0, pop.temp, pop.pressure, pop.beta)
+    g.set_weights(0, [[pop.weight_type]], [[pop.weight_magnitude]], [[pop.weight_exponent]])
+    return g
+
+
+def put(g, pop, klass):
+    n = pop.n_part
+    one = np.ones(n, np.int32)
+    g.upload(0, pop.vol, pop.ids(), one, np.full(n, klass, np.int32))
+    g.set_next_id(0, n + 1)
+
+
+def steps_as_the_oracle(g, pop, steps=3, dt=60.0):
+    ob = oracle_box(pop, 11)
+    total = 0
+    for s in range(steps):
+        want = ob.mc_coag(P.KERNEL_BROWN, dt, s)
+        got = g.mc_coag(P.KERNEL_BROWN, dt)
+        assert want == (int(got[0][0]), int(got[1][0])), s
+        total += want[1]
+    assert total > 0
+    compare_state(ob, g)
+
+
+# the population's radii span 8e-9 to 4e-5 m: grids that leave particles
+# outside below, above, on both sides, and all of them
+@pytest.mark.parametrize("grid", [(40, 5e-8, 1e-3), (40, 1e-10, 5e-8), (10, 4e-8, 6e-8),
+                                  (10, 1e-3, 1e-2)])
+def test_a_failed_set_bin_grid_leaves_no_request(grid):
+    pop = make_pop()
+    g = make_gpu(pop)
+    put(g, pop, 2)  # one class is set
+    with pytest.raises(CoagError) as e:
+        g.set_bin_grid(0, 10, 4e-8, 6e-3)  # fails on the class
+    assert e.value.code == BAD_CLASS
+    with pytest.raises(CoagError) as e:
+        g.set_bin_grid(0, *grid)  # the box holds that error
+    assert e.value.code == BAD_CLASS
+    put(g, pop, 1)
+    steps_as_the_oracle(g, pop)
+    g.close()
