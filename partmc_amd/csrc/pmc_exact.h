@@ -212,6 +212,7 @@ __global__ void k_mark_bounds(BoxDesc *boxes, int n_box, int type) {
   int box = blockIdx.x * blockDim.x + threadIdx.x;
   if (box >= n_box) return;
   BoxDesc *B = &boxes[box];
+  if (B->error) return;  // its bounds were not computed
   if (!B->bounds_valid || B->bounds_kernel != type) {
     B->bounds_valid = 1;
     B->bounds_kernel = type;
@@ -248,7 +249,7 @@ __global__ void k_pair_tables(BoxDesc *boxes, Arrays A) {
 __global__ void k_mark_tables(BoxDesc *boxes, int n_box) {
   int box = blockIdx.x * blockDim.x + threadIdx.x;
   if (box >= n_box) return;
-  boxes[box].tables_valid = 1;
+  if (!boxes[box].error) boxes[box].tables_valid = 1;  // else they were not computed
 }
 
 __device__ inline int64_t table_index(const Arrays &A, int box, int nb, int nc,

@@ -1,11 +1,13 @@
 """A box after a call that failed: once its particles are replaced, it steps
 as a box that never saw the failing call.  Whole numbers and list order are
-the oracle's, volumes are sums of the same doubles (relative 1e-12)."""
+the oracle's (the parallel mode's: a fresh handle's, bit for bit), volumes are
+sums of the same doubles (relative 1e-12)."""
 import numpy as np
 import pytest
 
 from helpers import compare_state, oracle_box, small
-from partmc_amd import CoagError, CoagGPU, populations as P
+from partmc_amd import (CoagError, CoagGPU, MODE_PARALLEL, PREC_FP32_RECHECK, PREC_FP64,
+                        populations as P)
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +67,41 @@ def test_a_failed_set_bin_grid_leaves_no_request(grid):
     put(g, pop, 1)
     steps_as_the_oracle(g, pop)
     g.close()
+
+
+def fail_a_step(g, pop):
+    """A step that makes the box's grid and then fails on the class, so that
+    the majorants and pair tables of the new grid are not computed."""
+    put(g, pop, 2)
+    with pytest.raises(CoagError) as e:
+        g.mc_coag(P.KERNEL_BROWN, 60.0)
+    assert e.value.code == BAD_CLASS
+
+
+def test_a_failed_exact_step_leaves_no_tables():
+    pop = make_pop()
+    g = make_gpu(pop)
+    fail_a_step(g, pop)
+    put(g, pop, 1)
+    g.set_rng(11, 0)
+    steps_as_the_oracle(g, pop)
+    g.close()
+
+
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_FP32_RECHECK])
+def test_a_failed_parallel_step_leaves_no_tables(precision):
+    pop = make_pop()
+    ends = []
+    for fail in (False, True):
+        g = make_gpu(pop)
+        g.set_mode(MODE_PARALLEL, precision, 1e-5)
+        if fail:
+            fail_a_step(g, pop)
+        put(g, pop, 1)
+        g.set_rng(11, 0)
+        counts = [tuple(int(x[0]) for x in g.mc_coag(P.KERNEL_BROWN, 60.0)) for _ in range(3)]
+        ends.append((counts, g.download(0)))
+        g.close()
+    assert ends[0][0] == ends[1][0] and ends[0][0][0][1] > 0
+    for k, v in ends[0][1].items():
+        np.testing.assert_array_equal(ends[1][1][k], v, err_msg=k)
