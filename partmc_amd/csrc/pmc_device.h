@@ -355,7 +355,9 @@ __host__ __device__ inline double powi(double x, int n) {
 // every test, merge and bin evaluates several in a chain: 20 replay steps of
 // 1e4 additive particles take 15.5 ms (17.1 with pow), three size
 // distributions of 1.5e6 particles 194 us (218).
-// Zero, negative, infinite and NaN arguments give what pow gives.
+// Other arguments give what pow gives: either zero 0, either infinity infinity
+// (a volume that overflowed lies outside every grid), and finite negatives
+// and NaN the NaN that the logarithm carries through.
 __device__ __forceinline__ double pow_third(double x) {
   // x = a 2^(3 q), a in [0.5, 4)
   const int e = __builtin_amdgcn_frexp_exp(x);
@@ -371,7 +373,8 @@ __device__ __forceinline__ double pow_third(double x) {
   const double lnx = ((double)(3 * q) + (double)l) * 0.69314718055994530942;
   const double z =
       __builtin_amdgcn_ldexp(fma(y, fma(r, c, -1.850371707708594e-17 * lnx), y), q);
-  return x > 0.0 && x < __builtin_huge_val() ? z : x < 0.0 ? __builtin_nan("") : x + 0.0;
+  constexpr int ZERO_OR_INF = 0x264;  // class bits of -inf, -0, +0 and +inf
+  return __builtin_amdgcn_class(x, ZERO_OR_INF) ? fabs(x) : z;
 }
 
 // x / PI and x / 3, correctly rounded as the division is: one correction of
