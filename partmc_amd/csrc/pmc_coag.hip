@@ -570,10 +570,19 @@ static int put_particles(pmc_gpu *h, int64_t base, int n_part, const double *vol
   const int ns = h->n_spec;
   const bool times = least && greatest;
   const unsigned fields = REC_VOL | REC_GROUP | REC_KLASS | (id ? REC_ID : 0) |
-                          (n_primary ? REC_NPRIM : 0) |
-                          (n_comp ? REC_NCOMP | REC_CSRC | REC_CTIME : 0) |
+                          (n_primary ? REC_NPRIM : 0) | (n_comp ? REC_NCOMP : 0) |
                           (times ? REC_LEAST | REC_GREATEST : 0);
   const int64_t chunk = (int64_t)(STAGE_BYTES / record_bytes(fields, ns));
+  if (n_comp && n_part > 0) {
+    // the caller's [n_part][MAX_COMP] arrays are the device layout
+    HIPCHECK(hipMemcpyAsync(h->A.csrc + comp_at(base, 0), comp_source,
+                            (size_t)n_part * MAX_COMP * sizeof(int), hipMemcpyHostToDevice,
+                            h->stream));
+    HIPCHECK(hipMemcpyAsync(h->A.ctime + comp_at(base, 0), comp_time,
+                            (size_t)n_part * MAX_COMP * sizeof(double), hipMemcpyHostToDevice,
+                            h->stream));
+    HIPCHECK(hipStreamSynchronize(h->stream));
+  }
   std::lock_guard<std::mutex> lock(h->stage_lock);
   for (int64_t i0 = 0, c = 0; i0 < n_part; i0 += chunk, ++c) {
     const int part = (int)(c % STAGE_PARTS);
@@ -585,12 +594,7 @@ static int put_particles(pmc_gpu *h, int64_t base, int n_part, const double *vol
     memcpy(R.group, group + i0, m * sizeof(int));
     memcpy(R.klass, klass + i0, m * sizeof(int));
     if (R.nprim) memcpy(R.nprim, n_primary + i0, m * sizeof(int));
-    if (R.ncomp) {
-      // the caller's [n_part][MAX_COMP] arrays are the device layout
-      memcpy(R.ncomp, n_comp + i0, m * sizeof(int));
-      memcpy(R.csrc, comp_source + i0 * MAX_COMP, m * MAX_COMP * sizeof(int));
-      memcpy(R.ctime, comp_time + i0 * MAX_COMP, m * MAX_COMP * sizeof(double));
-    }
+    if (R.ncomp) memcpy(R.ncomp, n_comp + i0, m * sizeof(int));
     if (times) {
       memcpy(R.least, least + i0, m * sizeof(double));
       memcpy(R.greatest, greatest + i0, m * sizeof(double));
