@@ -113,7 +113,8 @@ struct pmc_gpu {
   std::vector<double *> tape_buf;  // per box: device values of its tape, or null
   std::vector<int64_t> off;     // per-box first slot
   // pinned memory between the host's arrays and the device: a ring for
-  // particles (pmc_transfer.h) and a copy of the descriptors
+  // particles (pmc_transfer.h), allocated by the first of them, and a copy of
+  // the descriptors
   char *stage = nullptr;
   hipEvent_t stage_done[STAGE_PARTS] = {};  // the kernel that uses a part has ended
   BoxDesc *box_copy = nullptr;
@@ -192,6 +193,11 @@ static hipError_t read_boxes(pmc_gpu *h, BoxDesc *dst, int first, int n) {
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
   if (e == hipSuccess) memcpy((void *)dst, h->box_copy, sizeof(BoxDesc) * n);
   return e;
+}
+
+// the ring, with stage_lock held
+static hipError_t stage_ensure(pmc_gpu *h) {
+  return h->stage ? hipSuccess : hipHostMalloc((void **)&h->stage, STAGE_PARTS * STAGE_BYTES);
 }
 
 static int alloc_tables(pmc_gpu *h, int classes) {
@@ -447,7 +453,6 @@ int pmc_gpu_create(pmc_gpu **out, int device, int n_box, int n_spec, const doubl
   HIPCHECK(hipMemcpy(h->d_box, hb.data(), sizeof(BoxDesc) * n_box, hipMemcpyHostToDevice));
   h->cap.assign(n_box, 0);
   h->off.assign(n_box, 0);
-  HIPCHECK(hipHostMalloc((void **)&h->stage, STAGE_PARTS * STAGE_BYTES));
   HIPCHECK(hipHostMalloc((void **)&h->box_copy, sizeof(BoxDesc) * n_box));
   for (hipEvent_t &ev : h->stage_done)
     HIPCHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -573,7 +578,8 @@ static int put_particles(pmc_gpu *h, int64_t base, int n_part, const double *vol
                           (n_primary ? REC_NPRIM : 0) | (n_comp ? REC_NCOMP : 0) |
                           (times ? REC_LEAST | REC_GREATEST : 0);
   const int64_t chunk = (int64_t)(STAGE_BYTES / record_bytes(fields, ns));
-  if (n_comp && n_part > 0) {
+  if (n_part == 0) return 0;
+  if (n_comp) {
     // the caller's [n_part][MAX_COMP] arrays are the device layout
     HIPCHECK(hipMemcpyAsync(h->A.csrc + comp_at(base, 0), comp_source,
                             (size_t)n_part * MAX_COMP * sizeof(int), hipMemcpyHostToDevice,
@@ -584,6 +590,7 @@ static int put_particles(pmc_gpu *h, int64_t base, int n_part, const double *vol
     HIPCHECK(hipStreamSynchronize(h->stream));
   }
   std::lock_guard<std::mutex> lock(h->stage_lock);
+  HIPCHECK(stage_ensure(h));
   for (int64_t i0 = 0, c = 0; i0 < n_part; i0 += chunk, ++c) {
     const int part = (int)(c % STAGE_PARTS);
     const size_t m = (size_t)std::min<int64_t>(chunk, n_part - i0);
@@ -623,6 +630,7 @@ static int get_particles(pmc_gpu *h, int64_t base, int n, double *vol, int64_t *
   const int64_t chunk = (int64_t)(STAGE_BYTES / record_bytes(fields, ns));
   const int64_t chunks = (n + chunk - 1) / chunk;
   std::lock_guard<std::mutex> lock(h->stage_lock);
+  HIPCHECK(stage_ensure(h));
   auto records = [&](int64_t c) {
     return records_at(h->stage + (c % STAGE_PARTS) * STAGE_BYTES, fields,
                       std::min<int64_t>(chunk, n - c * chunk), ns);
@@ -1621,6 +1629,7 @@ int pmc_gpu_get_removed(pmc_gpu *h, int box, int max_n, int *n, int64_t *id, int
   if (cnt == 0) return 0;
   // through the pinned ring, all of it at a time
   std::lock_guard<std::mutex> lock(h->stage_lock);
+  HIPCHECK(stage_ensure(h));
   const int64_t chunk = (int64_t)(STAGE_PARTS * STAGE_BYTES / (2 * sizeof(int64_t) + sizeof(int)));
   int64_t *s_id = (int64_t *)h->stage, *s_other = s_id + chunk;
   int *s_action = (int *)(s_other + chunk);

@@ -27,7 +27,7 @@
 namespace pmc {
 
 constexpr int STAGE_PARTS = 4;
-constexpr size_t STAGE_BYTES = 1 << 20;  // of a part: past it more does not pay, and 4 MB a handle stay pinned
+constexpr size_t STAGE_BYTES = 1 << 20;  // of a part: past it more does not pay, and 4 MB of a handle that moves particles stay pinned
 constexpr int XFER_THREADS = 128;  // 32 KB of LDS for the most species
 
 // the fields of a chunk of particles in a part; null: absent

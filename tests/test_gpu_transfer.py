@@ -89,6 +89,35 @@ def test_scaled_weights_and_ids():
     g.close()
 
 
+def mapped_bytes():
+    """Address space of this process that the device's driver maps."""
+    total = 0
+    with open("/proc/self/maps") as f:
+        for line in f:
+            if "/dev/dri/" in line:
+                lo, hi = line.split()[0].split("-")
+                total += int(hi, 16) - int(lo, 16)
+    return total
+
+
+def test_a_handle_pins_its_ring_with_the_first_particles():
+    """Handles that move no particles hold no ring: each grows by one when its
+    first particle arrives, in slots that are there already."""
+    handles = [CoagGPU(1, np.array([1000.0])) for _ in range(4)]
+    for g in handles:
+        g.reserve([16])
+        g.sync()
+    before = mapped_bytes()
+    for g in handles:
+        g.upload(0, np.array([[1e-20]]), [1], [1], [1])
+        g.sync()
+    grown = mapped_bytes() - before
+    for g in handles:
+        np.testing.assert_array_equal(g.download(0)["id"], [1])
+        g.close()
+    assert grown >= len(handles) * 4 * PART
+
+
 def test_whole_records_go_up_at_the_rate_of_a_copy():
     """Records with their components (240 of 296 bytes each here) from pinned
     arrays of the caller's take less than twice a plain copy of as many bytes:
