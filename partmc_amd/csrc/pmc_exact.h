@@ -90,32 +90,6 @@ __device__ inline int weighted_kernel64(const Arrays &A, const Weights &w,
   return err;
 }
 
-// bin_grid_make (log), src/bin_grid.F90:83-138 via logspace
-// src/util.F90:497-520 (one thread)
-__device__ inline void make_log_grid(int n_bin, double rmin, double rmax,
-                                     double *edges, double *centers,
-                                     double *widths) {
-  if (n_bin <= 0) return;
-  double lmin = log(rmin), lmax = log(rmax);
-  int n = n_bin + 1;
-  for (int i = 2; i <= n - 1; ++i) {
-    double a = (double)(i - 1) / (double)(n - 1);
-    edges[i - 1] = exp((1.0 - a) * lmin + a * lmax);
-  }
-  edges[0] = rmin;
-  edges[n - 1] = rmax;
-  double c1 = exp(interp_linear_disc(lmin, lmax, 2 * n_bin + 1, 2));
-  double c2 = exp(interp_linear_disc(lmin, lmax, 2 * n_bin + 1, 2 * n_bin));
-  double lc1 = log(c1), lc2 = log(c2);
-  for (int i = 2; i <= n_bin - 1; ++i) {
-    double a = (double)(i - 1) / (double)(n_bin - 1);
-    centers[i - 1] = exp((1.0 - a) * lc1 + a * lc2);
-  }
-  centers[0] = c1;
-  centers[n_bin - 1] = c2;
-  for (int i = 0; i < n_bin; ++i) widths[i] = (lmax - lmin) / (double)n_bin;
-}
-
 // whole-record copy of particle slot `from` into slot `to`.  Fields are
 // read in chunks before they are written: a store between two loads of
 // the same arrays makes the second wait for the first, one memory round

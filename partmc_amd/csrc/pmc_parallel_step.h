@@ -196,7 +196,6 @@ struct ParallelWork {
   size_t sort_tmp_bytes = 0;
   std::vector<int> tiles_in_box;
   uint32_t *h_u32 = nullptr;  // pinned scalars
-  int *h_i32 = nullptr;
   unsigned long long *h_u64 = nullptr;
   // optional per-kernel timing hooks of the owning handle
   void (*tbegin)(void *, const char *, hipEvent_t *) = nullptr;
@@ -835,10 +834,6 @@ __device__ inline void atomic_max_double(double *addr, double v) {
 // A particle's status this step.  Statuses carry the epoch of the step that
 // set them, so a new step starts with every particle live without clearing
 // the array (it is cleared when the epoch wraps).
-__device__ inline uint8_t st_get(const PW &W, int64_t p) {
-  const uint32_t v = W.slot[p].st;
-  return (int)(v >> 2) == W.epoch ? (uint8_t)(v & 3) : ST_LIVE;
-}
 __device__ inline void st_set(const PW &W, int64_t p, uint8_t s) {
   W.slot[p].st = (uint32_t)((W.epoch << 2) | s);
 }
@@ -3685,7 +3680,6 @@ inline int parallel_init(ParallelWork &W, int n_box, int max_bin) {
   W.d.max_bin = max_bin;
   W.d.tab_classes = 1;
   if (hipHostMalloc((void **)&W.h_u32, 64 * sizeof(uint32_t)) != hipSuccess) return ERR_HIP;
-  if (hipHostMalloc((void **)&W.h_i32, 64 * sizeof(int)) != hipSuccess) return ERR_HIP;
   if (hipHostMalloc((void **)&W.h_u64, 8 * sizeof(unsigned long long)) != hipSuccess) return ERR_HIP;
   if (hipStreamCreate(&W.st2) != hipSuccess) return ERR_HIP;
   if (hipMalloc((void **)&W.pstat, 2 * sizeof(unsigned long long)) != hipSuccess) return ERR_HIP;
@@ -3760,11 +3754,9 @@ inline void parallel_free_arrays(ParallelWork &W) {
 inline void parallel_free(ParallelWork &W) {
   parallel_free_arrays(W);
   if (W.h_u32) (void)hipHostFree(W.h_u32);
-  if (W.h_i32) (void)hipHostFree(W.h_i32);
   if (W.h_u64) (void)hipHostFree(W.h_u64);
   W.h_u64 = nullptr;
   W.h_u32 = nullptr;
-  W.h_i32 = nullptr;
   if (W.ev_fork) (void)hipEventDestroy(W.ev_fork);
   if (W.ev_join) (void)hipEventDestroy(W.ev_join);
   if (W.st2) (void)hipStreamDestroy(W.st2);

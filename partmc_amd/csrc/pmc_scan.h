@@ -57,10 +57,10 @@ __device__ inline T block_reduce(T v, Op op, scan_storage<BLOCK, T> &st) {
 }
 
 // ------------------------------------------------------- device-wide scans
-// Up to SCAN_COLS arrays of 32-bit elements of one length n are scanned in
+// Exclusive sums: up to SCAN_COLS arrays of 32-bit elements of one length n in
 // the same launches (a claim round's four event flags).  Sums wrap modulo
-// 2^32, so int and uint32_t arrays scan alike.  An exclusive sum also
-// writes its total at out[n] and, when total_dst is set, there.
+// 2^32, so int and uint32_t arrays scan alike.  The total is also written at
+// out[n] and, when total_dst is set, there.
 constexpr int SCAN_COLS = 4;
 constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_UNROLL = 4;            // segments of SCAN_THREADS elements loaded together
@@ -74,7 +74,7 @@ struct ScanJob {
   const int *n_dev;    // element count in device memory, or null
   int64_t n_host;      // the count when n_dev is null
   uint32_t *partial;   // [SCAN_COLS * SCAN_MAX_BLOCKS] chunk totals
-  int *total_dst;      // exclusive sums: the first column's total also goes here
+  int *total_dst;      // the first column's total also goes here, or null
 };
 
 __device__ inline int64_t scan_n(const ScanJob &J) { return J.n_dev ? (int64_t)*J.n_dev : J.n_host; }
@@ -88,19 +88,18 @@ __device__ inline void scan_chunk(int64_t n, int g, int b, int64_t *s0, int64_t 
   *s1 = *s0 + per < segs ? *s0 + per : segs;
 }
 
-template <typename Op>
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_chunks(ScanJob J, Op op, uint32_t ident) {
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_chunks(ScanJob J) {
   __shared__ scan_storage<SCAN_THREADS, uint32_t> s;
   const int64_t n = scan_n(J);
   int64_t s0, s1;
   scan_chunk(n, gridDim.x, blockIdx.x, &s0, &s1);
   for (int c = 0; c < J.cols; ++c) {
-    uint32_t acc = ident;
+    uint32_t acc = 0;
     for (int64_t sg = s0; sg < s1; ++sg) {
       const int64_t i = sg * SCAN_THREADS + threadIdx.x;
-      if (i < n) acc = op(acc, J.in[c][i]);
+      if (i < n) acc += J.in[c][i];
     }
-    acc = block_reduce<SCAN_THREADS>(acc, op, s);
+    acc = block_reduce<SCAN_THREADS>(acc, OpSum(), s);
     if (threadIdx.x == 0) J.partial[c * SCAN_MAX_BLOCKS + blockIdx.x] = acc;
   }
 }
@@ -112,9 +111,8 @@ struct ScanOnly {
   __device__ void operator()(int64_t, uint32_t, uint32_t) const {}
 };
 
-template <typename Op, bool EXCL, typename F>
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(ScanJob J, Op op, uint32_t ident,
-                                                             F each) {
+template <typename F>
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(ScanJob J, F each) {
   __shared__ scan_storage<SCAN_THREADS, uint32_t> s;
   const int64_t n = scan_n(J);
   const int g = gridDim.x, b = blockIdx.x;
@@ -122,15 +120,13 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(ScanJob J, Op op, u
   scan_chunk(n, g, b, &s0, &s1);
   for (int c = 0; c < J.cols; ++c) {
     // the chunks before this one, and all of them for the total
-    uint32_t before = ident, all = ident;
+    uint32_t before = 0, all = 0;
     if (g > 1) {
       for (int q0 = 0; q0 < g; q0 += SCAN_THREADS) {
         const int q = q0 + threadIdx.x;
-        const uint32_t p = q < g ? J.partial[c * SCAN_MAX_BLOCKS + q] : ident;
-        const uint32_t rb = block_reduce<SCAN_THREADS>(q < b ? p : ident, op, s);
-        const uint32_t ra = block_reduce<SCAN_THREADS>(p, op, s);
-        before = op(before, rb);
-        all = op(all, ra);
+        const uint32_t p = q < g ? J.partial[c * SCAN_MAX_BLOCKS + q] : 0;
+        before += block_reduce<SCAN_THREADS>(q < b ? p : 0u, OpSum(), s);
+        all += block_reduce<SCAN_THREADS>(p, OpSum(), s);
       }
     }
     uint32_t carry = before;
@@ -141,24 +137,23 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(ScanJob J, Op op, u
 #pragma unroll
       for (int u = 0; u < SCAN_UNROLL; ++u) {
         const int64_t i = (sg + u) * SCAN_THREADS + threadIdx.x;
-        v[u] = (sg + u < s1 && i < n) ? in[i] : ident;
+        v[u] = (sg + u < s1 && i < n) ? in[i] : 0;
       }
 #pragma unroll
       for (int u = 0; u < SCAN_UNROLL; ++u) {
         if (sg + u >= s1) break;  // uniform over the workgroup
         const int64_t i = (sg + u) * SCAN_THREADS + threadIdx.x;
         uint32_t tot;
-        const uint32_t r = block_scan_incl<SCAN_THREADS>(v[u], op, s, &tot);
+        const uint32_t res = carry + block_sum_excl<SCAN_THREADS>(v[u], s, &tot);
         if (i < n) {
-          const uint32_t res = EXCL ? carry + (r - v[u]) : op(carry, r);
           out[i] = res;
           if (c == 0) each(i, v[u], res);
         }
-        carry = op(carry, tot);
+        carry += tot;
       }
     }
     if (g == 1) all = carry;
-    if (EXCL && b == 0 && threadIdx.x == 0) {
+    if (b == 0 && threadIdx.x == 0) {
       out[n] = all;
       if (c == 0 && J.total_dst) *J.total_dst = (int)all;
     }
@@ -176,9 +171,8 @@ inline int scan_blocks(int64_t n_bound) {
 template <typename F = ScanOnly>
 inline void scan_excl_sum(const ScanJob &J, int64_t n_bound, hipStream_t st, F each = F()) {
   const int g = scan_blocks(n_bound);
-  if (g > 1) hipLaunchKernelGGL(k_scan_chunks<OpSum>, dim3(g), dim3(SCAN_THREADS), 0, st, J, OpSum(), 0u);
-  hipLaunchKernelGGL((k_scan_apply<OpSum, true, F>), dim3(g), dim3(SCAN_THREADS), 0, st, J,
-                     OpSum(), 0u, each);
+  if (g > 1) hipLaunchKernelGGL(k_scan_chunks, dim3(g), dim3(SCAN_THREADS), 0, st, J);
+  hipLaunchKernelGGL(k_scan_apply<F>, dim3(g), dim3(SCAN_THREADS), 0, st, J, each);
 }
 
 // a job over one array
