@@ -2362,6 +2362,15 @@ __device__ inline void resample_components(const Arrays &A, Stream &s, int64_t p
   }
 }
 
+// Every lane's loads before any lane's stores after it.  The fence keeps the
+// compiler from moving either across; the barrier is convergent, so branches
+// before and after it on one condition stay two branches and no lane runs
+// ahead to its stores.  Neither is an instruction.
+__device__ inline void wave_handoff() {
+  wave_fence();
+  __builtin_amdgcn_wave_barrier();
+}
+
 // One lane's resampling by its whole wavefront: about 40 uniforms of one
 // stream are 20 Philox blocks, one a lane, and the components go through the
 // lanes.  Every lane takes part; the arguments are the resampling lane's,
@@ -2393,6 +2402,7 @@ __device__ inline void wave_resample(const Arrays &A, const Stream &s, int i0, i
   uint32_t take1, take2;
   const int n1_new = resample_masks(u, n1, n2, np1, np2, &take1, &take2);
   const uint32_t below = lane < 32 ? (1u << lane) - 1u : 0u;
+  wave_handoff();  // dst may be a parent's slot
   if (lane < MAX_COMP) {
     if ((take1 >> lane) & 1u) {
       const int c = __popc(take1 & below);
@@ -2675,6 +2685,7 @@ __device__ inline bool wave_components(const Arrays &A, const BoxDesc *B, bool w
       sb = A.csrc[comp_at(b, c)];
       tb = A.ctime[comp_at(b, c)];
     }
+    wave_handoff();  // d may be b: a lane's store is over another's load
     if (in_a) {
       A.csrc[comp_at(d, c)] = sa;
       A.ctime[comp_at(d, c)] = ta;
@@ -2683,6 +2694,7 @@ __device__ inline bool wave_components(const Arrays &A, const BoxDesc *B, bool w
       A.csrc[comp_at(d, na + c)] = sb;
       A.ctime[comp_at(d, na + c)] = tb;
     }
+    wave_handoff();
     for (int q = 0; q < JOIN_AT_ONCE; ++q) cat &= cat - 1;
   }
   uint64_t todo = __ballot(mine);
