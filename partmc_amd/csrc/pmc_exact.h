@@ -1264,6 +1264,7 @@ k_exact_sweep(BoxDesc *boxes, Arrays A, int type, double del_t, uint64_t seed, u
           }
         }
         const uint64_t vm = __ballot(valid);
+        if (!vm) break;  // no pair left (the second class may have no particle)
         uint64_t todo = __ballot(kind != 0 || n_samp > 0);
         bool changed = false;
         int at = 63 - __clzll((long long)vm);  // the last pair settled by this pass

@@ -60,3 +60,37 @@ def test_sweep_matches_oracle(n, weights, n_class, grid, max_bin, dt, steps):
     assert total > 0
     compare_state(ob, g, n_class=n_class)
     assert int(g.path_stats()["n_accel_pairs"][0]) == ob.n_accel
+
+
+@pytest.mark.parametrize("counts", [(0, 300, 200), (300, 0, 200), (300, 200, 0), (0, 0, 400),
+                                    (400, 0, 0), (0, 1, 0)])
+def test_classes_without_particles_match_oracle(counts):
+    """Pairs of classes of which the first, the second or both have no
+    particle."""
+    weights = ([[1, 1, 1]], [[2e9, 1e9, 3e9]], [[0.0, 0.0, 0.0]])
+    grid = (60, 1e-10, 1e-5)
+    n = sum(counts)
+    rng = np.random.default_rng(n)
+    vol = 10 ** rng.uniform(-24, -21, size=(n, 1)) * rng.dirichlet([1, 2, 1], size=n)
+    klass = np.repeat(np.arange(1, 4), counts).astype(np.int32)
+    ids, one = np.arange(1, n + 1), np.ones(n, np.int32)
+    dens = np.array([1800.0, 1000.0, 1400.0])
+    g = CoagGPU(1, dens)
+    g.set_rng(n, 0)
+    g.set_weights(0, *weights)
+    g.upload(0, vol, ids, one, klass, capacity=4 * n + 64)
+    g.set_next_id(0, n + 1)
+    g.set_bin_grid(0, *grid)
+    ob = oracle.Box(dens, oracle.Weights(*weights), seed=n)
+    ob.add_particles(vol, ids, one, klass)
+    ob.next_id = n + 1
+    ob.sort_with_grid(*grid)
+    total = 0
+    for s in range(4):
+        want = ob.mc_coag(P.KERNEL_BROWN, 30.0, s)
+        got = g.mc_coag(P.KERNEL_BROWN, 30.0)
+        assert want == (int(got[0][0]), int(got[1][0])), s
+        total += want[1]
+    assert total > 0 or n == 1
+    compare_state(ob, g, n_class=3)
+    g.close()
