@@ -104,8 +104,8 @@ struct PW {  // device view of the parallel work arrays
   int *s_app, *s_id, *s_info, *s_hole;
   int *box_first;
   uint64_t *holes, *holes_sorted;  // (box << 32 | slot)
-  int *cmp_lo, *cmp_hi, *cmp_head;
-  unsigned long long *acc_samp;  // samples drawn by the device-wide target walks  // [n_box] compaction: hole range and holes below the final count
+  int *cmp_lo, *cmp_hi, *cmp_head;  // [n_box] compaction: hole range and holes below the final count
+  unsigned long long *acc_samp;  // samples drawn by the device-wide target walks
   // accelerated per-particle path (try_per_particle_coag): one test slot per
   // target particle, one event record per target slot of a batch
   uint8_t *pair_acc;           // [NP] 0 per-set; 1 targets in (b1, c1); 2 targets in (b2, c2)
@@ -584,8 +584,6 @@ __device__ inline int pair_box(const PW &W, int64_t k, int64_t *q) {
   return box;
 }
 
-// loops over a record's species: unrolled over NS where that is few, so
-// that the record stays in registers
 // The step's arguments for the functions called out of line (target visits
 // and their merges), in LDS: passed by reference they would live in each
 // lane's private memory, and every pointer read from there waits for all
@@ -605,6 +603,8 @@ __device__ inline void step_ctx_fill(const Arrays &A, const PW &W) {
   __syncthreads();
 }
 
+// loops over a record's species: unrolled over NS where that is few, so
+// that the record stays in registers
 #define REC_FOR(s, ns) for (int s = 0; s < (NS <= FEW_SPEC ? NS : (ns)); ++s) if (NS > FEW_SPEC || s < (ns))
 
 // the record without its components (they are read in a second pass
@@ -3181,7 +3181,7 @@ __device__ inline void tail_barrier() {
 
 // The tail of a batch: the tests still pending after the device-wide claim
 // rounds, mostly chains of tests on one particle (a large particle drawn by
-// many tests of its bin pairs).  One wavefront per box runs claim rounds
+// many tests of its bin pairs).  One workgroup per box runs claim rounds
 // over a window of the box's next TAIL_THREADS pending tests, in sequential
 // order, with barriers in place of launches.  A test is run again only when
 // a particle it read or claimed was changed by an earlier winner; a test

@@ -14,9 +14,9 @@
 //     box's particles (slice b is [b n / NB, (b+1) n / NB)).  Each wavefront
 //     keeps its own LDS histogram.  Lanes that hold the same bin find each
 //     other with one ballot per bit of the bin; the first of them adds the
-//     others' values in lane order and updates the bin, one writer per bin.  The workgroup adds its wavefronts'
-//     histograms in order and writes the whole window (zeros included) to
-//     partials[b][.].
+//     others' values in lane order and updates the bin, one writer per bin.
+//     The workgroup adds its wavefronts' histograms in order and writes the
+//     whole window (zeros included) to partials[b][.].
 //   k_dist_reduce: adds partials[0..NB)[bin], RED_ROWS rows a thread and
 //     the rows' sums in order.
 // Bins are handled in windows of at most DIST_WIN, one pair of passes per
