@@ -2947,6 +2947,13 @@ k_par_apply_chains(BoxDesc *boxes, Arrays A, PW W, int rid) {
     apply_chain(boxes, A, W, e, lane, hole_base, rid);
 }
 
+// A box's count with `added` more particles.  Those beyond its capacity were
+// not written (the box holds ERR_CAPACITY), and no pass after this one, nor a
+// reader of the box, may go past the slots that were.
+__device__ inline int grown(const BoxDesc *B, int64_t added) {
+  return (int)min((int64_t)B->n_part + added, B->cap);
+}
+
 // per-box totals of a round: appended slots, new ids, records, winners
 __device__ inline void box_totals(BoxDesc *boxes, const PW &W, int E, int box) {
   const int first = W.box_first[box];
@@ -2958,7 +2965,7 @@ __device__ inline void box_totals(BoxDesc *boxes, const PW &W, int E, int box) {
   }
   const int last = lo;
   BoxDesc *B = &boxes[box];
-  B->n_part += W.s_app[last] + W.f_app[last] - W.s_app[first];
+  B->n_part = grown(B, (int64_t)W.s_app[last] + W.f_app[last] - W.s_app[first]);
   B->next_id += W.s_id[last] + W.f_id[last] - W.s_id[first];
   B->n_info += W.s_info[last] + W.f_info[last] - W.s_info[first];
 }
@@ -3393,7 +3400,7 @@ k_par_tail(BoxDesc *boxes, Arrays A, PW W, int n_box, const uint32_t *pend, int 
     }
     tail_barrier();
     if (tid == 0) {
-      B->n_part += s_tot[0];
+      B->n_part = grown(B, s_tot[0]);
       B->next_id += s_tot[1];
       B->n_info += s_tot[2];
     }

@@ -105,3 +105,65 @@ def test_a_failed_parallel_step_leaves_no_tables(precision):
     assert ends[0][0] == ends[1][0] and ends[0][0][0][1] > 0
     for k, v in ends[0][1].items():
         np.testing.assert_array_equal(ends[1][1][k], v, err_msg=k)
+
+
+CAPACITY = 3  # particle, list or grid capacity exceeded
+
+
+def power_pop(n, seed):
+    """Particles whose weights make merges keep their parents, so that a step
+    appends many."""
+    rng = np.random.default_rng(seed)
+    vol = 10 ** rng.uniform(-24, -20, size=(n, 1)) * rng.dirichlet([1, 1], size=n)
+    return P.Population(vol=vol, density=np.array([1800.0, 1000.0]), weight_type=P.WEIGHT_POWER,
+                        weight_magnitude=1e-14, weight_exponent=-3.0)
+
+
+def flat_pop(n, seed, weight):
+    """Larger particles under a flat weight: each merge is one particle less."""
+    pop = power_pop(n, seed)
+    pop.vol = pop.vol * 1e6
+    pop.weight_type, pop.weight_magnitude, pop.weight_exponent = P.WEIGHT_NONE, weight, 0.0
+    return pop
+
+
+def parallel_boxes(pops, room):
+    g = CoagGPU(len(pops), pops[0].density)
+    g.reserve([p.n_part + r for p, r in zip(pops, room)])
+    g.set_rng(3, 0)
+    for b, p in enumerate(pops):
+        g.load_population(b, p)
+    g.set_mode(MODE_PARALLEL, PREC_FP32_RECHECK, 1e-5)
+    return g
+
+
+@pytest.mark.parametrize("n,kernel,dt,flat", [(300, P.KERNEL_CONSTANT, 60.0, 2e6),
+                                              (3000, P.KERNEL_BROWN, 600.0, 5e7)])
+@pytest.mark.parametrize("room", [0, 1, 40])
+def test_a_parallel_step_beyond_the_capacity(n, kernel, dt, flat, room):
+    """A box that runs out of slots ends with its error, within its slots.  The
+    box whose slots follow conserves its particles (volumes in sums of n
+    terms, n 2^-52), and the full one is as a new handle's with its next
+    particles, which are larger, so that both make their grid anew."""
+    full, other = power_pop(n, 1), flat_pop(n, 2, flat)
+    g = parallel_boxes([full, other], [room, 0])
+    with pytest.raises(CoagError) as e:
+        g.mc_coag(kernel, dt)
+    assert e.value.code == CAPACITY
+    assert g.n_part(0) <= n + room
+    assert np.isfinite(g.download(0)["vol"]).all()
+    d, merges = g.download(1), int(g.counters()["n_coag"][1])
+    assert merges > 0 and len(d["id"]) == n - merges == len(np.unique(d["id"]))
+    assert d["n_primary"].sum() == n
+    np.testing.assert_allclose(d["vol"].sum(axis=0), other.vol.sum(axis=0), rtol=n * 2.0 ** -52,
+                               atol=0)
+    new = parallel_boxes([flat_pop(n, 5, flat), other], [room, 0])
+    g.load_population(0, flat_pop(n, 5, flat))
+    ends = []
+    for h in (g, new):
+        h.set_rng(7, 0)
+        ends.append(([int(x[0]) for x in h.mc_coag(kernel, dt)], h.download(0)))
+        h.close()
+    assert ends[0][0] == ends[1][0] and ends[0][0][1] > 0
+    for k, v in ends[0][1].items():
+        np.testing.assert_array_equal(ends[1][1][k], v, err_msg=k)
