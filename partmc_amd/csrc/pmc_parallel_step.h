@@ -249,13 +249,23 @@ static hipError_t pmalloc(T **p, size_t n) {
 __device__ inline int par_key(int bin, int cls, int nb) { return (bin - 1) + nb * (cls - 1); }
 
 // keys (and optionally FP32 terms and cached volumes) for every particle of
-// boxes whose keys are stale; terms for boxes whose terms are stale
+// boxes whose keys are stale; terms for boxes whose terms are stale.  A target
+// event that ended in an error held claims and is in no list that releases
+// them: the slots of a box that goes on after an error are released here (a
+// claim left on a source holds up every event that reads it, for good).
 __global__ void __launch_bounds__(TILE_THREADS)
 k_par_rekey(BoxDesc *boxes, Arrays A, PW W, int type, int want_terms, int phase) {
   const int tile = blockIdx.x;
   const int box = W.tile_box[tile];
   BoxDesc *B = &boxes[box];
   if (B->error) return;
+  if (phase == 0 && B->revived)
+    for (int it = 0; it < TILE_ITEMS; ++it) {
+      const int64_t i = W.tile_start[tile] + it * TILE_THREADS + threadIdx.x;
+      if (i >= B->cap) continue;
+      W.slot[B->off + i].claim = UNCLAIMED;
+      W.slot[B->off + i].claim_wr = UNCLAIMED;
+    }
   const bool do_keys = phase == 0 ? (!B->pkeys_valid && B->valid_sort && B->n_bin > 0)
                                   : (B->rekey != 0);
   const bool do_terms = want_terms && phase == 0 && B->terms_kernel != type;
@@ -308,6 +318,7 @@ __global__ void k_par_finish_rekey(BoxDesc *boxes, int n_box, int type, int want
   BoxDesc *B = &boxes[box];
   if (phase == 0) {
     if (!B->pkeys_valid && B->valid_sort && B->n_bin > 0) B->pkeys_valid = 1;
+    if (!B->error) B->revived = 0;
     // FP64 steps do not keep the terms of new particles current
     B->terms_kernel = want_terms ? type : 0;
   } else if (B->rekey) {

@@ -41,6 +41,7 @@ struct BoxDesc {
   int prep_sort;             // exact-mode preparation: the box sorts its particles
   int prep_outside;          // ... and its particles outside an explicit grid
   int error;
+  int revived;               // new particles ended an error: parallel-mode claims may be left
   int n_rounds, n_dropped;   // parallel mode: tail claim rounds, dropped samples
   int64_t n_tail_tests;      // parallel mode: tests finished in the tail
   int64_t n_arrivals;        // parallel mode: particles that joined a list within a step

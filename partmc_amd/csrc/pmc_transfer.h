@@ -184,6 +184,7 @@ __global__ void k_set_uploaded(BoxDesc *B, int n_part) {
   B->pkeys_valid = 0;
   B->terms_kernel = 0;
   B->n_info = 0;
+  if (B->error) B->revived = 1;
   B->error = 0;
 }
 

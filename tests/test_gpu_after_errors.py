@@ -167,3 +167,49 @@ def test_a_parallel_step_beyond_the_capacity(n, kernel, dt, flat, room):
     assert ends[0][0] == ends[1][0] and ends[0][0][1] > 0
     for k, v in ends[0][1].items():
         np.testing.assert_array_equal(ends[1][1][k], v, err_msg=k)
+
+
+# a parent with fewer primaries than components
+BAD_PRIMARIES = (465791384, 465791385)
+
+
+@pytest.mark.parametrize("share", [0.002, 0.02, 0.3])
+def test_a_target_event_that_fails_leaves_no_claims(share):
+    """Power weights, where targets sample sources and remove some of them: an
+    event that meets a particle without primaries fails with claims on the
+    sources it took before.  The box goes on with larger particles (a new
+    grid) as a new handle does."""
+    pop = small(P.config_c2(), 3000)
+    pop.weight_magnitude *= 30.0
+    pop.grid = None
+    n = pop.n_part
+    one = np.ones(n, np.int32)
+
+    def new_handle():
+        g = make_gpu(pop)
+        g.reserve([60 * n])
+        g.set_mode(MODE_PARALLEL, PREC_FP32_RECHECK, 1e-5)
+        return g
+
+    g = new_handle()
+    primaries = np.where(np.random.default_rng(4).uniform(size=n) < share, 0, 1).astype(np.int32)
+    g.upload(0, pop.vol, pop.ids(), one, one, n_primary=primaries)
+    g.set_next_id(0, n + 1)
+    with pytest.raises(CoagError) as e:
+        for _ in range(4):
+            g.mc_coag(P.KERNEL_BROWN, 60.0)
+    assert e.value.code in BAD_PRIMARIES
+    ends = []
+    for h in (g, new_handle()):
+        h.set_weights(0, [[pop.weight_type]], [[pop.weight_magnitude * 1e3]],
+                      [[pop.weight_exponent]])
+        h.upload(0, pop.vol * 1e3, pop.ids(), one, one)
+        h.set_next_id(0, n + 1)
+        h.set_rng(7, 0)
+        counts = [tuple(int(x[0]) for x in h.mc_coag(P.KERNEL_BROWN, 100.0)) for _ in range(3)]
+        ends.append((counts, h.download(0)))
+        assert int(h.accel_counts()["n_coag"][0]) > 0
+        h.close()
+    assert ends[0][0] == ends[1][0]
+    for k, v in ends[0][1].items():
+        np.testing.assert_array_equal(ends[1][1][k], v, err_msg=k)
