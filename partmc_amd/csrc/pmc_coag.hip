@@ -218,7 +218,10 @@ static int alloc_tables(pmc_gpu *h, int classes) {
 static int layout(pmc_gpu *h, const std::vector<int64_t> &new_cap) {
   h->work.clean_type = 0;
   std::vector<BoxDesc> hb(h->n_box);
-  HIPCHECK(read_boxes(h, hb.data(), 0, h->n_box));
+  // (like the copies below, after the stream's work and without starting the
+  // stream: its first use costs 70 us, which a handle's first transfer pays)
+  HIPCHECK(hipMemcpy((void *)hb.data(), h->d_box, sizeof(BoxDesc) * h->n_box,
+                     hipMemcpyDeviceToHost));
   Arrays old = h->A;
   int64_t total = 0, pool_total = 0, info_total = 0;
   std::vector<int64_t> off(h->n_box), poff(h->n_box), ioff(h->n_box), phalf(h->n_box);
