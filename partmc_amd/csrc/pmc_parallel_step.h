@@ -733,6 +733,10 @@ __device__ inline int accel_kind(const Weights &w, const double *edges, int b1, 
   return kind;
 }
 
+// The most tests a bin pair may expect: its draw stays within an int by more
+// than a thousand standard deviations.
+constexpr double MAX_PAIR_TESTS = 2.0e9;
+
 // n_samp of every (box, c1, c2, b1, b2), compute_n_samp
 // src/coagulation.F90:648-702 on the pair's own Poisson stream
 __global__ void k_par_pairs(BoxDesc *boxes, Arrays A, PW W, double del_t, uint64_t seed,
@@ -777,6 +781,10 @@ __global__ void k_par_pairs(BoxDesc *boxes, Arrays A, PW W, double del_t, uint64
         bool same = (b1 == b2) && (c1 == c2);
         double n_possible = same ? N1 * (N2 - 1.0) / 2.0 : N1 * N2;
         double mean = k_max * del_t * n_possible;
+        if (n_possible > 0.0 && !(mean <= MAX_PAIR_TESTS)) {  // past an int, or no number
+          atomicExch(&B->error, ERR_CAPACITY);
+          mean = 0.0;
+        }
         Stream ps;
         ps.open(seed, box, step, pair_site(nb, nc, b1, b2, c1, c2), 0, RNG_POISSON);
         ns = n_possible > 0.0 ? (uint32_t)rand_poisson(ps, mean) : 0u;
@@ -2009,20 +2017,28 @@ k_par_acc_tests(BoxDesc *boxes, Arrays A, PW W, int n_box, int type, uint64_t se
 
 // the largest batch end t1 <= min(T, t0 + T_cap) whose target slots fit the
 // records; out[0] = t1, out[1] = acc_count(t0), out[2] = acc_count(t1),
-// out[3] and [4] the step's tests and target slots, out[5] whether a box got
-// a new grid (then nothing else)
+// out[3] and [4] the step's tests and target slots, out[5] 0, or why there is
+// nothing else: BE_REGRID (a box got a new grid), BE_TESTS (the step's tests
+// are more than their 32-bit indices; the boxes' own 64-bit counts tell)
+constexpr uint32_t BE_REGRID = 1, BE_TESTS = 2;
 __device__ inline uint32_t acc_count(const PW &W, int64_t NP, uint32_t T, uint32_t t) {
   if (t >= T) return W.acc_exc[NP];
   int64_t k = test_pair(W, NP, t);
   return W.acc_exc[k] + (W.pair_acc[k] ? t - W.pair_exc[k] : 0u);
 }
 
-__global__ void k_batch_end(PW W, int64_t NP, uint32_t t0, uint32_t t_cap, uint32_t a_cap,
-                            uint32_t *out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ void __launch_bounds__(64)
+k_batch_end(const BoxDesc *boxes, PW W, int n_box, int64_t NP, uint32_t t0, uint32_t t_cap,
+            uint32_t a_cap, uint32_t *out) {
   const bool regrid = W.rc[RC_REGRID] == W.tag;
-  out[5] = regrid ? 1u : 0u;
-  if (regrid) return;
+  long long tests = 0;
+  if (t0 == 0)  // the first batch's: step_samp holds this step's draws
+    for (int b = threadIdx.x; b < n_box; b += 64) tests += boxes[b].step_samp;
+  for (int o = 32; o > 0; o >>= 1) tests += __shfl_xor(tests, o);
+  if (threadIdx.x != 0) return;
+  tests += W.acc_exc[NP];
+  out[5] = regrid ? BE_REGRID : tests > (long long)UINT32_MAX ? BE_TESTS : 0u;
+  if (out[5]) return;
   const uint32_t T = W.pair_exc[NP];
   const uint32_t a0 = acc_count(W, NP, T, t0);
   uint32_t lo = t0 + 1, hi = (T - t0 < t_cap) ? T : t0 + t_cap;
@@ -3975,8 +3991,8 @@ inline void parallel_sort_and_pairs(ParallelWork &W, const Arrays &A, BoxDesc *d
   J.cols = 2;
   scan_excl_sum(J, W.NP, st);
   // the step's test count, its target slots and the first batch's bounds
-  hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, d, W.NP, 0u, (uint32_t)W.T_cap,
-                     (uint32_t)ACC_CAP, W.h_u32 + 4);
+  hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, d_box, d, n_box, W.NP, 0u,
+                     (uint32_t)W.T_cap, (uint32_t)ACC_CAP, W.h_u32 + 4);
 }
 
 // the pair space of grids of up to mb bins
@@ -4028,7 +4044,7 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
     // 2.-4. on the last step's grids; W.h_u32[9] tells whether they still hold
     parallel_sort_and_pairs(W, A, d_box, n_box, st, del_t, seed, step);
     PCHECK(hipStreamSynchronize(st));
-    clean = W.h_u32[9] == 0;
+    clean = W.h_u32[9] != BE_REGRID;
   }
   if (!clean) {
     if (++W.tag == INT32_MAX) W.tag = 1;
@@ -4056,6 +4072,10 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
     parallel_sort_and_pairs(W, A, d_box, n_box, st, del_t, seed, step);
     PCHECK(hipStreamSynchronize(st));
   }
+  if (W.h_u32[9] == BE_TESTS) {
+    g_parallel_error = "more than 2^32 - 1 tests in a step: reduce del_t or remake the grid";
+    return ERR_CAPACITY;
+  }
   const uint32_t T = W.h_u32[7];
   const uint32_t T_acc = W.h_u32[8];
   if (T_acc > 0 && d.ev == nullptr) {
@@ -4081,8 +4101,8 @@ inline int parallel_step(ParallelWork &W, const Arrays &A, BoxDesc *d_box, int n
     const bool first = t0 == 0;
     if (!first) {
       // the batch ends where its target slots would overflow the records
-      hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, d, W.NP, t0, (uint32_t)W.T_cap,
-                         (uint32_t)d.acc_cap, W.h_u32 + 4);
+      hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, d_box, d, n_box, W.NP, t0,
+                         (uint32_t)W.T_cap, (uint32_t)d.acc_cap, W.h_u32 + 4);
       PCHECK(hipStreamSynchronize(st));
     }
     t1 = W.h_u32[4];

@@ -213,3 +213,36 @@ def test_a_target_event_that_fails_leaves_no_claims(share):
     assert ends[0][0] == ends[1][0]
     for k, v in ends[0][1].items():
         np.testing.assert_array_equal(ends[1][1][k], v, err_msg=k)
+
+
+@pytest.mark.parametrize("n_box,mean", [(1, 5e9), (3, 1.9e9)])
+def test_more_tests_than_a_step_can_number(n_box, mean):
+    """All particles in the middle one of three bins: more tests than a pair's
+    draw holds, and pairs of which each can be drawn but whose sum passes 32
+    bits.  Neither makes a test; the boxes then step as a new handle's with
+    other particles."""
+    n, flat = 2000, 2e6
+    k_max = 2.0 * 0.25 / (60.0 * 2e8)  # the constant kernel's majorant, over-estimated by 2
+    dt = mean / (k_max * flat * n * (n - 1) / 2)
+    pops = [flat_pop(n, 20 + b, flat) for b in range(n_box)]
+    g = parallel_boxes(pops, [64] * n_box)
+    for b in range(n_box):
+        g.set_bin_grid(b, 3, 1e-10, 1e-1)
+    with pytest.raises(CoagError) as e:
+        g.mc_coag(P.KERNEL_CONSTANT, dt)
+    assert e.value.code == CAPACITY
+    # smaller particles, so that both make their grid anew
+    new = parallel_boxes(pops, [64] * n_box)
+    ends = []
+    for h in (g, new):
+        for b, p in enumerate(pops):
+            p.vol = flat_pop(n, 20 + b, flat).vol * 1e-12
+            h.load_population(b, p)
+        h.set_rng(7, 0)
+        ends.append(([x.tolist() for x in h.mc_coag(P.KERNEL_CONSTANT, 6.0)],
+                     [h.download(b) for b in range(n_box)]))
+        h.close()
+    assert ends[0][0] == ends[1][0] and min(ends[0][0][1]) > 0
+    for x, y in zip(ends[0][1], ends[1][1]):
+        for k, v in x.items():
+            np.testing.assert_array_equal(y[k], v, err_msg=k)
