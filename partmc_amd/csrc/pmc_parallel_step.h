@@ -3953,10 +3953,12 @@ inline int parallel_layout(ParallelWork &W, const Arrays &A, int n_box,
   return 0;
 }
 
+// more weight classes: the arrays go, so that nothing reads them with the new
+// strides, and the next step lays them out again
 inline int parallel_classes(ParallelWork &W, int n_box, int classes) {
   (void)n_box;
+  parallel_free_arrays(W);
   W.d.tab_classes = classes;
-  // arrays are re-laid out at the next parallel_layout call; mark stale
   W.d.K_stride = W.d.max_bin * classes;
   W.d.P_stride = (int64_t)classes * classes * W.d.max_bin * W.d.max_bin;
   g_parallel_error = "";

@@ -246,3 +246,24 @@ def test_more_tests_than_a_step_can_number(n_box, mean):
     for x, y in zip(ends[0][1], ends[1][1]):
         for k, v in x.items():
             np.testing.assert_array_equal(y[k], v, err_msg=k)
+
+
+def test_step_lists_across_a_new_class_count():
+    """The lists of the last step end with the class count they were made for:
+    asking for them before the next step is an error, and the next step's are
+    the particles' counts."""
+    pops = [flat_pop(400, 30 + b, 2e6) for b in range(3)]
+    g = parallel_boxes(pops, [64] * 3)
+    g.mc_coag(P.KERNEL_CONSTANT, 6.0)
+    assert g.step_lists(2).sum() == 400
+    for b in range(3):
+        g.set_weights(b, [[1, 1, 1]], [[2e6, 2e6, 2e6]], [[0.0, 0.0, 0.0]])
+    for b in range(3):
+        with pytest.raises(CoagError):
+            g.step_lists(b, 3)
+    left = [g.n_part(b) for b in range(3)]
+    g.mc_coag(P.KERNEL_CONSTANT, 6.0)
+    for b in range(3):
+        counts = g.step_lists(b, 3)
+        assert counts.sum() == left[b]
+    g.close()
