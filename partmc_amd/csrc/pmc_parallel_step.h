@@ -1529,12 +1529,10 @@ __device__ inline bool rm_has(const PW &W, const RmChain &c, int slot) {
 // particles 116 ms in place of 127 with one entry at a time
 constexpr int WALK = 4;
 
-// visit the chain of record r in order: removed sources (>= 0) and the
-// owner markers (-1 - k: the removals that follow belong to copy k)
+// visit the entries of a list of `left` kept in chunks from `head` on
 template <class F>
-__device__ inline void chain_walk(const PW &W, int r, F f) {
-  int left = W.ev[r].nchain;
-  for (int ch = W.ev[r].head; ch >= 0 && left > 0; ch = W.rm_buf[ch]) {
+__device__ inline void chunk_walk(const PW &W, int head, int left, F f) {
+  for (int ch = head; ch >= 0 && left > 0; ch = W.rm_buf[ch]) {
     const int m = left < RM_CHUNK - 1 ? left : RM_CHUNK - 1;
     for (int q = 1; q <= m; q += WALK) {
       int e[WALK];
@@ -1548,10 +1546,11 @@ __device__ inline void chain_walk(const PW &W, int r, F f) {
   }
 }
 
-// visit the removed sources of record r in removal order
+// visit the removed sources of record r in removal order; its chain also
+// holds owner markers (-1 - k: the removals that follow belong to copy k)
 template <class F>
 __device__ inline void rm_walk(const PW &W, int r, F f) {
-  chain_walk(W, r, [&](int q) {
+  chunk_walk(W, W.ev[r].head, W.ev[r].nchain, [&](int q) {
     if (q >= 0) f(q);
   });
 }
@@ -1559,19 +1558,7 @@ __device__ inline void rm_walk(const PW &W, int r, F f) {
 // visit the sources record r read from small lists
 template <class F>
 __device__ inline void rd_walk(const PW &W, int r, F f) {
-  int left = W.ev[r].nrd;
-  for (int ch = W.ev[r].rdhead; ch >= 0 && left > 0; ch = W.rm_buf[ch]) {
-    const int m = left < RM_CHUNK - 1 ? left : RM_CHUNK - 1;
-    for (int q = 1; q <= m; q += WALK) {
-      int e[WALK];
-#pragma unroll
-      for (int u = 0; u < WALK; ++u) e[u] = W.rm_buf[ch + min(q + u, m)];
-#pragma unroll
-      for (int u = 0; u < WALK; ++u)
-        if (q + u <= m) f(e[u]);
-    }
-    left -= m;
-  }
+  chunk_walk(W, W.ev[r].rdhead, W.ev[r].nrd, f);
 }
 
 template <int NS>
